@@ -60,7 +60,8 @@ typedef struct {
                                 matrix, computed at the first such solve and kept (ILU_MATRIX);
                               3 "PointJacobi" as the reference's branch runs it: the scaling and no
                                 solver call, so x = x0 (zeros) with the fixed values */
-  int32_t spmv_kind;     /* 0 auto (blocked when the CRS has DOF=3 node blocks and pads little, else CRS
+  int32_t spmv_kind;     /* 0 auto (element by element on large systems whose values are exactly a
+                            hex8 mesh's stiffness; else blocked when the CRS has DOF=3 node blocks and pads little, else CRS
                             rows, with x staged in LDS for the unpreconditioned FP64 solve from 2^18
                             rows on), 1 CRS row kernel, 2 blocked, 4 CRS rows with x staged in LDS per
                             row block (FP64, no ILU) */
@@ -89,7 +90,8 @@ typedef struct {
   int32_t status;           /* PF_* code of the solve */
   int32_t iterations;       /* BiCGSTAB iterations (FP64 or, for precision 32, FP32) */
   int32_t outer_iterations; /* FP64 residual replacements (mixed), 0 for FP64 */
-  int32_t spmv_kind_used;   /* 1 CRS row kernel, 2 blocked, 4 CRS rows with x staged in LDS */
+  int32_t spmv_kind_used;   /* 1 CRS row kernel, 2 blocked, 4 CRS rows with x staged in LDS, 5 element
+                               by element */
   double rr;                /* final r.r of the recurrence (FP64 form) */
   double rr1;               /* r.r after iteration 1 */
   double true_relres;       /* ||b - A x|| / ||b|| in FP64 after the solve (eliminated system) */
@@ -368,6 +370,13 @@ int pf_system_ilu_reset(pf_system *sys);
  * reuse the last x; y NULL: keep on device).  The kernel is launched `repeat` times and *ms
  * (may be NULL) receives the average device time of one launch (hipEvents). */
 int pf_system_spmv(pf_system *sys, int32_t kind, const double *x, double *y, int32_t repeat, double *ms);
+
+/* y = A x (host vectors) element by element from the mesh and the resident materials, as the
+ * solver applies a stiffness from pf_system_stiffness without streaming its values: A is the CRS
+ * matrix after the Dirichlet elimination of the current fixes (applied first) and any PointJacobi
+ * scaling, to rounding.  PF_INVALID when the CRS values come from anything else, or the mesh's
+ * elements share too few nodes for it. */
+int pf_system_elem_apply(pf_system *sys, const double *x, double *y);
 
 /* Device pointers of the system's arrays, for torch interop (valid until the next call
  * that reallocates: set_mesh, zero_matrix, set_crs, destroy). */

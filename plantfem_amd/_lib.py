@@ -161,6 +161,7 @@ SIGNATURES = {
     "pf_ilu_apply_crs": (C.c_int, [P, I64, PI64, PI32, PF64, PF64, PF64]),
     "pf_system_view_get": (C.c_int, [P, C.POINTER(SystemView)]),
     "pf_system_spmv": (C.c_int, [P, I32, PF64, PF64, I32, PF64]),
+    "pf_system_elem_apply": (C.c_int, [P, PF64, PF64]),
     "pf_system_add_tractions": (C.c_int, [P, I32, PI64, PF64, PF64]),
     "pf_system_batch_set": (C.c_int, [P, I32, PI64, PF64]),
     "pf_system_batch_solve": (C.c_int, [P, C.POINTER(SolveOpts), C.POINTER(BatchTune), PF64, P,

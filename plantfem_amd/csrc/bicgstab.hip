@@ -33,12 +33,13 @@
 #include <type_traits>
 #include <vector>
 
+#include "elem_dev.hpp"
 #include "spmv_dev.hpp"
 
 namespace {
 
 constexpr int BT = 256;  // threads per block of every fused kernel (4 wavefronts)
-constexpr int KEY_WORDS = 45;      // words of the key of a captured iteration chunk
+constexpr int KEY_WORDS = 50;      // words of the key of a captured iteration chunk
 constexpr int ILU_KEY_WORDS = 32;  // the same for the ILU chunk
 
 struct Scal {
@@ -50,7 +51,8 @@ struct Scal {
   double maxr[2];      // reliable updates: largest |r| since the last replacement (slot by parity)
   double relres;       // reliable updates: FP64 |b - A x| / |b| at the last replacement
   double target, delta;
-  int32_t pending;     // reliable updates: a replacement is due after this iteration
+  int32_t pending;     // reliable updates: a replacement is due (kernels return until it is done)
+  int32_t skip;        // the same for K4, set by the first kernel after the iteration that asked
   int32_t nupd;        // replacements done
   int32_t itr_rep;     // iteration of the last replacement
   int32_t itr[2];      // completed iterations, slot by parity (written by K4)
@@ -74,6 +76,9 @@ struct Mat {
   const int32_t *col;
   const M *sval;
   pfdev::Stage st;  // L = 2: the row blocks' staged columns
+  ElemView el;      // layout 3: the element tiles (ntile = 0 otherwise)
+  double *epart;    // layout 3: the tiles' slot sums
+  int jmode;        // layout 3
 };
 
 // Visit every row of y = A*xf with the calling thread's share of the grid; op(row, sum) is
@@ -112,9 +117,10 @@ __device__ inline void for_rows(const Mat<V, M> &m, XF xf, OP op) {
 }
 
 // block sum of NV values, result in every thread
-template <int NV>
+template <int NV, int T = BT>
 __device__ inline void block_sum(double (&v)[NV]) {
-  __shared__ double sh[NV][BT / 64];
+  static_assert(T == 256 || T == 128, "four or two wavefronts");
+  __shared__ double sh[NV][T / 64];
 #pragma unroll
   for (int k = 0; k < NV; ++k)
 #pragma unroll
@@ -125,7 +131,10 @@ __device__ inline void block_sum(double (&v)[NV]) {
     for (int k = 0; k < NV; ++k) sh[k][w] = v[k];
   __syncthreads();
 #pragma unroll
-  for (int k = 0; k < NV; ++k) v[k] = ((sh[k][0] + sh[k][1]) + sh[k][2]) + sh[k][3];
+  for (int k = 0; k < NV; ++k) {
+    v[k] = sh[k][0] + sh[k][1];
+    if constexpr (T == 256) v[k] = (v[k] + sh[k][2]) + sh[k][3];
+  }
   __syncthreads();
 }
 
@@ -139,14 +148,14 @@ __device__ inline void write_partials(double (&v)[NV], double *part) {
 }
 
 // all G partials of the previous kernel, summed in a fixed order (same result in every block)
-template <int NV>
+template <int NV, int T = BT>
 __device__ inline void read_partials(const double *part, int G, double (&out)[NV]) {
 #pragma unroll
   for (int k = 0; k < NV; ++k) out[k] = 0.0;
-  for (int b = threadIdx.x; b < G; b += BT)
+  for (int b = threadIdx.x; b < G; b += T)
 #pragma unroll
     for (int k = 0; k < NV; ++k) out[k] += part[(int64_t)k * G + b];
-  block_sum<NV>(out);
+  block_sum<NV, T>(out);
 }
 
 // ---- K0: r = b - A x (or r = b when x0 = 0); r0 = p = r  -> partials r.r, b.b ----------
@@ -203,12 +212,20 @@ __global__ void __launch_bounds__(BT) k_init_finish(const double *__restrict__ p
   }
 }
 
+// A residual replacement is due: the iterations enqueued before it return at entry.  The first
+// kernel of an iteration hands the flag on to K4, whose own launch raises it.
+__device__ inline bool iteration_pending(Scal *sc) {
+  if (!sc->pending) return false;
+  if (blockIdx.x == 0 && threadIdx.x == 0) sc->skip = 1;
+  return true;
+}
+
 // ---- K1: y = A p -> partials r0.y ------------------------------------------------------
 template <typename V, int L, int SUB, typename M>
 __global__ void __launch_bounds__(BT) k_spmv_p(Mat<V, M> m, const V *__restrict__ p, V *__restrict__ y,
-                                               const V *__restrict__ r0, const Scal *__restrict__ sc,
+                                               const V *__restrict__ r0, Scal *__restrict__ sc,
                                                double *__restrict__ part) {
-  if (sc->done) return;
+  if (sc->done || iteration_pending(sc)) return;
   double acc[1] = {0.0};
   auto op = [&](int64_t row, V yv) {
     y[row] = yv;
@@ -232,7 +249,7 @@ __global__ void __launch_bounds__(BT) k_spmv_e(Mat<V, M> m, const V *__restrict_
                                                V *__restrict__ v, Scal *__restrict__ sc,
                                                const double *__restrict__ pin, int Gin,
                                                double *__restrict__ part) {
-  if (sc->done) return;
+  if (sc->done || sc->pending) return;
   double t[1];
   read_partials<1>(pin, Gin, t);
   const double c2 = t[0];
@@ -268,7 +285,7 @@ template <typename V>
 __global__ void __launch_bounds__(BT) k_evec(int64_t n, const V *__restrict__ r, const V *__restrict__ y,
                                              V *__restrict__ e, Scal *__restrict__ sc,
                                              const double *__restrict__ pin, int Gin) {
-  if (sc->done) return;
+  if (sc->done || sc->pending) return;
   double t[1];
   read_partials<1>(pin, Gin, t);
   const double c2 = t[0];
@@ -295,7 +312,7 @@ __global__ void __launch_bounds__(BT) k_evec(int64_t n, const V *__restrict__ r,
 template <typename V, int L, int SUB, typename M>
 __global__ void __launch_bounds__(BT, L == 1 ? 1 : 8) k_spmv_ev(Mat<V, M> m, const V *__restrict__ e, V *__restrict__ v,
                                                 Scal *__restrict__ sc, double *__restrict__ part) {
-  if (sc->done) return;
+  if (sc->done || sc->pending) return;
   const pfdev::PlainX<V> ef{e};
   double acc[2] = {0.0, 0.0};
   auto op = [&](int64_t row, V vv) {
@@ -308,6 +325,94 @@ __global__ void __launch_bounds__(BT, L == 1 ? 1 : 8) k_spmv_ev(Mat<V, M> m, con
   write_partials<2>(acc, part);
 }
 
+// ---- K1, K2 element by element (layout 3): the tiles' slot sums, then each node's sums with the
+// dot products.  alpha comes from K1's partials in the first half of K2.
+// At 3.09M rows (100^3 bricks) the tiles take 53 and 57 us and the sums 33 and 31 us, against 367
+// and 384 us of the blocked products: 165 MB (slot tables, coordinates, slot sums) and 460
+// operations per element instead of 2.1 GB.  The tiles hold 128 VGPRs and 25 KB of LDS (six
+// workgroups per CU); elements that are no parallelepipeds need 1250 operations and 256 VGPRs
+// (two waves per SIMD): 14 and 16 us at 248k rows.
+template <typename V, int JM, bool AFF>
+__global__ void __launch_bounds__(pfelem::ET, AFF ? 3 : 2) k_el_p(ElemView el, const V *__restrict__ p,
+                                                                  Scal *__restrict__ sc, double *__restrict__ epart) {
+  if (sc->done || iteration_pending(sc)) return;
+  extern __shared__ double esh[];
+  for (int k = blockIdx.x; k < ((el.ntile + 7) & ~7); k += gridDim.x) {
+    const int t = pfelem::tile_of(k, el.ntile, gridDim.x);
+    if (t >= 0) pfelem::tile<JM, AFF>(el, t, esh, pfdev::PlainX<V>{p}, epart);
+  }
+}
+
+template <typename V, int JM, bool AFF>
+__global__ void __launch_bounds__(pfelem::ET, AFF ? 3 : 2) k_el_e(ElemView el, const V *__restrict__ r,
+                                                                  const V *__restrict__ y, Scal *__restrict__ sc,
+                                                                  const double *__restrict__ pin, int Gin,
+                                                                  double *__restrict__ epart) {
+  if (sc->done || sc->pending) return;
+  double t[1];
+  read_partials<1, pfelem::ET>(pin, Gin, t);
+  const double c2 = t[0];
+  const double alpha_d = sc->c1 / c2;
+  const bool first = threadIdx.x == 0 && blockIdx.x == 0;
+  if (first) {
+    sc->c2 = c2;
+    sc->alpha = alpha_d;
+  }
+  if (sc->guard && !isfinite(alpha_d)) {  // r0.Ap lost: stop before x is touched
+    if (first) {
+      sc->status = PF_BREAKDOWN_C2C3;
+      sc->done = 1;
+    }
+    return;
+  }
+  extern __shared__ double esh[];
+  for (int k = blockIdx.x; k < ((el.ntile + 7) & ~7); k += gridDim.x) {
+    const int t = pfelem::tile_of(k, el.ntile, gridDim.x);
+    if (t >= 0) pfelem::tile<JM, AFF>(el, t, esh, EFromRY<V>{r, y, (V)alpha_d}, epart);
+  }
+}
+
+template <typename V>
+__global__ void __launch_bounds__(BT) k_el_rows_p(ElemView el, const V *__restrict__ p, V *__restrict__ y,
+                                                  const V *__restrict__ r0, const Scal *__restrict__ sc,
+                                                  const double *__restrict__ epart, double *__restrict__ part) {
+  if (sc->done || sc->pending) return;
+  double acc[1] = {0.0};
+  for (int64_t i = blockIdx.x * (int64_t)BT + threadIdx.x; i < el.nn; i += (int64_t)gridDim.x * BT) {
+    double s[3];
+    pfelem::node_sum(el, i, epart, pfdev::PlainX<V>{p}, s);
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      const V yv = (V)s[d];
+      y[3 * i + d] = yv;
+      acc[0] += (double)r0[3 * i + d] * (double)yv;
+    }
+  }
+  write_partials<1>(acc, part);
+}
+
+template <typename V>
+__global__ void __launch_bounds__(BT) k_el_rows_e(ElemView el, const V *__restrict__ r, const V *__restrict__ y,
+                                                  V *__restrict__ v, const Scal *__restrict__ sc,
+                                                  const double *__restrict__ epart, double *__restrict__ part) {
+  if (sc->done || sc->pending) return;
+  const EFromRY<V> ef{r, y, (V)sc->alpha};
+  double acc[2] = {0.0, 0.0};
+  for (int64_t i = blockIdx.x * (int64_t)BT + threadIdx.x; i < el.nn; i += (int64_t)gridDim.x * BT) {
+    double s[3];
+    pfelem::node_sum(el, i, epart, ef, s);
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      const V vv = (V)s[d];
+      v[3 * i + d] = vv;
+      const V e = ef(3 * i + d);
+      acc[0] += (double)e * (double)vv;
+      acc[1] += (double)vv * (double)vv;
+    }
+  }
+  write_partials<2>(acc, part);
+}
+
 // ---- K3: omega ; x += alpha p + omega e ; r = e - omega v -> partials r.r, r0.r --------
 template <typename V>
 __global__ void __launch_bounds__(BT) k_update(int64_t n, V *__restrict__ x, V *__restrict__ r,
@@ -315,7 +420,7 @@ __global__ void __launch_bounds__(BT) k_update(int64_t n, V *__restrict__ x, V *
                                                const V *__restrict__ y, const V *__restrict__ v,
                                                Scal *__restrict__ sc, const double *__restrict__ pin, int Gin,
                                                double *__restrict__ part) {
-  if (sc->done) return;
+  if (sc->done || sc->pending) return;
   double t[2];
   read_partials<2>(pin, Gin, t);
   const bool first = threadIdx.x == 0 && blockIdx.x == 0;
@@ -355,7 +460,7 @@ __global__ void __launch_bounds__(BT) k_pupdate(int64_t n, V *__restrict__ p, co
                                                 const double *__restrict__ pin, int Gin, int par,
                                                 double *__restrict__ hist, double *__restrict__ xhi,
                                                 V *__restrict__ xlo) {
-  if (sc->done) return;
+  if (sc->done || sc->skip) return;
   double t[2];
   read_partials<2>(pin, Gin, t);
   const bool first = threadIdx.x == 0 && blockIdx.x == 0;
@@ -647,7 +752,9 @@ __global__ void __launch_bounds__(BT) k_rel_finish(const double *__restrict__ pa
   sc->c1 = t[2];
   sc->rr = t[0];
   sc->maxr[0] = sc->maxr[1] = sqrt(t[0]);
+  sc->itr[0] = sc->itr[1] = sc->itr_last;  // iterations skipped while pending do not count
   sc->pending = 0;
+  sc->skip = 0;
   if (!(relres >= sc->target)) {  // converged, or NaN
     sc->status = isfinite(relres) ? PF_OK : PF_BREAKDOWN_C2C3;
     sc->done = 1;
@@ -664,6 +771,11 @@ __global__ void k_rel_final(int64_t n, const double *__restrict__ zhi, const VI 
 
 __global__ void k_ones(int64_t n, double *__restrict__ a) {
   for (int64_t i = blockIdx.x * (int64_t)BT + threadIdx.x; i < n; i += (int64_t)gridDim.x * BT) a[i] = 1.0;
+}
+
+__global__ void k_product(int64_t n, const double *__restrict__ a, const double *__restrict__ b,
+                          double *__restrict__ c) {
+  for (int64_t i = blockIdx.x * (int64_t)BT + threadIdx.x; i < n; i += (int64_t)gridDim.x * BT) c[i] = a[i] * b[i];
 }
 
 __global__ void k_f64_to_f32(int64_t n, const double *__restrict__ a, float *__restrict__ b) {
@@ -694,6 +806,7 @@ struct SolverWork {
   DevBuf<int32_t> flag;
   DevBuf<double> jscale;  // FP32 system row scale: 1/sqrt|a_ii| (symmetric) or 1/a_ii (row)
   DevBuf<double> jones;   // column scale of the row-scaled form
+  DevBuf<double> escale;  // element form: product of the matrix's own row scale and jscale
   // ILU(0) form: the factor is kept across solves, as FEMSolver_%ILU_MATRIX is
   // (FEMSolverClass.f90:1777-1784), until pf_ilu_reset
   IluFactor ilu;
@@ -740,7 +853,7 @@ struct Launch {
   unsigned grid;    // SpMV kernels
   unsigned grid_e;  // element-wise kernels
   int sub;
-  int layout;  // 0 CRS, 1 Sell3, 2 CRS with x staged in LDS per row block
+  int layout;  // 0 CRS, 1 Sell3, 2 CRS with x staged in LDS per row block, 3 element tiles
 };
 
 // partial-sum rows of G doubles each: K1 (1 dot), K2 (2), K3 (2), and one region shared by
@@ -772,6 +885,13 @@ unsigned elem_grid(pf_ctx *ctx, int64_t n) {
   return (unsigned)b;
 }
 
+// element tiles: the resident workgroups, each walking its share of the tiles
+unsigned elem_tile_grid(pf_ctx *ctx, const ElemView &el) {
+  const int64_t cap = (el.affine ? 6 : 4) * (int64_t)ctx->num_cus;
+  const int64_t all = ((int64_t)el.ntile + 7) & ~(int64_t)7;
+  return (unsigned)(all < cap ? all : cap);
+}
+
 // every partial row holds one double per block of the writing kernel: grids above G would
 // write past w->part
 int check_grid(pf_ctx *ctx, const Launch &L) {
@@ -788,6 +908,24 @@ int choose_sub(double avg_row) {  // ~five nonzeros per lane, 4..64 lanes per CR
   while (sub < 64 && sub * 1.4142 * 5.0 < avg_row) sub *= 2;
   return sub;
 }
+
+#define PF_DISPATCH_ELEM(M, ...)                                            \
+  if ((M).jmode == 0) {                                                     \
+    constexpr int J_ = 0;                                                   \
+    if ((M).el.affine) { constexpr bool A_ = true; __VA_ARGS__; }           \
+    else { constexpr bool A_ = false; __VA_ARGS__; }                        \
+  } else {                                                                  \
+    constexpr int J_ = 1;                                                   \
+    if ((M).el.affine) { constexpr bool A_ = true; __VA_ARGS__; }           \
+    else { constexpr bool A_ = false; __VA_ARGS__; }                        \
+  }
+
+constexpr int REPL_EVERY = 8;
+// rows from which the element tiles are taken: their iteration is six launches, 25-31 us up to
+// 50,000 rows on MI355X, the other forms four.  Microseconds per iteration, blocked / tiles:
+// Cube3D 28k rows 44 / 31, 73k 49 / 33, 207k 80 / 44, 681k 200 / 70, 3.09M 846 / 228;
+// cylinders 35k 43 / 37, 156k 61 / 49, 266k 94 / 59
+constexpr int64_t ELEM_MIN_ROWS = 40000;
 
 #define PF_DISPATCH_SUB(SUBV, ...)                          \
   switch (SUBV) {                                           \
@@ -861,11 +999,19 @@ int enqueue_iters(pf_ctx *ctx, const Launch &L, const Mat<V, M> &m, V *x, V *r, 
   hipStream_t st = ctx->stream;
   const size_t G = (size_t)ctx->num_cus * 8;
   double *p1 = part + PART_P1 * G, *p2 = part + PART_P2 * G, *p3 = part + PART_P3 * G;
-  const int g1 = (int)L.grid, ge = (int)L.grid_e;
+  const int ge = (int)L.grid_e;
+  const int g1 = L.layout == 3 ? ge : (int)L.grid;  // blocks that write the partials of K1 and K2
+  const size_t lds = L.layout == 3 ? pf_elem_lds(m.el) : 0;
   for (int it = 0; it < count; ++it) {
     const int par = it & 1;
     if (ev) PF_HIP(hipEventRecord(ev[5 * it + 0], st));
-    if (L.layout == 1) {
+    if (L.layout == 3) {
+      PF_DISPATCH_ELEM(m, (k_el_p<V, J_, A_><<<L.grid, pfelem::ET, lds, st>>>(m.el, p, sc, m.epart)));
+      k_el_rows_p<V><<<L.grid_e, BT, 0, st>>>(m.el, p, y, r0, sc, m.epart, p1);
+      if (ev) PF_HIP(hipEventRecord(ev[5 * it + 1], st));
+      PF_DISPATCH_ELEM(m, (k_el_e<V, J_, A_><<<L.grid, pfelem::ET, lds, st>>>(m.el, r, y, sc, p1, g1, m.epart)));
+      k_el_rows_e<V><<<L.grid_e, BT, 0, st>>>(m.el, r, y, v, sc, m.epart, p2);
+    } else if (L.layout == 1) {
       k_spmv_p<V, 1, 64><<<L.grid, BT, 0, st>>>(m, p, y, r0, sc, p1);
       if (ev) PF_HIP(hipEventRecord(ev[5 * it + 1], st));
       if (ebuf) {  // e streamed, then v = A e gathering e alone
@@ -895,7 +1041,10 @@ int enqueue_iters(pf_ctx *ctx, const Launch &L, const Mat<V, M> &m, V *x, V *r, 
     k_pupdate<V><<<L.grid_e, BT, 0, st>>>(m.n, p, r, y, sc, p3, ge, par, hist, rel ? rel->zhi : nullptr,
                                           rel ? x : nullptr);
     if (eva) PF_HIP(hipEventRecord(eva[5 * it + 4], st));
-    if (rel) PF_CHECK(enqueue_replacement<false>(ctx, *rel, sc, part + PART_PI * G));
+    // a due replacement is done every REPL_EVERY iterations (the ones in between return at
+    // entry): its two kernels cost 11 us when nothing is due, 2% of a 3.1M-row iteration
+    if (rel && (ev || it % REPL_EVERY == REPL_EVERY - 1 || it == count - 1))
+      PF_CHECK(enqueue_replacement<false>(ctx, *rel, sc, part + PART_PI * G));
   }
   PF_HIP(hipGetLastError());
   return PF_OK;
@@ -936,7 +1085,9 @@ int run_loop(pf_ctx *ctx, SolverWork *w, int slot, const Launch &L, const Mat<V,
       rel ? (uint64_t)(uintptr_t)rel->r : 0, rel ? (uint64_t)(uintptr_t)rel->r0 : 0,
       rel ? (uint64_t)(uintptr_t)rel->p : 0, rel ? (uint64_t)(uintptr_t)rel->zlo : 0,
       (uint64_t)(uintptr_t)m.st.lidx, (uint64_t)(uintptr_t)m.st.ucnt, (uint64_t)(uintptr_t)m.st.ubase,
-      (uint64_t)(uintptr_t)m.st.ucol, (uint64_t)m.st.nb * 4099 + (uint64_t)m.st.rpb};
+      (uint64_t)(uintptr_t)m.st.ucol, (uint64_t)m.st.nb * 4099 + (uint64_t)m.st.rpb,
+      (uint64_t)(uintptr_t)m.el.tdesc, (uint64_t)(uintptr_t)m.epart, (uint64_t)(uintptr_t)m.el.nrec,
+      (uint64_t)(uintptr_t)m.el.rscale, ((uint64_t)m.el.ntile << 32) + (uint64_t)m.el.umax * 4 + (uint64_t)m.el.affine * 2 + (uint64_t)m.jmode};
   if (use_graph && (w->gexec[slot] == nullptr || std::memcmp(w->gkey[slot], key, sizeof(key)) != 0)) {
     if (w->gexec[slot]) {
       PF_HIP(hipGraphExecDestroy(w->gexec[slot]));
@@ -1029,7 +1180,11 @@ struct NonDeduced {
 template <typename V, typename M = V>
 Mat<V, M> make_mat(int64_t n, const int64_t *row_ptr, const int32_t *col_idx, const M *val,
                    const typename NonDeduced<Sell3<M>>::type *s) {
-  Mat<V, M> m{n, row_ptr, col_idx, val, 0, 0, nullptr, nullptr, nullptr, nullptr};
+  Mat<V, M> m{};
+  m.n = n;
+  m.row_ptr = row_ptr;
+  m.col_idx = col_idx;
+  m.val = val;
   if (s) {
     m.nn = s->nn;
     m.nslices = s->nslices;
@@ -1140,7 +1295,8 @@ int run_loop_ilu(pf_ctx *ctx, SolverWork *w, const Launch &L, const Mat<double> 
 template <typename VI>
 int solve_refined(pf_ctx *ctx, SolverWork *w, int64_t n, const int64_t *row_ptr, const int32_t *col_idx,
                   const double *val, const double *b, double *x, const pf_solve_opts &o, int layout, int sub,
-                  int smode, const double *scale, const double *cscale, SolveResult &res) {
+                  int smode, const double *scale, const double *cscale, const ElemView *el, int jmode, double *epart,
+                  SolveResult &res) {
   const size_t G = (size_t)ctx->num_cus * 8;
   const unsigned ge = elem_grid(ctx, n);
   const int64_t sell_threads = ((n / 3 + 63) / 64) * 64;
@@ -1168,12 +1324,18 @@ int solve_refined(pf_ctx *ctx, SolverWork *w, int64_t n, const int64_t *row_ptr,
     y = w->y.p;
     v = w->v.p;
   }
-  const Mat<VI, float> mi = make_mat<VI, float>(n, row_ptr, col_idx, w->have_v32 ? w->val32.p : nullptr,
-                                                layout == 1 ? &w->s32 : nullptr);
-  const Launch Li{fused_grid(ctx, layout == 1 ? sell_threads : n * (int64_t)sub), ge, sub, layout};
+  Mat<VI, float> mi = make_mat<VI, float>(n, row_ptr, col_idx, w->have_v32 ? w->val32.p : nullptr,
+                                          layout == 1 ? &w->s32 : nullptr);
+  Launch Li{fused_grid(ctx, layout == 1 ? sell_threads : n * (int64_t)sub), ge, sub, layout};
+  if (layout == 3) {
+    mi.el = *el;
+    mi.jmode = jmode;
+    mi.epart = epart;
+    Li.grid = elem_tile_grid(ctx, *el);
+  }
   Rel<VI> R;
   R.m = make_mat<double>(n, row_ptr, col_idx, val, layout == 1 ? &w->s64 : nullptr);
-  R.L = Launch{fused_grid(ctx, layout == 1 ? sell_threads : n * (int64_t)sub), ge, sub, layout};
+  R.L = Launch{fused_grid(ctx, layout == 1 ? sell_threads : n * (int64_t)sub), ge, sub, layout == 1 ? 1 : 0};
   R.b = b;
   R.scale = scale;
   R.cscale = cscale;
@@ -1215,7 +1377,7 @@ int solve_refined(pf_ctx *ctx, SolverWork *w, int64_t n, const int64_t *row_ptr,
 
 int pf_bicgstab_device(pf_ctx *ctx, SolverWork *w, int64_t n, const int64_t *row_ptr, const int32_t *col_idx,
                        const double *val, int64_t nnz, const double *b, double *x, const pf_solve_opts &o,
-                       bool matrix_changed, SolveResult &res) {
+                       bool matrix_changed, SolveResult &res, const ElemSource *elem) {
   res = SolveResult();
   for (int k = 0; k < 4; ++k) {
     w->t_sum[k] = 0.0;
@@ -1247,7 +1409,21 @@ int pf_bicgstab_device(pf_ctx *ctx, SolverWork *w, int64_t n, const int64_t *row
     pf_set_error("spmv_kind must be 0 (auto), 1 (CRS rows), 2 (blocked) or 4 (CRS rows, x staged in LDS)");
     return PF_INVALID;
   }
-  if (o.spmv_kind != 1 && o.spmv_kind != 4) {
+  // element by element when the matrix is a mesh's stiffness, from ELEM_MIN_ROWS rows on, unless
+  // the options ask for a matrix layout, the ILU factor or the symmetric scaling
+  ElemView ev{};
+  double *epart = nullptr;
+  if (elem && o.spmv_kind == 0 && n >= ELEM_MIN_ROWS && o.preconditioning != 2 &&
+      (o.precision == 64 || ((o.precision == 48 || o.precision == 32) && (o.jacobi == 0 || o.jacobi == 2)))) {
+    bool ok = false;
+    PF_CHECK(pf_elem_plan(ctx, *elem->g, &ok));
+    if (ok) {
+      PF_CHECK(pf_elem_view(ctx, *elem, &ev));
+      epart = elem->g->elem.part.p;
+      layout = 3;
+    }
+  }
+  if (layout != 3 && o.spmv_kind != 1 && o.spmv_kind != 4) {
     PF_CHECK(check_blocks(ctx, w, n, row_ptr, col_idx));
     layout = w->block_ok ? 1 : 0;
     if (o.spmv_kind == 2 && !layout) {
@@ -1300,7 +1476,7 @@ int pf_bicgstab_device(pf_ctx *ctx, SolverWork *w, int64_t n, const int64_t *row
       w->have_s32 = true;
       w->s32_mode = smode;
     }
-  } else if (refined && (!w->have_v32 || w->v32_mode != smode)) {
+  } else if (layout != 3 && refined && (!w->have_v32 || w->v32_mode != smode)) {
     PF_CHECK(w->val32.ensure((size_t)nnz + 1));
     PF_CHECK(pf_crs_to_f32(ctx, n, row_ptr, col_idx, val, scale, w->val32.p, cscale));
     w->have_v32 = true;
@@ -1342,7 +1518,7 @@ int pf_bicgstab_device(pf_ctx *ctx, SolverWork *w, int64_t n, const int64_t *row
   // FP64 CRS rows: refinement residual and the final true residual
   Mat<double> mcrs = make_mat<double>(n, row_ptr, col_idx, val, nullptr);
   Launch Lres{fused_grid(ctx, n * (int64_t)sub), elem_grid(ctx, n), sub, 0};
-  res.kind = layout == 1 ? 2 : (layout == 2 ? 4 : 1);
+  res.kind = layout == 1 ? 2 : (layout == 2 ? 4 : (layout == 3 ? 5 : 1));
   const size_t G = (size_t)ctx->num_cus * 8;
   double *pres = w->part.p + PART_PI * G;
 
@@ -1369,14 +1545,20 @@ int pf_bicgstab_device(pf_ctx *ctx, SolverWork *w, int64_t n, const int64_t *row
                             w->stage.rpb};
       L64.grid = fused_grid(ctx, w->stage.nb * (int64_t)BT);
       L64.sub = w->stage.sub;
+    } else if (layout == 3) {
+      m64.el = ev;
+      m64.jmode = elem->jmode;
+      m64.epart = epart;
+      L64.grid = elem_tile_grid(ctx, ev);
     }
     const int guard = o.stop_mode == 1 ? 1 : 0;  // modes 0 and 2 keep the reference's unguarded arithmetic
     // kernel stop rules: 0 bicgstab_CRS_2, 1 |r| < relative_er |b|, 3 bicgstab_CRS (er = er0)
     const int kmode = o.stop_mode == 2 ? 3 : o.stop_mode;
     PF_CHECK(prepare_scalars(ctx, w, 0, o, o.itrmax, o.relative_er, kmode, 0, guard));
-    PF_CHECK(enqueue_init<double>(ctx, L64, m64, b, x, w->r.p, w->r0.p, w->p.p, w->sc.p, w->part.p, false));
+    PF_CHECK(enqueue_init<double>(ctx, layout == 3 ? Lres : L64, m64, b, x, w->r.p, w->r0.p, w->p.p, w->sc.p,
+                                  w->part.p, false));
     double *ebuf = nullptr;
-    if (layout != 1) {  // CRS rows: e as a stream, then the product gathers (or stages) e alone
+    if (layout != 1 && layout != 3) {  // CRS rows: e as a stream, then the product gathers (or stages) e alone
       PF_CHECK(w->e.ensure(n));
       ebuf = w->e.p;
     }
@@ -1399,12 +1581,22 @@ int pf_bicgstab_device(pf_ctx *ctx, SolverWork *w, int64_t n, const int64_t *row
       scale = cscale = w->jscale.p;
       w->have_scale = false;
     }
+    if (layout == 3) {  // the inner system is D^-1 (matrix); the matrix itself may be row-scaled already
+      if (ev.rscale) {
+        PF_CHECK(w->escale.ensure(n));
+        k_product<<<elem_grid(ctx, n), BT, 0, ctx->stream>>>(n, ev.rscale, scale, w->escale.p);
+        PF_HIP(hipGetLastError());
+        ev.rscale = w->escale.p;
+      } else if (smode == 2) {
+        ev.rscale = scale;
+      }
+    }
     if (mixed)
-      PF_CHECK(solve_refined<float>(ctx, w, n, row_ptr, col_idx, val, b, x, o, layout, sub, smode, scale, cscale,
-                                    res));
+      PF_CHECK(solve_refined<float>(ctx, w, n, row_ptr, col_idx, val, b, x, o, layout, sub, smode, scale, cscale, &ev,
+                                    elem ? elem->jmode : 0, epart, res));
     else
-      PF_CHECK(solve_refined<double>(ctx, w, n, row_ptr, col_idx, val, b, x, o, layout, sub, smode, scale, cscale,
-                                     res));
+      PF_CHECK(solve_refined<double>(ctx, w, n, row_ptr, col_idx, val, b, x, o, layout, sub, smode, scale, cscale, &ev,
+                                     elem ? elem->jmode : 0, epart, res));
   }
   PF_HIP(hipEventRecord(ctx->ev1, ctx->stream));
   PF_HIP(hipEventSynchronize(ctx->ev1));

@@ -105,6 +105,7 @@ int set_mesh(pf_ctx *ctx, NodeGraph &g, int64_t nn, int64_t ne, int32_t nne, con
   g.ne = ne;
   g.nne = nne;
   g.built = g.cols_built = false;
+  g.elem.tried = g.elem.ok = false;
   g.has_coords = nodcoord != nullptr;
   if (nodcoord) PF_CHECK(upload(ctx, g.nodcoord, nodcoord, (size_t)nn * 3));
   PF_CHECK(upload(ctx, g.elemnod, elemnod, (size_t)ne * nne));
@@ -643,6 +644,10 @@ struct pf_system {
   int32_t direct_mfma = 1;       // direct solve: 1 MFMA tile products, 0 the VALU form
   int32_t ke_kernel = 0;         // element matrices: 0 reference order, 1/2 isotropic split VALU/MFMA
   int32_t jmode = 0;          // J mode of the last assembly (reused by the sensitivities)
+  bool elem_matrix = false;   // val = the stiffness of g with E, nu, jmode, eliminated by the fixes and
+                              // scaled by rscale (if set): the element-by-element product applies it
+  bool rscaled = false;
+  DevBuf<double> rscale, rdiag;
   bool ubar_nonzero = false;  // some fixed DOF has a nonzero prescribed value
   // keepThisMatrixAs: named copies of the CRS values (same pattern) and the fix_eig list
   struct Kept {
@@ -662,7 +667,15 @@ struct pf_system {
 
 static inline void mark_changed(pf_system *s) {
   s->matrix_changed = true;
+  s->elem_matrix = false;
   ++s->mat_version;
+}
+
+// after the stiffness was assembled into the ZeroMatrix pattern
+static inline void mark_stiffness(pf_system *s) {
+  mark_changed(s);
+  s->elem_matrix = s->graph_crs && s->dof == 3;
+  s->rscaled = false;
 }
 
 // Dirichlet elimination (FEMSolverClass.f90:1707-1756) of the current fixes on the current
@@ -674,11 +687,20 @@ static int apply_bc(pf_system *s) {
   const bool matrix_part = s->bc_mat != s->mat_version || s->bc_fix != s->fix_version;
   PF_CHECK(pf_bc_apply(s->ctx, s->n, s->row_ptr.p, s->col_idx.p, s->val.p, s->rhs.p, s->fixed.p, s->ubar.p,
                        s->n > 0 ? (double)s->nnz / (double)s->n : 1.0));
-  if (matrix_part) mark_changed(s);
+  if (matrix_part) {
+    const bool em = s->elem_matrix;
+    mark_changed(s);
+    s->elem_matrix = em;
+  }
   s->bc_mat = s->mat_version;
   s->bc_rhs = s->rhs_version;
   s->bc_fix = s->fix_version;
   return PF_OK;
+}
+
+static ElemSource elem_source(pf_system *s) {
+  return ElemSource{&s->g, s->E.p, s->nu.p, s->jmode, s->has_fix ? s->fixed.p : nullptr,
+                    s->rscaled ? s->rscale.p : nullptr};
 }
 
 namespace {
@@ -857,7 +879,7 @@ extern "C" int pf_system_stiffness(pf_system *s, const double *E, const double *
   else PF_CHECK(pf_assemble_hex8(ctx, s->g, s->E.p, s->nu.p, jmode, s->row_ptr.p, s->val.p, s->ke_kernel));
   PF_HIP(hipStreamSynchronize(ctx->stream));
   s->jmode = jmode;
-  mark_changed(s);
+  mark_stiffness(s);
   return PF_OK;
 }
 
@@ -880,7 +902,7 @@ extern "C" int pf_system_stiffness_dev(pf_system *s, const double *E_dev, const 
   else PF_CHECK(pf_assemble_hex8(ctx, s->g, s->E.p, s->nu.p, jmode, s->row_ptr.p, s->val.p, s->ke_kernel));
   PF_HIP(hipStreamSynchronize(ctx->stream));
   s->jmode = jmode;
-  mark_changed(s);
+  mark_stiffness(s);
   return PF_OK;
 }
 
@@ -1020,8 +1042,17 @@ extern "C" int pf_system_solve(pf_system *s, const pf_solve_opts *opts, const do
     // JacobiPreconditionerCRS on CRS_val / CRS_RHS after the elimination
     // (FEMSolverClass.f90:1769-1775); the elimination stays valid (the fixed rows hold
     // a unit diagonal), re-running it is a no-op
+    const bool em = s->elem_matrix;
+    if (em) {  // the scaling the rows are about to get, on top of an earlier one
+      PF_CHECK(s->rscale.ensure((size_t)s->n));
+      PF_CHECK(s->rdiag.ensure((size_t)s->n));
+      PF_CHECK(pf_jacobi_row_scale(ctx, s->n, s->row_ptr.p, s->col_idx.p, s->val.p, s->rdiag.p));
+      PF_CHECK(pf_scale_update(ctx, s->n, s->rdiag.p, s->rscaled, s->rscale.p));
+      s->rscaled = true;
+    }
     PF_CHECK(pf_jacobi_rows(ctx, s->n, s->row_ptr.p, s->col_idx.p, s->val.p, s->rhs.p));
     mark_changed(s);
+    s->elem_matrix = em;
     ++s->rhs_version;
   }
   if (x0) {
@@ -1034,8 +1065,9 @@ extern "C" int pf_system_solve(pf_system *s, const pf_solve_opts *opts, const do
     // the reference's PointJacobi branch calls no solver: x = x0 (or zeros), then the fixed values
     res.status = PF_OK;
   } else {
+    const ElemSource es = elem_source(s);
     PF_CHECK(pf_bicgstab_device(ctx, s->work, s->n, s->row_ptr.p, s->col_idx.p, s->val.p, s->nnz, s->rhs.p,
-                                s->x.p, o, s->matrix_changed, res));
+                                s->x.p, o, s->matrix_changed, res, s->elem_matrix ? &es : nullptr));
     s->matrix_changed = false;
   }
   if (s->has_fix) PF_CHECK(pf_bc_set_fixed_x(ctx, s->n, s->fixed.p, s->ubar.p, s->x.p));
@@ -1193,6 +1225,7 @@ extern "C" int pf_system_get_x(pf_system *s, double *x) {
 extern "C" int pf_system_view_get(pf_system *s, pf_system_view *v) {
   PF_CHECK(sys_check(s, false));
   if (!v) return PF_INVALID;
+  s->elem_matrix = false;  // the caller may write the values
   v->n = s->n;
   v->nnz = s->nnz;
   v->nn = s->g.nn;
@@ -1222,6 +1255,27 @@ extern "C" int pf_system_spmv(pf_system *s, int32_t kind, const double *x, doubl
                         s->sx.p, s->sy.p, repeat, ms));
   s->matrix_changed = false;
   if (y) PF_CHECK(download(ctx, y, s->sy.p, (size_t)s->n));
+  return PF_OK;
+}
+
+extern "C" int pf_system_elem_apply(pf_system *s, const double *x, double *y) {
+  PF_CHECK(sys_check(s, true));
+  if (!x || !y) return PF_INVALID;
+  pf_ctx *ctx = s->ctx;
+  DeviceGuard guard(ctx);
+  PF_CHECK(apply_bc(s));
+  bool ok = false;
+  if (s->elem_matrix) PF_CHECK(pf_elem_plan(ctx, s->g, &ok));
+  if (!ok) {
+    pf_set_error("pf_system_elem_apply: the CRS values are not the stiffness of a hex8 mesh");
+    return PF_INVALID;
+  }
+  PF_CHECK(s->sx.ensure((size_t)s->n + 1));
+  PF_CHECK(s->sy.ensure((size_t)s->n + 1));
+  PF_CHECK(upload(ctx, s->sx, x, (size_t)s->n));
+  PF_CHECK(pf_elem_apply(ctx, elem_source(s), s->sx.p, s->sy.p));
+  PF_CHECK(download(ctx, y, s->sy.p, (size_t)s->n));
+  PF_HIP(hipStreamSynchronize(ctx->stream));
   return PF_OK;
 }
 

@@ -69,6 +69,35 @@ struct DevBuf {
 };
 
 // ---------------------------------------------------------------------------------
+// elem.hip: the tiles of the element-by-element stiffness product (elem_dev.hpp)
+struct ElemView {
+  int32_t ntile, umax;          // tiles; most slots of a tile
+  int32_t affine;               // every element is a parallelepiped
+  int64_t nn;
+  const int4 *tdesc;            // per tile: first element, elements, first slot, slots
+  const int32_t *snode;         // per slot: 0-based node; bit 29 + d set when its DOF d is fixed
+  const double *sxyz;           // per slot: coordinates, relative to the tile's first node
+  const uint4 *stab;            // per slot: its contributions a * ET + e as eight 16-bit numbers (unused: 8 ET)
+  const uint4 *lconn;           // per element: its 8 nodes as 16-bit positions in the tile's slots
+  const double2 *lamu;          // per element: lambda, mu
+  const int2 *nrec;             // per node: (its slot, 1) or (offset into nslot, slots); fixed flags in bits 29-31 of .y
+  const int32_t *nslot;         // slots per node, ascending
+  const double *rscale;         // per row scale (NULL: none)
+};
+
+struct ElemPlan {
+  bool tried = false, ok = false;  // built for the current mesh; usable
+  int32_t ntile = 0, umax = 0, affine = 0;
+  int64_t nslots = 0;
+  DevBuf<int4> tdesc;
+  DevBuf<int32_t> eperm, snode, nslot;
+  DevBuf<int2> nrec;
+  DevBuf<double> sxyz, part;
+  DevBuf<uint4> lconn, stab;
+  DevBuf<double2> lamu;
+};
+
+// ---------------------------------------------------------------------------------
 // mesh + node-level graph (row structure shared by the DOF rows of one node)
 struct NodeGraph {
   int64_t nn = 0, ne = 0;
@@ -88,7 +117,27 @@ struct NodeGraph {
   bool built = false;        // eoff/elist valid
   bool cols_built = false;   // deg/noff/ncol valid
   mutable DevBuf<double> kebuf;  // element matrices of the two-pass stiffness assembly (ne x 576)
+  ElemPlan elem;                 // tiles of the element-by-element product, built on first use
 };
+
+// a system whose matrix is exactly the eliminated stiffness of a hex8 mesh: what the
+// element-by-element product needs
+struct ElemSource {
+  NodeGraph *g = nullptr;
+  const double *E = nullptr, *nu = nullptr;
+  int jmode = 0;
+  const uint8_t *fixed = nullptr;   // per DOF (NULL: none)
+  const double *rscale = nullptr;   // row scale the matrix was multiplied by (NULL: none)
+};
+// tiles of the mesh (once per mesh); *ok = false when the mesh does not suit them
+int pf_elem_plan(pf_ctx *ctx, NodeGraph &g, bool *ok);
+// Lame constants and fixed flags of the source's current state; view of the plan
+int pf_elem_view(pf_ctx *ctx, const ElemSource &src, ElemView *v);
+// y = K x (device vectors) through the tiles
+int pf_elem_apply(pf_ctx *ctx, const ElemSource &src, const double *x, double *y);
+size_t pf_elem_lds(const ElemView &v);
+// scale = d (again: scale * d): the row scale a matrix has been multiplied by
+int pf_scale_update(pf_ctx *ctx, int64_t n, const double *d, bool again, double *scale);
 
 // blocked sliced-ELL copy of a DOF=3 CRS: 64 nodes per slice (one wavefront), slot t of
 // node l of slice s at block index (soff[s] + t)*64 + l; the 3x3 values of the slot's 64
@@ -296,7 +345,8 @@ void pf_solver_work_destroy(SolverWork *w);
 // built inside.  x holds x0 on entry.
 int pf_bicgstab_device(pf_ctx *ctx, SolverWork *w, int64_t n, const int64_t *row_ptr,
                        const int32_t *col_idx, const double *val, int64_t nnz, const double *b,
-                       double *x, const pf_solve_opts &o, bool matrix_changed, SolveResult &res);
+                       double *x, const pf_solve_opts &o, bool matrix_changed, SolveResult &res,
+                       const ElemSource *elem = nullptr);
 // bicgstab_CRS_2 (or the stop rules of stop_mode 1 and 2) in FP64 on the CRS layout with every
 // work vector, partial sum and scalar in the caller's device workspace ws (ws_doubles doubles,
 // at least pf_bicgstab_workspace_doubles(ctx, n)): no device allocation, no hipGraph; host polls
