@@ -556,6 +556,426 @@ __global__ void __launch_bounds__(BT) k_pupdate(int64_t n, V *__restrict__ p, co
   }
 }
 
+// ---- whole iterations in one kernel (small systems) --------------------------------------
+// Below about 80,000 rows an iteration of four to six launches is their latency (17-49 us); here
+// one workgroup per CU keeps its rows' matrix entries and vectors in registers, every x entry its
+// rows use (its "halo", the sorted distinct columns of RowSplit) in LDS, and iterates without
+// returning to the host.  Per iteration the workgroups publish y = A p and v = A e once each; r, p
+// and e of the halo are updated by everyone from y, v and the scalars with the owner's operations
+// (explicit fma), so the copies stay bitwise equal to the owner's values.
+//
+// Products.  A row is cut into segments of SUB entries; the block's segments, row by row, are dealt
+// to its subgroups of SUB lanes in equal runs, so a lane holds at most NREG entries whatever the
+// row lengths.  At the end of every row or run each lane leaves its sum in an LDS cell (the rank of
+// the row + the subgroup: distinct, and consecutive along a row), and the row's owner adds them up.
+//
+// Synchronisation.  Published values and the workgroups' partial sums travel through relaxed atomic
+// loads and stores at agent scope, which bypass the caches that are not coherent across the XCDs,
+// and carry their own arrival: a place holds EMPTY (a NaN no arithmetic produces) until its value
+// is stored, and readers poll it.  Three sums per iteration (r0.y; e.v, v.v; r.r, r0.r) keep the
+// workgroups within one sum of each other.  Places take turns and are emptied in between:
+//  * sums: eight buffers; at sum s a workgroup empties its place of sum s + 4, last read by anyone
+//    before sum s - 3 completed;
+//  * y and v: two buffers each, by iteration parity; those of iteration k + 1 are emptied after the
+//    first sum of iteration k, when everyone is done with those of k - 1.
+// Every wave waits for its emptying stores (vmcnt 0) before the workgroup barrier that precedes the
+// store of the iteration's third sum; the next turn of a place is read only after the sum that
+// follows such a wait, so nobody can still see its old value.
+// No fence: an agent-scope acquire would empty the caches (measured, 256 workgroups: 10 us per
+// barrier with release/acquire, 2.5 us without).
+// The launch is cooperative, so all workgroups are resident.  Polls are bounded all the same: a
+// workgroup that gives up raises *fail and ends, the others follow, and the host starts over with
+// the launches above.
+constexpr int PT = 512;  // threads of a workgroup: 256 registers each, half of them for the matrix
+constexpr unsigned long long EMPTY = 0xfff8dead5107e317ull;
+constexpr int POLLS = 1 << 17;                                    // about 0.1 s
+constexpr int PG_MAX = 1024;                                      // workgroups a sum's buffer holds
+constexpr int SUM_WORDS = 8 * 2 * PG_MAX;                         // buffers x sums x workgroups
+
+struct PersistArgs {
+  int64_t n;
+  const int64_t *row_ptr;
+  const double *val;
+  const uint16_t *lidx;
+  const int32_t *roff, *ucnt, *ucol;
+  int umax, maxrows;           // most halo entries and rows of a workgroup
+  double *x, *r, *p;           // state between launches
+  const double *r0;
+  unsigned long long *yg, *vg; // published products, 2 n each
+  unsigned long long *sums;
+  Scal *sc;
+  int32_t *fail;
+  int32_t most;                // iterations of this launch
+};
+
+__device__ inline void put(unsigned long long *p, double d) {
+  unsigned long long v = (unsigned long long)__double_as_longlong(d);
+  if (v == EMPTY) v = 0x7ff8000000000000ull;
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+__device__ inline void empty(unsigned long long *p) {
+  __hip_atomic_store(p, EMPTY, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// out[k] = *at(k) for k < cnt <= N, all of them awaited together
+template <int N, typename F>
+__device__ inline void take(F at, int cnt, double (&out)[N], int &bad) {
+  unsigned long long v[N];
+  int polls = 0;
+  bool more;
+  do {
+    more = false;
+#pragma unroll
+    for (int k = 0; k < N; ++k)
+      v[k] = k < cnt ? __hip_atomic_load(at(k), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0ull;
+#pragma unroll
+    for (int k = 0; k < N; ++k) more = more || v[k] == EMPTY;
+  } while (more && ++polls < POLLS);
+  if (more) bad = 1;
+#pragma unroll
+  for (int k = 0; k < N; ++k) out[k] = __longlong_as_double((long long)v[k]);
+}
+
+// sum over the wavefront in lane 63 (row shifts and row broadcasts: no LDS permutes), then in all
+template <int CTRL, int ROWS>
+__device__ inline double dpp_add(double x) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), CTRL, ROWS, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), CTRL, ROWS, 0xf, true);
+  return x + __hiloint2double(hi, lo);
+}
+__device__ inline double wave_total(double x) {
+  x = dpp_add<0x111, 0xf>(x);  // row_shr:1, 2, 4, 8: sums of 16 in lanes 15, 31, 47, 63
+  x = dpp_add<0x112, 0xf>(x);
+  x = dpp_add<0x114, 0xf>(x);
+  x = dpp_add<0x118, 0xf>(x);
+  x = dpp_add<0x142, 0xa>(x);  // row_bcast:15 into rows 1 and 3
+  x = dpp_add<0x143, 0xc>(x);  // row_bcast:31 into rows 2 and 3
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(x), 63),
+                          __builtin_amdgcn_readlane(__double2loint(x), 63));
+}
+
+constexpr int PW = PT / 64;                      // wavefronts
+constexpr int PH = pfdev::ST_UMAX / PT;          // halo entries of a thread
+constexpr int PG_LANE = 8;                       // workgroups' sums a lane of the first wave awaits at once
+
+// d summed over all threads of all workgroups, the same value in every thread; `between` runs after
+// this workgroup's sum is out and before the others' are awaited; false when a poll gave up
+template <int NV, typename F>
+__device__ inline bool all_sum(const PersistArgs &a, unsigned seq, double (&d)[NV], double (&red)[2][PW + 1], int &bad,
+                               F between) {
+  const int tid = threadIdx.x, G = gridDim.x;
+#pragma unroll
+  for (int k = 0; k < NV; ++k) {
+    const double t = wave_total(d[k]);
+    if ((tid & 63) == 0) red[k][tid >> 6] = t;
+  }
+  __syncthreads();
+  unsigned long long *buf = a.sums + (size_t)(seq & 7) * (2 * PG_MAX);
+  if (tid < 64) {
+    double t[NV];
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+      t[k] = red[k][0];
+#pragma unroll
+      for (int w = 1; w < PW; ++w) t[k] += red[k][w];
+    }
+    if (tid == 0) {
+#pragma unroll
+      for (int k = 0; k < NV; ++k) {
+        if (G > 1) put(buf + k * PG_MAX + blockIdx.x, t[k]);
+        else red[k][PW] = t[k];
+      }
+      if (G > 1) {
+        unsigned long long *next = a.sums + (size_t)((seq + 4) & 7) * (2 * PG_MAX);
+#pragma unroll
+        for (int k = 0; k < 2; ++k) empty(next + k * PG_MAX + blockIdx.x);
+      }
+    }
+  }
+  between();
+  if (G > 1 && tid < 64) {
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+      double t = 0.0;
+      for (int g0 = 0; g0 < G; g0 += 64 * PG_LANE) {
+        double got[PG_LANE];
+        const int left = G - g0 - tid;  // this lane's workgroups: g0 + tid + 64 i
+        take<PG_LANE>([&](int i) { return buf + k * PG_MAX + g0 + tid + 64 * i; }, left > 0 ? (left + 63) / 64 : 0,
+                      got, bad);
+#pragma unroll
+        for (int i = 0; i < PG_LANE; ++i) t += got[i];
+      }
+      t = wave_total(t);
+      if (tid == 0) red[k][PW] = t;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < NV; ++k) d[k] = red[k][PW];
+  if (bad) {
+    if (tid == 0) *a.fail = 1;
+    return false;
+  }
+  return true;
+}
+
+template <int SUB, int NREG>
+__global__ void __launch_bounds__(PT) k_persist(PersistArgs a) {
+  static_assert(NREG <= 32, "ends has a bit per segment");
+  constexpr int NSG = PT / SUB;
+  constexpr int CS = SUB + 1;  // stride of a cell: lanes of a wave read different banks
+  extern __shared__ double psh[];
+  __shared__ double red[2][PW + 1];
+  __shared__ int bad;
+  const int tid = threadIdx.x, b = blockIdx.x;
+  Scal *sc = a.sc;
+  if (sc->done) return;
+  const int row0 = a.roff[b], rows = a.roff[b + 1] - row0;
+  const int U = a.ucnt[b];
+  double *hp = psh, *he = hp + a.umax, *cell = he + a.umax;
+  // rows + 1: segments before a row, and in the upper bits the rows with entries before it
+  int *first = reinterpret_cast<int *>(cell + (size_t)(a.maxrows + NSG) * CS);
+  const bool own = tid < rows;
+  const int64_t gi = row0 + tid;
+  if (tid == 0) {
+    bad = 0;
+    first[0] = 0;
+  }
+  if (own) {
+    const int s = (int)((a.row_ptr[gi + 1] - a.row_ptr[gi] + SUB - 1) / SUB);
+    first[tid + 1] = s > 0 ? s | (1 << 20) : 0;
+  }
+  __syncthreads();
+  for (int off = 1; off < rows; off <<= 1) {
+    const int add = own && tid >= off ? first[tid + 1 - off] : 0;
+    __syncthreads();
+    if (own) first[tid + 1] += add;
+    __syncthreads();
+  }
+  constexpr int SEG = (1 << 20) - 1;
+  const int nseg = first[rows] & SEG;
+  const int Q = (nseg + NSG - 1) / NSG;  // segments per subgroup, at most NREG
+  const int sg = tid / SUB, sub = tid % SUB;
+  const int q0 = sg * Q < nseg ? sg * Q : nseg, q1 = q0 + Q < nseg ? q0 + Q : nseg;
+  int row = 0;  // row of segment q0: the last one with first <= q0 (a row without entries has none)
+  for (int hi = rows; hi - row > 1;) {
+    const int mid = (row + hi) >> 1;
+    if ((first[mid] & SEG) <= q0) row = mid; else hi = mid;
+  }
+  // this lane's entries; bit j of ends: segment j closes its row or this subgroup's run
+  double mv[NREG];
+  uint32_t mi[(NREG + 1) / 2];
+  uint32_t ends = 0;
+  const int cell0 = ((rows > 0 ? first[row] >> 20 : 0) + sg) * CS + sub;
+  {
+    int64_t k0 = 0, k1 = 0;
+    int at = 0;
+#pragma unroll
+    for (int j = 0; j < NREG; ++j) {
+      mv[j] = 0.0;
+      uint32_t ix = 0;
+      const int q = q0 + j;
+      if (q < q1) {
+        const bool next = j > 0 && q == (first[row + 1] & SEG);
+        if (next) do ++row; while (q >= (first[row + 1] & SEG));
+        if (j == 0 || next) {
+          k0 = a.row_ptr[row0 + row] - 1;
+          k1 = a.row_ptr[row0 + row + 1] - 1;
+          at = q - (first[row] & SEG);
+        }
+        const int64_t k = k0 + (int64_t)at * SUB + sub;
+        if (k < k1) {
+          mv[j] = a.val[k];
+          ix = a.lidx[k];
+        }
+        ++at;
+        if (q + 1 == (first[row + 1] & SEG) || q + 1 == q1) ends |= 1u << j;
+      }
+      if (j & 1) mi[j / 2] |= ix << 16;
+      else mi[j / 2] = ix;
+    }
+  }
+  // the cells of this thread's row
+  int c0 = 0, cn = 0;
+  if (own) {
+    const int f0 = first[tid] & SEG, f1 = first[tid + 1] & SEG;
+    if (f1 > f0) {
+      c0 = ((first[tid] >> 20) + f0 / Q) * CS;
+      cn = (f1 - 1) / Q - f0 / Q + 1;
+    }
+  }
+  const auto product = [&](const double *xs) {
+    double acc = 0.0;
+    int c = cell0;
+#pragma unroll
+    for (int j = 0; j < NREG; ++j) {
+      const uint32_t ix = (j & 1) ? mi[j / 2] >> 16 : mi[j / 2] & 0xffffu;
+      acc = __builtin_fma(mv[j], xs[ix], acc);
+      if (ends & (1u << j)) {
+        cell[c] = acc;
+        c += CS;
+        acc = 0.0;
+      }
+    }
+    __syncthreads();
+    double s = 0.0;
+    for (int k = 0; k < cn; ++k) {
+      const double *q = cell + c0 + k * CS;
+      double h[SUB];
+#pragma unroll
+      for (int l = 0; l < SUB; ++l) h[l] = q[l];
+#pragma unroll
+      for (int o = 1; o < SUB; o *= 2)
+#pragma unroll
+        for (int l = 0; l < SUB; l += 2 * o) h[l] += h[l + o];
+      s += h[0];
+    }
+    return s;
+  };
+  double r = 0.0, p = 0.0, x = 0.0, r0 = 0.0, y = 0.0, v = 0.0, e = 0.0;
+  if (own) {
+    r = a.r[gi];
+    p = a.p[gi];
+    x = a.x[gi];
+    r0 = a.r0[gi];
+  }
+  // this thread's share of the halo: entries tid + k PT
+  const int hn = U > tid ? (U - tid + PT - 1) / PT : 0;
+  int32_t hc[PH];
+  double hr[PH], hy[PH];
+#pragma unroll
+  for (int k = 0; k < PH; ++k) {
+    hc[k] = k < hn ? a.ucol[(int64_t)b * pfdev::ST_UMAX + tid + k * PT] : 0;
+    hr[k] = hy[k] = 0.0;
+    if (k < hn) {
+      hr[k] = a.r[hc[k]];
+      hp[tid + k * PT] = a.p[hc[k]];
+    }
+  }
+  // the scalars, the same in every thread of every workgroup throughout
+  double cc1 = sc->c1, rr1 = sc->rr1, rr = sc->rr;
+  const int mode = sc->stop_mode, guard = sc->guard, itrmax = sc->itrmax;
+  int itr = sc->itr_last, status = PF_NOT_CONVERGED, done = 0;
+  unsigned seq = 0;
+  __syncthreads();
+  for (int it = 0; it < a.most; ++it) {
+    const int64_t now = it & 1 ? a.n : 0, other = it & 1 ? 0 : a.n;
+    double d1[1] = {0.0}, d2[2] = {0.0, 0.0};
+    y = product(hp);
+    if (own) {
+      put(a.yg + now + gi, y);
+      d1[0] = r0 * y;
+    }
+    if (!all_sum<1>(a, seq++, d1, red, bad,
+                    [&] { take<PH>([&](int k) { return a.yg + now + hc[k]; }, hn, hy, bad); }))
+      return;
+    const double c2 = d1[0], alpha = cc1 / c2;
+    if (guard && !isfinite(alpha)) {  // r0.Ap lost: stop before x is touched
+      status = PF_BREAKDOWN_C2C3;
+      done = 1;
+      break;
+    }
+    if (own) {  // the other buffers, for the next iteration
+      empty(a.yg + other + gi);
+      empty(a.vg + other + gi);
+    }
+    e = __builtin_fma(-alpha, y, r);
+#pragma unroll
+    for (int k = 0; k < PH; ++k) {
+      hr[k] = __builtin_fma(-alpha, hy[k], hr[k]);  // e of the halo
+      if (k < hn) he[tid + k * PT] = hr[k];
+    }
+    __syncthreads();
+    v = product(he);
+    if (own) {
+      put(a.vg + now + gi, v);
+      d2[0] = e * v;
+      d2[1] = v * v;
+    }
+    double hv[PH];
+    if (!all_sum<2>(a, seq++, d2, red, bad,
+                    [&] { take<PH>([&](int k) { return a.vg + now + hc[k]; }, hn, hv, bad); }))
+      return;
+    if (d2[1] == 0.0) {  // "Bicgstab devide by zero" (FEMSolverClass.f90:2266)
+      status = PF_BREAKDOWN_VV;
+      done = 1;
+      break;
+    }
+    const double omega = d2[0] / d2[1];
+    if (guard && !isfinite(omega)) {
+      status = PF_BREAKDOWN_VV;
+      done = 1;
+      break;
+    }
+    x = __builtin_fma(omega, e, __builtin_fma(alpha, p, x));
+    r = __builtin_fma(-omega, v, e);
+    d2[0] = own ? r * r : 0.0;
+    d2[1] = own ? r0 * r : 0.0;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the emptied places are empty for everyone
+    if (!all_sum<2>(a, seq++, d2, red, bad, [&] {
+#pragma unroll
+          for (int k = 0; k < PH; ++k) hr[k] = __builtin_fma(-omega, hv[k], hr[k]);
+        }))
+      return;
+    rr = d2[0];
+    ++itr;
+    if (itr == 1) rr1 = rr;
+    bool stop;
+    if (mode == 0)  // FEMSolverClass.f90:2275-2289
+      stop = (sqrt(rr / rr1) < sc->rel) || (sqrt(rr) < sc->er0);
+    else if (mode == 1)
+      stop = sqrt(rr) < sc->rel * sqrt(sc->bnorm2);
+    else  // bicgstab_CRS: rr / init_rr < er, no square root (:1561)
+      stop = rr / sc->rr0 < sc->er0;
+    if (stop) {
+      status = PF_OK;
+      done = 1;
+      break;
+    }
+    const double c2w = c2 * omega, beta = d2[1] / c2w;
+    if (c2w == 0.0 || (guard && !(isfinite(beta) && isfinite(rr)))) {  // FEMSolverClass.f90:2295
+      status = PF_BREAKDOWN_C2C3;
+      done = 1;
+      break;
+    }
+    if (itr >= itrmax) {
+      done = 1;
+      break;
+    }
+    cc1 = d2[1];
+    p = __builtin_fma(beta, __builtin_fma(-omega, y, p), r);
+#pragma unroll
+    for (int k = 0; k < PH; ++k)
+      if (k < hn) {
+        double &q = hp[tid + k * PT];
+        q = __builtin_fma(beta, __builtin_fma(-omega, hy[k], q), hr[k]);
+      }
+    __syncthreads();
+  }
+  if (own) {
+    a.x[gi] = x;
+    a.r[gi] = r;
+    a.p[gi] = p;
+  }
+  if (b == 0 && tid == 0) {
+    sc->c1 = cc1;
+    sc->rr = rr;
+    sc->rr1 = rr1;
+    sc->itr_last = itr;
+    sc->status = status;
+    sc->done = done;
+  }
+}
+
+__global__ void k_persist_empty(int64_t n, unsigned long long *__restrict__ sums, unsigned long long *__restrict__ yv,
+                                int32_t *__restrict__ fail) {
+  const int64_t i = blockIdx.x * (int64_t)256 + threadIdx.x;
+  if (i < SUM_WORDS) sums[i] = EMPTY;
+  if (i < 4 * n) yv[i] = EMPTY;
+  if (i == 0) *fail = 0;
+}
+
 // ---- bicgstab_CRS_ILU (LinearSolverClass.f90:4104-4229) ---------------------------------
 // Right-preconditioned: pd = M^-1 p and ps = M^-1 e come from the level-scheduled sweeps
 // (the p update and e = r - alpha y are formed inside them), so one iteration is
@@ -803,9 +1223,14 @@ struct SolverWork {
   Sell3<double> s64;
   Sell3<float> s32;
   CrsStage stage;  // CRS product with x staged in LDS per row block
+  RowSplit split;  // the one-kernel iterations' rows per workgroup
+  DevBuf<unsigned long long> sums, published;
+  DevBuf<int32_t> pfail;
+  int32_t *h_fail = nullptr;
   DevBuf<int32_t> flag;
   DevBuf<double> jscale;  // FP32 system row scale: 1/sqrt|a_ii| (symmetric) or 1/a_ii (row)
   DevBuf<double> jones;   // column scale of the row-scaled form
+  DevBuf<double> xstart;  // x0 of a solve in one kernel
   DevBuf<double> escale;  // element form: product of the matrix's own row scale and jscale
   // ILU(0) form: the factor is kept across solves, as FEMSolver_%ILU_MATRIX is
   // (FEMSolverClass.f90:1777-1784), until pf_ilu_reset
@@ -829,6 +1254,7 @@ struct SolverWork {
     if (gexec_ilu) (void)hipGraphExecDestroy(gexec_ilu);
     for (hipEvent_t e : evs) (void)hipEventDestroy(e);
     if (h_sc) (void)hipHostFree(h_sc);
+    if (h_fail) (void)hipHostFree(h_fail);
   }
 };
 
@@ -1131,6 +1557,121 @@ int run_loop(pf_ctx *ctx, SolverWork *w, int slot, const Launch &L, const Mat<V,
   return PF_OK;
 }
 
+// ---- one-kernel iterations ---------------------------------------------------------------
+// Microseconds per iteration, one kernel / CRS rows / blocked or (73k rows) element tiles, Cube3D on
+// MI355X: 1029 rows 8.2 / 18 / 28, 10k 8.7 / 21 / 38, 28k 10.8 / 30 / 43, 47k 12.3 / 39 / 46 (tiles 31).
+// Above, the entries do not fit the registers of 256 workgroups (16384 each).
+// Below 64 rows the launches stay: systems of a few rows end by finite termination, where one
+// rounding decides the iteration count, and theirs ends where the reference's does.
+constexpr int64_t PERSIST_MIN_ROWS = 64, PERSIST_MAX_ROWS = 100000;
+constexpr int PERSIST_CHUNK = 4096;  // iterations of a launch (tens of milliseconds)
+
+// the kernel for `sub` lanes per segment and at least `need` segments per subgroup
+const void *persist_kernel(int sub, int need) {
+#define PF_PERSIST_CASE(S)                                        \
+  if (sub == S) {                                                 \
+    if (need <= 8) return (const void *)k_persist<S, 8>;          \
+    if (need <= 16) return (const void *)k_persist<S, 16>;        \
+    if (need <= 24) return (const void *)k_persist<S, 24>;        \
+    if (need <= 32) return (const void *)k_persist<S, 32>;        \
+  }
+  PF_PERSIST_CASE(4)
+  PF_PERSIST_CASE(8)
+  PF_PERSIST_CASE(16)
+#undef PF_PERSIST_CASE
+  return nullptr;
+}
+
+int persist_segments(const RowSplit &p) {
+  const int nsg = PT / p.sub;
+  return (p.maxslots + nsg - 1) / nsg;
+}
+
+size_t persist_lds(const RowSplit &p) {
+  return sizeof(double) * ((size_t)2 * p.umax + (size_t)(p.maxrows + PT / p.sub) * (p.sub + 1)) +
+         sizeof(int) * ((size_t)p.maxrows + 2);
+}
+
+// the split of the rows (once per matrix): *ok = false when the system does not suit it
+int persist_prepare(pf_ctx *ctx, SolverWork *w, int64_t n, const int64_t *row_ptr, const int32_t *col_idx, int64_t nnz,
+                    bool *ok) {
+  *ok = false;
+  if (n < PERSIST_MIN_ROWS || n > PERSIST_MAX_ROWS || nnz < 1) return PF_OK;
+  RowSplit &p = w->split;
+  if (!p.ready) {
+    const double avg = (double)nnz / (double)n;
+    const int sub = avg <= 24.0 ? 4 : (avg <= 160.0 ? 8 : 16);
+    // a system that one workgroup's registers hold needs no exchange at all; otherwise 2048 entries
+    // per workgroup (1029 rows: 8.2 us per iteration, 8.9 with 4096, 10.1 with 8192), at most one
+    // workgroup per CU
+    int64_t G = nnz <= 16384 && n <= PT ? 1 : (nnz + 2047) / 2048;
+    if (G > ctx->num_cus) G = ctx->num_cus;
+    if (G > PG_MAX) G = PG_MAX;
+    if (G > n) G = n;
+    PF_CHECK(pf_row_split_build(ctx, n, row_ptr, col_idx, nnz, (int)G, sub, p));
+    p.ready = true;
+  }
+  *ok = p.staged && p.maxrows <= PT && persist_kernel(p.sub, persist_segments(p)) && persist_lds(p) <= 140 * 1024;
+  return PF_OK;
+}
+
+// the iterations of scalars slot 0 to their stop; *ran = false when the workgroups could not run
+// together (nothing is lost but x, r and p, which the caller sets up again)
+int run_persist(pf_ctx *ctx, SolverWork *w, int64_t n, const int64_t *row_ptr, const double *val, double *x,
+                const pf_solve_opts &o, bool *ran) {
+  *ran = false;
+  const RowSplit &p = w->split;
+  PF_CHECK(w->sums.ensure(SUM_WORDS));
+  PF_CHECK(w->published.ensure(4 * (size_t)n));
+  PF_CHECK(w->pfail.ensure(1));
+  if (!w->h_fail) PF_HIP(hipHostMalloc((void **)&w->h_fail, sizeof(int32_t), hipHostMallocDefault));
+  PersistArgs a{};
+  a.n = n;
+  a.row_ptr = row_ptr;
+  a.val = val;
+  a.lidx = p.lidx.p;
+  a.roff = p.info.p;
+  a.ucnt = p.info.p + p.G + 1;
+  a.ucol = p.ucol.p;
+  a.umax = p.umax;
+  a.maxrows = p.maxrows;
+  a.x = x;
+  a.r = w->r.p;
+  a.p = w->p.p;
+  a.r0 = w->r0.p;
+  a.yg = w->published.p;
+  a.vg = w->published.p + 2 * n;
+  a.sums = w->sums.p;
+  a.sc = w->sc.p;
+  a.fail = w->pfail.p;
+  a.most = o.debug && o.check_every > 0 ? o.check_every : PERSIST_CHUNK;
+  const size_t lds = persist_lds(p);
+  const void *kernel = persist_kernel(p.sub, persist_segments(p));
+  Scal *hs = w->h_sc;
+  for (;;) {
+    k_persist_empty<<<pf_blocks(std::max<int64_t>(SUM_WORDS, 4 * n), 256, INT32_MAX), 256, 0, ctx->stream>>>(
+        n, w->sums.p, w->published.p, w->pfail.p);
+    PF_HIP(hipGetLastError());
+    void *args[] = {&a};
+    hipError_t e = hipSuccess;
+    if (lds > 64 * 1024) e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e == hipSuccess)
+      e = hipLaunchCooperativeKernel(kernel, dim3((unsigned)p.G), dim3(PT), args, (unsigned)lds, ctx->stream);
+    if (e != hipSuccess) {  // e.g. fewer CUs available to this process: the launches then
+      (void)hipGetLastError();
+      return PF_OK;
+    }
+    PF_HIP(hipMemcpyAsync(hs, w->sc.p, sizeof(Scal), hipMemcpyDeviceToHost, ctx->stream));
+    PF_HIP(hipMemcpyAsync(w->h_fail, w->pfail.p, sizeof(int32_t), hipMemcpyDeviceToHost, ctx->stream));
+    PF_HIP(hipStreamSynchronize(ctx->stream));
+    if (*w->h_fail) return PF_OK;
+    if (o.debug) std::printf("BiCGSTAB >> itr %d  sqrt(rr) %.6e\n", hs->itr_last, std::sqrt(hs->rr));
+    if (hs->done) break;
+  }
+  *ran = true;
+  return PF_OK;
+}
+
 int prepare_scalars(pf_ctx *ctx, SolverWork *w, int slot, const pf_solve_opts &o, int itrmax, double rel,
                     int stop_mode, int hist_cap, int guard, int stall = 0) {
   Scal h;
@@ -1157,7 +1698,7 @@ void note_matrix(SolverWork *w, int64_t n, const double *val, bool &matrix_chang
   w->key_val = val;
   if (matrix_changed) {
     w->have_s64 = w->have_s32 = w->have_v32 = w->have_scale = false;
-    w->stage.ready = false;
+    w->stage.ready = w->split.ready = false;
     w->block_ok = -1;
     std::memset(w->gkey, 0, sizeof(w->gkey));
   }
@@ -1413,7 +1954,10 @@ int pf_bicgstab_device(pf_ctx *ctx, SolverWork *w, int64_t n, const int64_t *row
   // the options ask for a matrix layout, the ILU factor or the symmetric scaling
   ElemView ev{};
   double *epart = nullptr;
-  if (elem && o.spmv_kind == 0 && n >= ELEM_MIN_ROWS && o.preconditioning != 2 &&
+  bool persist = false;
+  if (o.spmv_kind == 0 && o.precision == 64 && o.preconditioning != 2 && o.kernel_timing == 0)
+    PF_CHECK(persist_prepare(ctx, w, n, row_ptr, col_idx, nnz, &persist));
+  if (!persist && elem && o.spmv_kind == 0 && n >= ELEM_MIN_ROWS && o.preconditioning != 2 &&
       (o.precision == 64 || ((o.precision == 48 || o.precision == 32) && (o.jacobi == 0 || o.jacobi == 2)))) {
     bool ok = false;
     PF_CHECK(pf_elem_plan(ctx, *elem->g, &ok));
@@ -1423,7 +1967,7 @@ int pf_bicgstab_device(pf_ctx *ctx, SolverWork *w, int64_t n, const int64_t *row
       layout = 3;
     }
   }
-  if (layout != 3 && o.spmv_kind != 1 && o.spmv_kind != 4) {
+  if (!persist && layout != 3 && o.spmv_kind != 1 && o.spmv_kind != 4) {
     PF_CHECK(check_blocks(ctx, w, n, row_ptr, col_idx));
     layout = w->block_ok ? 1 : 0;
     if (o.spmv_kind == 2 && !layout) {
@@ -1503,7 +2047,7 @@ int pf_bicgstab_device(pf_ctx *ctx, SolverWork *w, int64_t n, const int64_t *row
     pf_set_error("spmv_kind 4 (x staged in LDS) runs the FP64 solve without ILU only");
     return PF_INVALID;
   }
-  if (layout == 0 && !refined && !ilu && (o.spmv_kind == 4 || (o.spmv_kind == 0 && n >= ((int64_t)1 << 18)))) {
+  if (!persist && layout == 0 && !refined && !ilu && (o.spmv_kind == 4 || (o.spmv_kind == 0 && n >= ((int64_t)1 << 18)))) {
     if (!w->stage.ready) PF_CHECK(pf_crs_stage_build(ctx, n, row_ptr, col_idx, nnz, w->stage));
     layout = 2;
   }
@@ -1562,8 +2106,20 @@ int pf_bicgstab_device(pf_ctx *ctx, SolverWork *w, int64_t n, const int64_t *row
       PF_CHECK(w->e.ensure(n));
       ebuf = w->e.p;
     }
-    PF_CHECK(run_loop<double>(ctx, w, 0, L64, m64, x, w->r.p, w->r0.p, w->p.p, w->y.p, w->v.p, nullptr, o, nullptr,
-                              ebuf));
+    bool ran = false;
+    if (persist) {
+      PF_CHECK(w->xstart.ensure(n));
+      PF_HIP(hipMemcpyAsync(w->xstart.p, x, sizeof(double) * n, hipMemcpyDeviceToDevice, ctx->stream));
+      PF_CHECK(run_persist(ctx, w, n, row_ptr, val, x, o, &ran));
+      if (!ran) {  // from the start again, by launches
+        PF_HIP(hipMemcpyAsync(x, w->xstart.p, sizeof(double) * n, hipMemcpyDeviceToDevice, ctx->stream));
+        PF_CHECK(prepare_scalars(ctx, w, 0, o, o.itrmax, o.relative_er, kmode, 0, guard));
+        PF_CHECK(enqueue_init<double>(ctx, L64, m64, b, x, w->r.p, w->r0.p, w->p.p, w->sc.p, w->part.p, false));
+      }
+    }
+    if (!ran)
+      PF_CHECK(run_loop<double>(ctx, w, 0, L64, m64, x, w->r.p, w->r0.p, w->p.p, w->y.p, w->v.p, nullptr, o, nullptr,
+                                ebuf));
     const Scal &h = w->h_sc[0];
     res.status = h.status;
     // the reference's loop counter: a v.v == 0 stop happens inside iteration itr+1

@@ -269,6 +269,20 @@ struct CrsStage {
 };
 int pf_crs_stage_build(pf_ctx *ctx, int64_t n, const int64_t *row_ptr, const int32_t *col_idx, int64_t nnz,
                        CrsStage &st);
+// A CRS split into G blocks of consecutive rows with about the same number of entries each: per
+// block its rows roff[b] .. roff[b+1]-1, sorted distinct columns (ucnt[b] of them at
+// ucol[b * ST_UMAX], -1: too many) and row segments of `sub` entries; per entry the position of its
+// column in its block's list.
+struct RowSplit {
+  int G = 0, sub = 0, maxrows = 0, maxslots = 0, umax = 0;
+  bool staged = false;   // every block has its list
+  bool ready = false;
+  DevBuf<int32_t> info;  // roff (G + 1), ucnt (G), segments (G)
+  DevBuf<int32_t> ucol;
+  DevBuf<uint16_t> lidx;
+};
+int pf_row_split_build(pf_ctx *ctx, int64_t n, const int64_t *row_ptr, const int32_t *col_idx, int64_t nnz, int G,
+                       int sub, RowSplit &p);
 // y = A x (accumulate: y += A x), the sums of pf_spmv_crs_launch bitwise (same subgroup width,
 // same per-lane order), x read from the staged copies
 template <typename V>

@@ -1,4 +1,5 @@
 // spmv.hip -- y = A x kernels and the blocked (Sell3) layout built from a DOF=3 CRS.
+#include <algorithm>
 #include <vector>
 
 #include "spmv_dev.hpp"
@@ -256,12 +257,14 @@ __device__ inline int block_excl_scan(int v, int *sh, int &total) {
 // probe run of ST_PROBE).  FILL sorts them (bitonic, <= ST_UMAX), writes them to
 // ucol[ubase[b] ..] and every entry's rank among them to lidx; a block whose insertion now
 // needs too long a probe run is marked unstaged instead (slot placement depends on the order
-// of the atomics; the set of columns and hence the sorted list do not).
+// of the atomics; the set of columns and hence the sorted list do not).  roff (FILL only, in one
+// pass without COUNT): block b holds rows roff[b] .. roff[b+1]-1 and its list starts at b * ST_UMAX.
 template <bool FILL>
 __global__ void __launch_bounds__(ST_T) k_stage_build(int64_t n, int rpb, const int64_t *__restrict__ row_ptr,
                                                       const int32_t *__restrict__ col_idx, int32_t *__restrict__ ucnt,
                                                       const int64_t *__restrict__ ubase, int32_t *__restrict__ ucol,
-                                                      uint16_t *__restrict__ lidx) {
+                                                      uint16_t *__restrict__ lidx,
+                                                      const int32_t *__restrict__ roff = nullptr) {
   __shared__ int32_t key[ST_HASH];
   __shared__ int32_t rank[FILL ? ST_HASH : 1];
   __shared__ int32_t srt[FILL ? pfdev::ST_UMAX : 1];
@@ -269,9 +272,9 @@ __global__ void __launch_bounds__(ST_T) k_stage_build(int64_t n, int rpb, const 
   __shared__ int ovf;
   const int tid = threadIdx.x;
   const int64_t b = blockIdx.x;
-  if (FILL && ucnt[b] < 0) return;  // whole block
-  const int64_t r0 = b * rpb;
-  const int64_t r1 = r0 + rpb < n ? r0 + rpb : n;
+  if (FILL && !roff && ucnt[b] < 0) return;  // whole block
+  const int64_t r0 = roff ? roff[b] : b * rpb;
+  const int64_t r1 = roff ? roff[b + 1] : (r0 + rpb < n ? r0 + rpb : n);
   const int64_t k0 = row_ptr[r0] - 1, k1 = row_ptr[r1] - 1;
   for (int i = tid; i < ST_HASH; i += ST_T) key[i] = -1;
   if (tid == 0) ovf = 0;
@@ -297,6 +300,7 @@ __global__ void __launch_bounds__(ST_T) k_stage_build(int64_t n, int rpb, const 
     if (tid == 0) ucnt[b] = staged ? total : -1;
     return;
   }
+  if (roff && tid == 0) ucnt[b] = total;
   int pos = ex;
   for (int i = 0; i < CH; ++i) {
     const int32_t c = key[tid * CH + i];
@@ -320,7 +324,7 @@ __global__ void __launch_bounds__(ST_T) k_stage_build(int64_t n, int rpb, const 
       }
       __syncthreads();
     }
-  int32_t *uc = ucol + ubase[b];
+  int32_t *uc = ucol + (roff ? b * pfdev::ST_UMAX : ubase[b]);
   for (int i = tid; i < total; i += ST_T) {
     const int32_t c = srt[i];
     uc[i] = c;
@@ -454,6 +458,62 @@ int pf_crs_stage_build(pf_ctx *ctx, int64_t n, const int64_t *row_ptr, const int
   for (int32_t c : h) st.staged += c >= 0;
   st.unique = total;
   st.ready = true;
+  return PF_OK;
+}
+
+namespace {
+// first row of every block: entries split evenly (row ends at or after b * nnz / G)
+__global__ void k_row_split(int64_t n, int64_t nnz, int G, const int64_t *__restrict__ row_ptr,
+                            int32_t *__restrict__ roff) {
+  const int b = blockIdx.x * blockDim.x + threadIdx.x;
+  if (b > G) return;
+  const int64_t want = nnz / G * b + nnz % G * b / G;
+  int64_t lo = 0, hi = n;  // first row with row_ptr[row] - 1 >= want
+  while (lo < hi) {
+    const int64_t mid = (lo + hi) >> 1;
+    if (row_ptr[mid] - 1 >= want) hi = mid; else lo = mid + 1;
+  }
+  roff[b] = b == G ? (int32_t)n : (b == 0 ? 0 : (int32_t)lo);
+}
+
+// per block: its row segments of `sub` entries
+__global__ void __launch_bounds__(ST_T) k_row_slots(int sub, const int64_t *__restrict__ row_ptr,
+                                                    const int32_t *__restrict__ roff, int32_t *__restrict__ slots) {
+  __shared__ int sh[ST_T];
+  int s = 0;
+  for (int r = roff[blockIdx.x] + threadIdx.x; r < roff[blockIdx.x + 1]; r += ST_T)
+    s += (int)((row_ptr[r + 1] - row_ptr[r] + sub - 1) / sub);
+  int total = 0;
+  block_excl_scan(s, sh, total);
+  if (threadIdx.x == 0) slots[blockIdx.x] = total;
+}
+}  // namespace
+
+int pf_row_split_build(pf_ctx *ctx, int64_t n, const int64_t *row_ptr, const int32_t *col_idx, int64_t nnz, int G,
+                       int sub, RowSplit &p) {
+  hipStream_t st = ctx->stream;
+  p.G = G;
+  p.sub = sub;
+  p.maxrows = p.maxslots = p.umax = 0;
+  PF_CHECK(p.info.ensure((size_t)3 * G + 1));  // roff (G + 1), ucnt (G), slots (G)
+  PF_CHECK(p.ucol.ensure((size_t)G * pfdev::ST_UMAX));
+  PF_CHECK(p.lidx.ensure((size_t)nnz + 1));
+  int32_t *roff = p.info.p, *ucnt = roff + G + 1, *slots = ucnt + G;
+  k_row_split<<<pf_blocks(G + 1, 256), 256, 0, st>>>(n, nnz, G, row_ptr, roff);
+  k_stage_build<true><<<G, ST_T, 0, st>>>(n, 0, row_ptr, col_idx, ucnt, nullptr, p.ucol.p, p.lidx.p, roff);
+  k_row_slots<<<G, ST_T, 0, st>>>(sub, row_ptr, roff, slots);
+  PF_HIP(hipGetLastError());
+  std::vector<int32_t> h((size_t)3 * G + 1);
+  PF_HIP(hipMemcpyAsync(h.data(), p.info.p, sizeof(int32_t) * h.size(), hipMemcpyDeviceToHost, st));
+  PF_HIP(hipStreamSynchronize(st));
+  bool staged = true;
+  for (int b = 0; b < G; ++b) {
+    p.maxrows = std::max(p.maxrows, h[b + 1] - h[b]);
+    staged = staged && h[G + 1 + b] >= 0;
+    p.umax = std::max(p.umax, h[G + 1 + b]);
+    p.maxslots = std::max(p.maxslots, h[2 * G + 1 + b]);
+  }
+  p.staged = staged;
   return PF_OK;
 }
 
