@@ -8,8 +8,8 @@
 // of x is a contiguous R-wide load.  Each case keeps its own scalars (alpha, omega, beta,
 // r.r, stop state); a case that has stopped leaves its x, r, p untouched while the others
 // continue.  Per iteration: five streaming kernels (the two products with their fused dot
-// products, e = r - alpha y, the x/r update, the p update) and three one-block kernels that
-// reduce the per-block partial sums of every case in a fixed order and advance its scalars.
+// products, e = r - alpha y, the x/r update, the p update) and three small kernels, one workgroup
+// per case, that reduce the case's per-block partial sums in a fixed order and advance its scalars.
 //
 // The matrix is read in a node-block CSR copy of the system's CRS (9 values of a 3x3
 // block contiguous, one int32 node column per block), built once per matrix.
@@ -31,6 +31,7 @@ struct MScal {
 
 struct MCtl {
   int32_t all_done, itrmax, stop_mode, nrhs;
+  int32_t ndone, pad;
   double er0, rel;
 };
 
@@ -71,7 +72,24 @@ __device__ inline void case_partials(double (&v)[NV], int R, double *part) {
 constexpr int MCHUNK_MAX = 9;
 template <int RP>
 constexpr int mchunk() {
-  return RP == 64 ? 9 : 3;  // block values in scalar registers with one node per wavefront
+  return RP >= 8 ? 9 : 3;
+}
+// 8 to 32 cases: every lane of a node would load each block value itself, 243 load instructions
+// per node beside the 81 of x, and their issue bounds the product (30^3, 32 cases: 106 us).  The
+// node's lanes load the step's 81 values and 9 columns once, contiguously, and pass them through LDS
+// (the next step's are on their way meanwhile).  With 64 cases a wavefront owns one node and
+// the values come through scalar loads.
+template <int RP>
+constexpr bool mstaged() {
+  return RP >= 8 && RP <= 32;
+}
+
+__device__ inline void wave_lds_sync() {
+  // LDS operations of one wavefront are performed in issue order; the fences keep the compiler
+  // from moving LDS accesses across this point
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 // every node row of y = A x for the calling thread's case lane; op(dof, case, sum).  The
@@ -81,6 +99,8 @@ template <int RP, typename XF, typename OP>
 __device__ inline void node_rows(const Blk &B, int R, XF xf, OP op) {
   constexpr int MC = mchunk<RP>();
   static_assert(MC <= MCHUNK_MAX, "row step longer than the zero blocks after the last row");
+  __shared__ double sval[mstaged<RP>() ? MBT / RP : 1][mstaged<RP>() ? 9 * MC + 1 : 1];
+  __shared__ int32_t scol[mstaged<RP>() ? MBT / RP : 1][mstaged<RP>() ? MC + 1 : 1];
   const int l = threadIdx.x % RP;
   const bool live = l < R;
   const int lc = live ? l : 0;
@@ -105,6 +125,50 @@ __device__ inline void node_rows(const Blk &B, int R, XF xf, OP op) {
     const int64_t i = RP == 64 ? (int64_t)__builtin_amdgcn_readfirstlane((int)i0) : i0;
     const int64_t b0 = B.noff[i], b1 = B.noff[i + 1];
     double a0 = 0.0, a1 = 0.0, a2 = 0.0;
+    if constexpr (mstaged<RP>()) {
+      constexpr int NQ = (9 * MC + RP - 1) / RP, NJ = (MC + RP - 1) / RP;
+      double *sv = sval[threadIdx.x / RP];
+      int32_t *sj = scol[threadIdx.x / RP];
+      double q[NQ];
+      int32_t c[NJ];
+      const auto fetch = [&](int64_t blk) {  // lanes past the step's end repeat its last entry
+#pragma unroll
+        for (int t = 0; t < NQ; ++t) q[t] = B.bval[blk * 9 + (l + t * RP < 9 * MC ? l + t * RP : 9 * MC - 1)];
+#pragma unroll
+        for (int t = 0; t < NJ; ++t) c[t] = B.bcol[blk + (l + t * RP < MC ? l + t * RP : MC - 1)];
+      };
+      if (b0 < b1) fetch(b0);
+      for (int64_t blk = b0; blk < b1; blk += MC) {
+#pragma unroll
+        for (int t = 0; t < NQ; ++t)
+          if (l + t * RP < 9 * MC) sv[l + t * RP] = q[t];
+#pragma unroll
+        for (int t = 0; t < NJ; ++t)
+          if (l + t * RP < MC) sj[l + t * RP] = c[t];
+        wave_lds_sync();
+        double x[MC][3];
+#pragma unroll
+        for (int u = 0; u < MC; ++u) {
+          const int64_t j = 3 * (int64_t)sj[u];
+          x[u][0] = xf(j, lc);
+          x[u][1] = xf(j + 1, lc);
+          x[u][2] = xf(j + 2, lc);
+        }
+        if (blk + MC < b1) fetch(blk + MC);
+#pragma unroll
+        for (int u = 0; u < MC; ++u) {
+          const double *w = sv + 9 * u;
+          const double t0 = w[0] * x[u][0] + w[1] * x[u][1] + w[2] * x[u][2];
+          const double t1 = w[3] * x[u][0] + w[4] * x[u][1] + w[5] * x[u][2];
+          const double t2 = w[6] * x[u][0] + w[7] * x[u][1] + w[8] * x[u][2];
+          const bool own = blk + u < b1;
+          a0 = own ? a0 + t0 : a0;
+          a1 = own ? a1 + t1 : a1;
+          a2 = own ? a2 + t2 : a2;
+        }
+        wave_lds_sync();  // the next step rewrites the values
+      }
+    } else
     for (int64_t blk = b0; blk < b1; blk += MC) {
       int64_t j[MC];
 #pragma unroll
@@ -148,17 +212,27 @@ __device__ inline void node_entries(int64_t nn, int R, OP op) {
     for (int d = 0; d < 3; ++d) op(3 * i + d, l);
 }
 
-// one-block reductions: 16 lanes per case (cases 0..63 in a 1024-thread block) sum the G
-// partials of their case in a fixed order and leave the total in the case's lane 0
-constexpr int RBT = 1024, RLANES = 16;
-
+// reductions: one workgroup per case sums the G partials of its case in a fixed order; the total
+// reaches every thread.  (One workgroup for all cases, 16 lanes each, took 20 us per sum with 32
+// cases and 1024 partials.)
 __device__ inline double case_total(const double *__restrict__ part, int64_t row, int G) {
-  const int j = threadIdx.x % RLANES;
+  __shared__ double sh[MBT / 64];
   double t = 0.0;
-  for (int b = j; b < G; b += RLANES) t += part[row * G + b];
+  for (int b = threadIdx.x; b < G; b += MBT) t += part[row * G + b];
 #pragma unroll
-  for (int off = RLANES / 2; off > 0; off >>= 1) t += __shfl_xor(t, off, RLANES);
+  for (int off = 32; off > 0; off >>= 1) t += __shfl_xor(t, off, 64);
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = t;
+  __syncthreads();
+  t = ((sh[0] + sh[1]) + sh[2]) + sh[3];
+  __syncthreads();
   return t;
+}
+
+// one more case has stopped; the last one ends the iteration
+__device__ inline void case_done(MScal *s, MCtl *ctl, int status) {
+  s->status = status;
+  s->done = 1;
+  if (atomicAdd(&ctl->ndone, 1) + 1 == ctl->nrhs) ctl->all_done = 1;
 }
 
 struct Vec {
@@ -221,30 +295,20 @@ __global__ void __launch_bounds__(MBT) k_m_fix_x0(int64_t nn, int R, const doubl
   });
 }
 
-__global__ void __launch_bounds__(RBT) k_m_init_finish(const double *__restrict__ part, int G, MScal *__restrict__ sc,
+__global__ void __launch_bounds__(MBT) k_m_init_finish(const double *__restrict__ part, int G, MScal *__restrict__ sc,
                                                        MCtl *__restrict__ ctl) {
-  const int l = threadIdx.x / RLANES;
-  const int R = ctl->nrhs;
-  if (l < R) {
-    const double t = case_total(part, l, G);      // r.r
-    const double bb = case_total(part, R + l, G);  // b.b
-    if (threadIdx.x % RLANES == 0) {
-      MScal s{};
-      s.c1 = t;
-      s.rr = t;
-      s.bnorm2 = bb;
-      s.status = PF_NOT_CONVERGED;
-      s.done = (ctl->itrmax <= 0 || !(t > 0.0)) ? 1 : 0;  // r = 0: x (0, or the guess) solves it
-      if (!(t > 0.0)) s.status = PF_OK;
-      sc[l] = s;
-    }
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int all = 1;
-    for (int k = 0; k < R; ++k) all &= sc[k].done;
-    ctl->all_done = all;
-  }
+  const int l = blockIdx.x;
+  const double t = case_total(part, l, G);                // r.r
+  const double bb = case_total(part, ctl->nrhs + l, G);  // b.b
+  if (threadIdx.x != 0) return;
+  MScal s{};
+  s.c1 = t;
+  s.rr = t;
+  s.bnorm2 = bb;
+  s.status = PF_NOT_CONVERGED;
+  sc[l] = s;
+  if (!(t > 0.0)) case_done(&sc[l], ctl, PF_OK);  // r = 0: x (0, or the guess) solves it
+  else if (ctl->itrmax <= 0) case_done(&sc[l], ctl, PF_NOT_CONVERGED);
 }
 
 // ---- K1: y = A p ; partials r0.y -----------------------------------------------------
@@ -261,12 +325,12 @@ __global__ void __launch_bounds__(MBT) k_m_spmv_p(Blk B, int R, const double *__
   case_partials<RP, 1>(acc, R, part);
 }
 
-__global__ void __launch_bounds__(RBT) k_m_alpha(const double *__restrict__ part, int G, MScal *__restrict__ sc,
+__global__ void __launch_bounds__(MBT) k_m_alpha(const double *__restrict__ part, int G, MScal *__restrict__ sc,
                                                  const MCtl *__restrict__ ctl) {
-  const int l = threadIdx.x / RLANES;
-  if (ctl->all_done || l >= ctl->nrhs || sc[l].done) return;
+  const int l = blockIdx.x;
+  if (ctl->all_done || sc[l].done) return;
   const double t = case_total(part, l, G);
-  if (threadIdx.x % RLANES == 0) {
+  if (threadIdx.x == 0) {
     sc[l].c2 = t;
     sc[l].alpha = sc[l].c1 / t;
   }
@@ -302,18 +366,16 @@ __global__ void __launch_bounds__(MBT) k_m_spmv_e(Blk B, int R, const double *__
   case_partials<RP, 2>(acc, R, part);
 }
 
-__global__ void __launch_bounds__(RBT) k_m_omega(const double *__restrict__ part, int G, MScal *__restrict__ sc,
-                                                 const MCtl *__restrict__ ctl) {
-  const int l = threadIdx.x / RLANES;
-  if (ctl->all_done || l >= ctl->nrhs || sc[l].done) return;
-  const int R = ctl->nrhs;
+__global__ void __launch_bounds__(MBT) k_m_omega(const double *__restrict__ part, int G, MScal *__restrict__ sc,
+                                                 MCtl *__restrict__ ctl) {
+  const int l = blockIdx.x;
+  if (ctl->all_done || sc[l].done) return;
   const double ev = case_total(part, l, G);
-  const double vv = case_total(part, R + l, G);
-  if (threadIdx.x % RLANES != 0) return;
+  const double vv = case_total(part, ctl->nrhs + l, G);
+  if (threadIdx.x != 0) return;
   if (vv == 0.0 || !isfinite(sc[l].alpha)) {  // FEMSolverClass.f90:2266
-    sc[l].status = vv == 0.0 ? PF_BREAKDOWN_VV : PF_BREAKDOWN_C2C3;
     sc[l].itr += vv == 0.0 ? 1 : 0;
-    sc[l].done = 1;
+    case_done(&sc[l], ctl, vv == 0.0 ? PF_BREAKDOWN_VV : PF_BREAKDOWN_C2C3);
     return;
   }
   sc[l].omega = ev / vv;
@@ -344,44 +406,30 @@ __global__ void __launch_bounds__(MBT) k_m_update(int64_t nn, int R, double *__r
   case_partials<RP, 2>(acc, R, part);
 }
 
-__global__ void __launch_bounds__(RBT) k_m_beta(const double *__restrict__ part, int G, MScal *__restrict__ sc,
+__global__ void __launch_bounds__(MBT) k_m_beta(const double *__restrict__ part, int G, MScal *__restrict__ sc,
                                                 MCtl *__restrict__ ctl) {
-  const int l = threadIdx.x / RLANES;
-  const int R = ctl->nrhs;
-  const bool live = !ctl->all_done && l < R && !sc[l].done;
-  if (live) {
-    const double rr = case_total(part, l, G);
-    const double r0r = case_total(part, R + l, G);
-    if (threadIdx.x % RLANES == 0) {
-      MScal s = sc[l];
-      s.itr += 1;
-      s.rr = rr;
-      if (s.itr == 1) s.rr1 = rr;
-      const bool stop = ctl->stop_mode == 0 ? (sqrt(rr / s.rr1) < ctl->rel || sqrt(rr) < ctl->er0)
-                                            : sqrt(rr) < ctl->rel * sqrt(s.bnorm2);
-      const double c2w = s.c2 * s.omega;
-      const double beta = r0r / c2w;
-      if (stop) {
-        s.status = PF_OK;
-        s.done = 1;
-      } else if (c2w == 0.0 || !isfinite(beta) || !isfinite(rr)) {  // FEMSolverClass.f90:2295
-        s.status = PF_BREAKDOWN_C2C3;
-        s.done = 1;
-      } else if (s.itr >= ctl->itrmax) {
-        s.status = PF_NOT_CONVERGED;
-        s.done = 1;
-      } else {
-        s.c1 = r0r;
-        s.beta = beta;
-      }
-      sc[l] = s;
-    }
-  }
-  __syncthreads();
-  if (threadIdx.x == 0 && !ctl->all_done) {
-    int all = 1;
-    for (int k = 0; k < R; ++k) all &= sc[k].done;
-    ctl->all_done = all;
+  const int l = blockIdx.x;
+  if (ctl->all_done || sc[l].done) return;
+  const double rr = case_total(part, l, G);
+  const double r0r = case_total(part, ctl->nrhs + l, G);
+  if (threadIdx.x != 0) return;
+  MScal &s = sc[l];
+  s.itr += 1;
+  s.rr = rr;
+  if (s.itr == 1) s.rr1 = rr;
+  const bool stop = ctl->stop_mode == 0 ? (sqrt(rr / s.rr1) < ctl->rel || sqrt(rr) < ctl->er0)
+                                        : sqrt(rr) < ctl->rel * sqrt(s.bnorm2);
+  const double c2w = s.c2 * s.omega;
+  const double beta = r0r / c2w;
+  if (stop) {
+    case_done(&s, ctl, PF_OK);
+  } else if (c2w == 0.0 || !isfinite(beta) || !isfinite(rr)) {  // FEMSolverClass.f90:2295
+    case_done(&s, ctl, PF_BREAKDOWN_C2C3);
+  } else if (s.itr >= ctl->itrmax) {
+    case_done(&s, ctl, PF_NOT_CONVERGED);
+  } else {
+    s.c1 = r0r;
+    s.beta = beta;
   }
 }
 
@@ -501,13 +549,13 @@ int enqueue_chunk(pf_ctx *ctx, MultiWork *w, const MLaunch &L, const Blk &B, dou
   double *p1 = w->part.p, *p2 = w->part.p + (size_t)R * G, *p3 = w->part.p + (size_t)3 * R * G;
   for (int it = 0; it < count; ++it) {
     PF_DISPATCH_RP(L.rp, (k_m_spmv_p<RP_><<<L.grid, MBT, 0, st>>>(B, R, w->p.p, w->y.p, w->r0.p, w->ctl.p, p1)));
-    k_m_alpha<<<1, RBT, 0, st>>>(p1, G, w->sc.p, w->ctl.p);
+    k_m_alpha<<<R, MBT, 0, st>>>(p1, G, w->sc.p, w->ctl.p);
     PF_DISPATCH_RP(L.rp, (k_m_evec<RP_><<<L.grid, MBT, 0, st>>>(B.nn, R, w->r.p, w->y.p, w->e.p, w->sc.p, w->ctl.p)));
     PF_DISPATCH_RP(L.rp, (k_m_spmv_e<RP_><<<L.grid, MBT, 0, st>>>(B, R, w->e.p, w->v.p, w->ctl.p, p2)));
-    k_m_omega<<<1, RBT, 0, st>>>(p2, G, w->sc.p, w->ctl.p);
+    k_m_omega<<<R, MBT, 0, st>>>(p2, G, w->sc.p, w->ctl.p);
     PF_DISPATCH_RP(L.rp, (k_m_update<RP_><<<L.grid, MBT, 0, st>>>(B.nn, R, x, w->r.p, w->r0.p, w->p.p, w->e.p, w->v.p,
                                                                   w->sc.p, w->ctl.p, p3)));
-    k_m_beta<<<1, RBT, 0, st>>>(p3, G, w->sc.p, w->ctl.p);
+    k_m_beta<<<R, MBT, 0, st>>>(p3, G, w->sc.p, w->ctl.p);
     PF_DISPATCH_RP(L.rp, (k_m_pupdate<RP_><<<L.grid, MBT, 0, st>>>(B.nn, R, w->p.p, w->r.p, w->y.p, w->sc.p, w->ctl.p)));
   }
   PF_HIP(hipGetLastError());
@@ -581,9 +629,7 @@ int pf_multi_solve_device(pf_ctx *ctx, MultiWork **pw, int64_t n, const int64_t 
   MLaunch L;
   L.rp = rp_of(R);
   {
-    // at most 4 blocks per CU (16 waves): every block leaves one partial per case that the
-    // one-block reductions sum (measured at 40^3, 64 cases: 8 blocks/CU -> 106 us of
-    // reductions per iteration)
+    // at most 4 blocks per CU (16 waves): every block leaves one partial per case to be summed
     const int64_t nodes_per_block = MBT / L.rp;
     int64_t g = (nn + nodes_per_block - 1) / nodes_per_block;
     const int64_t cap = (int64_t)ctx->num_cus * 4;
@@ -609,7 +655,7 @@ int pf_multi_solve_device(pf_ctx *ctx, MultiWork **pw, int64_t n, const int64_t 
     PF_DISPATCH_RP(L.rp, (k_m_init<RP_><<<L.grid, MBT, 0, ctx->stream>>>(nn, R, B_dev, fixed, w->bt.p, X_dev,
                                                                         w->r.p, w->r0.p, w->p.p, w->part.p)));
   }
-  k_m_init_finish<<<1, RBT, 0, ctx->stream>>>(w->part.p, (int)L.grid, w->sc.p, w->ctl.p);
+  k_m_init_finish<<<R, MBT, 0, ctx->stream>>>(w->part.p, (int)L.grid, w->sc.p, w->ctl.p);
   PF_HIP(hipGetLastError());
   int chunk = o.check_every > 0 ? o.check_every : 32;
   const bool use_graph = o.use_graph != 0 && pf_graphs_allowed();
