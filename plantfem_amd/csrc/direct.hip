@@ -14,13 +14,19 @@
 //  * band storage (LAPACK dpbtrf 'L' layout): entry (r, c), 0 <= r - c <= b, of the permuted
 //    matrix at band[c*ld + r - c], ld >= b + 1; the order is padded to a multiple of 32 with
 //    unit diagonal rows;
-//  * factorization: one workgroup per mesh from a largest-first queue (persistent kernel),
-//    left-looking by blocks of 32 columns: the block's (b+32) x 32 rows are updated by the
-//    previous b columns with FP64 MFMA 16x16x4 tiles, the two 16 x 16 diagonal tiles are
-//    factored with cross-lane operations and the tiles below are multiplied by their inverse
-//    transposes;
-//  * triangular solves: blocks of 16, the diagonal solve in one wave, the off-diagonal
-//    update with one thread per row (forward) or column (backward).
+//  * factorization: left-looking by blocks of 32 columns: the block's (b+32) x 32 rows are
+//    updated by the previous b columns with FP64 MFMA 16x16x4 tiles, the two 16 x 16 diagonal
+//    tiles are factored with cross-lane operations and the tiles below are multiplied by their
+//    inverse transposes.  A persistent kernel takes (mesh, share) items from a largest-first
+//    queue; a mesh that alone would decide the time is shared by several workgroups, which take
+//    its blocks in turn: a workgroup updates its block with the columns that are complete while
+//    the others finish the preceding blocks, and publishes its own block as the mesh's progress;
+//  * triangular solves (k_band_solve, half bandwidths up to 1024): blocks of 32 rows; the
+//    diagonal blocks' inverses, formed in parallel beforehand, turn the serial solve into a
+//    32 x 32 product, the moving window of the right-hand side stays in LDS, and a second,
+//    row-major copy of L (written by the factorization beside the band) makes the backward
+//    update's loads contiguous too.  Wider bands, and systems whose second copy does not fit the
+//    memory: band_solve (blocks of 16, the diagonal solve in one wave).
 // Fixed-precision iterative refinement on the true residual b - A x (the CRS values, in
 // FP64) follows as requested.
 #include <algorithm>
@@ -39,7 +45,6 @@ namespace {
 typedef double d4 __attribute__((ext_vector_type(4)));
 
 constexpr int DBT = 512;   // threads per workgroup of the factor/solve kernel
-constexpr int MAXT = 2;    // row tiles a wave holds at once (each 16 rows x 32 columns)
 
 struct DMesh {
   int64_t d0;    // first DOF of the mesh in the system
@@ -51,13 +56,23 @@ struct DMesh {
   int32_t ld;    // leading dimension of the band (>= b + 1, even)
 };
 
+// share g of G of a mesh's factorization: blocks g, g + G, g + 2 G, ...
+struct DItem {
+  int32_t m, g, G, pad;
+};
+
 struct DArgs {
   const DMesh *mesh;
   const int32_t *order;  // queue order (largest first)
+  const DItem *item;     // factorization: queue of shares, those of a mesh adjacent
+  int32_t nitem;
+  int32_t *progress;     // per mesh: blocks of 32 columns complete (-1: not positive definite, -2: gave up)
   int32_t *queue;
   int32_t nmesh;
-  int32_t mode;          // 0: factor, then solve x = A^-1 rhs; 1: solve only, x += A^-1 rhs
+  int32_t mode;          // 0: factor, then solve x = A^-1 rhs; 1: solve only, x += A^-1 rhs; 2: factor only
   double *band;
+  double *rows;          // L row by row: entry (r, c) at rows[boff + r ld + (r - c)] (NULL: not kept)
+  const double *dinv;    // inverses of the 32 x 32 diagonal blocks: block J row i at dinv[32 (woff + 32 J + i)]
   const int32_t *perm;   // band index q of mesh m -> local DOF (perm[woff + q], q < n)
   double *w;             // work vector (npad per mesh)
   const double *rhs;
@@ -67,6 +82,14 @@ struct DArgs {
 };
 
 __device__ inline double shfl(double v, int src) { return __shfl(v, src, 64); }
+
+// A value read from LDS that is the same in every lane, as a scalar.
+__device__ inline int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+
+// p[i]: scalar base, 32-bit lane offset (one address register per load instead of two)
+__device__ inline double at(const double *__restrict__ p, uint32_t i) {
+  return *(const double *)((const char *)p + (i * 8u));
+}
 
 // The wave index within the workgroup as a scalar: the compiler cannot tell that
 // threadIdx.x / 64 is the same in every lane of a wave, and without this every tile index,
@@ -82,43 +105,9 @@ __device__ inline int lane_id() {
   return l;
 }
 
-// Cholesky of the 16 x 16 diagonal tile held in the FP64 MFMA accumulator layout (lane l,
-// element v: row 4*v + l/16, column l%16).  Lower part becomes L11; bad is set on a
-// non-positive pivot.
-__device__ inline void chol16(d4 &a, int q, int jl, bool &bad) {
-#pragma unroll
-  for (int k = 0; k < 16; ++k) {
-    const double piv = shfl(a[k >> 2], (k & 3) * 16 + k);
-    bad = bad || !(piv > 0.0);
-    const double s = sqrt(piv);
-    const double rs = 1.0 / s;
-    if (jl == k) {
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int i = 4 * v + q;
-        if (i > k) a[v] *= rs;
-        else if (i == k) a[v] = s;
-      }
-    }
-    // L[i][k] of this lane's rows (same lane group, column k) and L[jl][k]
-    double lik[4];
-#pragma unroll
-    for (int v = 0; v < 4; ++v) lik[v] = shfl(a[v], 16 * q + k);
-    const int src = 16 * (jl & 3) + k;
-    const double e0 = shfl(a[0], src), e1 = shfl(a[1], src), e2 = shfl(a[2], src), e3 = shfl(a[3], src);
-    const int sel = jl >> 2;
-    const double ljk = sel == 0 ? e0 : (sel == 1 ? e1 : (sel == 2 ? e2 : e3));
-    if (jl > k) {
-#pragma unroll
-      for (int v = 0; v < 4; ++v)
-        if (4 * v + q >= jl) a[v] -= lik[v] * ljk;
-    }
-  }
-}
-
 // acc += A B for the 16x4 fragment A (lane l holds A[l%16][l/16]) and the 4x16 fragment B
-// (lane l holds B[l/16][l%16]); accumulator layout as chol16 (the register layout of
-// v_mfma_f64_16x16x4f64).  MF: the matrix core; else the
+// (lane l holds B[l/16][l%16]); accumulator layout (that of
+// v_mfma_f64_16x16x4f64): lane l, element v: row 4 v + l/16, column l%16.  MF: the matrix core; else the
 // same product from cross-lane reads and FMAs.
 template <bool MF>
 __device__ inline void tile_fma(d4 &acc, double af, double bf, int q, int jl) {
@@ -137,7 +126,10 @@ __device__ inline void tile_fma(d4 &acc, double af, double bf, int q, int jl) {
 // Geometry of one block of 32 columns j0 .. j0+31 and of a wave's tiles in one pass: row
 // tiles t (rows R = j0 + 16 t .. R+15, t < T) of the rows j0 .. j0+31+b, column tiles
 // ct = 0 (columns j0 .. j0+15) and ct = 1 (j0+16 .. j0+31); the wave holds tiles
-// tb, tb + W, ..., tb + (MAXT-1) W.
+// tb, tb + W, ..., tb + (MAXT-1) W.  MAXT tiles of 16 rows x 32 columns per wave: 2, 4 or 6, the
+// fewest that hold the whole block in one pass where 6 do.  A second pass would start its update
+// only after the first one's diagonal tiles, which the shares of a mesh cannot overlap, and every
+// B fragment feeds all of a wave's tiles.
 struct BlockGeom {
   int j0, b, npad, T, tb, W;
   int64_t ld;
@@ -147,38 +139,38 @@ struct BlockGeom {
 // fragments L[R + l%16][c + l/16] of the wave's tiles and B fragments L[j0 + 16 ct + l%16]
 // [c + l/16] of both column tiles.  This is the form for the first chunks of a tile (where
 // some lanes' entries lie outside the band) and the last rows: every load has an index
-// clamped into the band, so the loads are unconditional and stay in flight together, and the
-// entries outside the band are replaced by zero where they are used.  Chunks below cend.
-template <int U>
+// clamped into the band and chunks from cend on repeat the last one, so the loads are
+// unconditional and stay in flight together (a load under a condition keeps the register's older
+// value alive across the loop and spills it), and the entries outside the band are replaced by zero
+// where they are used.
+template <int U, int MAXT>
 struct Frags {
   double b[U][2];
   double a[U][MAXT];
 };
 
-template <int U>
-__device__ inline void load_frags(Frags<U> &f, const double *__restrict__ band, const BlockGeom &g, int c0,
+template <int U, int MAXT>
+__device__ inline void load_frags(Frags<U, MAXT> &f, const double *__restrict__ band, const BlockGeom &g, int c0,
                                   int cend, int q, int jl) {
 #pragma unroll
   for (int u = 0; u < U; ++u) {
-    const int c = c0 + 4 * u;
-    if (c >= cend) continue;  // wave-uniform
-    const int64_t ck = c + q;
+    const int c = min(c0 + 4 * u, cend - 4);
+    const double *col = band + (int64_t)c * g.ld;
+    const uint32_t lq = (uint32_t)(q * (int)g.ld);
+    const int ck = c + q;
 #pragma unroll
-    for (int ct = 0; ct < 2; ++ct) {
-      const int db = g.j0 + 16 * ct + jl - (int)ck;  // >= 1
-      f.b[u][ct] = band[ck * g.ld + min(db, g.b)];
-    }
+    for (int ct = 0; ct < 2; ++ct) f.b[u][ct] = at(col, lq + min(g.j0 + 16 * ct + jl - ck, g.b));  // j0 + jl > ck
 #pragma unroll
     for (int i = 0; i < MAXT; ++i) {
-      const int da = g.j0 + 16 * (g.tb + g.W * i) + jl - (int)ck;  // >= 1
-      f.a[u][i] = band[ck * g.ld + min(da, g.b)];
+      const int R = g.j0 + 16 * (g.tb + g.W * i);
+      f.a[u][i] = at(col, lq + min(R + jl - ck, g.b));  // R + jl > ck
     }
   }
 }
 
 // acc[i][ct] += A (-B_ct) over the group's chunks (tile 0 has no column tile 1)
-template <bool MF, int U>
-__device__ inline void mfma_frags(const Frags<U> &f, d4 (*acc)[2], const BlockGeom &g, int c0, int cend, int q,
+template <bool MF, int U, int MAXT>
+__device__ inline void mfma_frags(const Frags<U, MAXT> &f, d4 (*acc)[2], const BlockGeom &g, int c0, int cend, int q,
                                   int jl) {
 #pragma unroll
   for (int u = 0; u < U; ++u) {
@@ -202,36 +194,32 @@ __device__ inline void mfma_frags(const Frags<U> &f, d4 (*acc)[2], const BlockGe
   }
 }
 
-// The steady part of a pass: chunks cs <= c < j0, where every lane's entry of each of the
+// The steady part of a pass: chunks cs <= c < ce, where every lane's entry of each of the
 // wave's nt existing tiles and of both column tiles lies inside the band and the tiles' rows
-// end before the padding.  Branch-free: per tile a pointer that advances by 4 (ld - 1)
+// end before the padding.  Branch-free: scalar bases that advance by 4 (ld - 1)
 // doubles per chunk, two groups of chunks in flight, each A fragment used by both column
 // tiles.
-template <bool MF, int U>
+template <bool MF, int U, int MAXT>
 __device__ inline void steady_update(d4 (*acc)[2], const double *__restrict__ band, const BlockGeom &g, int cs,
-                                     int nt, int q, int jl) {
+                                     int ce, int nt, int q, int jl) {
   const int64_t step = g.ld - 1;
-  const double *pa[MAXT];
-#pragma unroll
-  for (int i = 0; i < MAXT; ++i) pa[i] = band + (int64_t)(cs + q) * step + g.j0 + 16 * (g.tb + g.W * i) + jl;
-  const double *pb = band + (int64_t)(cs + q) * step + g.j0 + jl;
+  const double *pb = band + (int64_t)cs * step + g.j0;
+  const uint32_t lq = (uint32_t)(q * (int)step + jl);
   double a0[U][MAXT], a1[U][MAXT], b0[U][2], b1[U][2];
   auto load = [&](double (&a)[U][MAXT], double (&bb)[U][2], int c) {
-    const int64_t off = (int64_t)(c - cs) * step;
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      if (c + 4 * u >= g.j0) continue;  // wave-uniform
+      const double *col = pb + (int64_t)(min(c + 4 * u, ce - 4) - cs) * step;
 #pragma unroll
-      for (int i = 0; i < MAXT; ++i)
-        if (i < nt) a[u][i] = pa[i][off + (int64_t)(4 * u) * step];
+      for (int i = 0; i < MAXT; ++i) a[u][i] = at(col + 16 * (g.tb + g.W * min(i, nt - 1)), lq);
 #pragma unroll
-      for (int ct = 0; ct < 2; ++ct) bb[u][ct] = pb[off + (int64_t)(4 * u) * step + 16 * ct];
+      for (int ct = 0; ct < 2; ++ct) bb[u][ct] = at(col + 16 * ct, lq);
     }
   };
   auto prod = [&](const double (&a)[U][MAXT], const double (&bb)[U][2], int c) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      if (c + 4 * u >= g.j0) continue;  // wave-uniform
+      if (c + 4 * u >= ce) continue;  // wave-uniform
       const double bn0 = -bb[u][0], bn1 = -bb[u][1];
 #pragma unroll
       for (int i = 0; i < MAXT; ++i)
@@ -241,57 +229,79 @@ __device__ inline void steady_update(d4 (*acc)[2], const double *__restrict__ ba
         }
     }
   };
-  int c = cs;
-  if (c < g.j0) load(a0, b0, c);
-  for (; c < g.j0; c += 8 * U) {
-    const int c1 = c + 4 * U, c2 = c1 + 4 * U;
-    if (c1 < g.j0) load(a1, b1, c1);
+  load(a0, b0, cs);
+  for (int c = cs; c < ce; c += 8 * U) {
+    load(a1, b1, c + 4 * U);
     prod(a0, b0, c);
-    if (c2 < g.j0) load(a0, b0, c2);
-    if (c1 < g.j0) prod(a1, b1, c1);
+    load(a0, b0, c + 8 * U);
+    prod(a1, b1, c + 4 * U);
   }
 }
 
+// LDS written by other lanes of the wave may be read after this.  (The hardware keeps a wave's LDS
+// accesses in order; without the fence the compiler may hand a lane back what it wrote itself.)
+__device__ inline void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// v of one lane, as a scalar
+__device__ inline double bcast(double v, int lane) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                          __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+
+constexpr int LS = 17;  // row stride of 16 x 16 tiles in LDS: rows and columns both without bank conflicts
+
 // Diagonal tile of column tile ct (held by the calling wave in accumulator layout): Cholesky
-// factor L_d to the band (columns col0 .. col0+15) and LDS sL, then L_d^-T (the solution X of
-// X L_d^T = I, column by column across the lanes) to sLi; *sflag on a non-positive pivot.
-template <bool MF>
-__device__ inline void diag_block(d4 &a, double *__restrict__ band, int64_t ld, int b, int col0, double *sL,
-                                  double *sLi, int32_t *sflag) {
+// factor L_d to the band (columns col0 .. col0+15), and L_d^-T to LDS sLi; *sflag on a non-positive
+// pivot.  This is the serial chain of a block, so it is kept short: lane i < 16 holds row i of the
+// tile and lane 16 + j column j of the identity, both in registers; step k scales entry k and
+// subtracts the multiples L[j][k] (scalars, from lane j) of it from the entries j > k.  The same
+// instructions turn the rows into L_d and the identity's columns into those of L_d^-1, without a
+// branch.  (Before: the factor in the accumulator layout and the inverse after it, by cross-lane
+// reads under masks, which were most of a block's 47 us.)
+__device__ inline void diag_block(const d4 &a, double *__restrict__ band, double *__restrict__ lrow, int64_t ld,
+                                  int b, int col0, double *sL, double *sLi, int32_t *sflag) {
   const int ln = lane_id();
   const int q = ln >> 4, jl = ln & 15;
+#pragma unroll
+  for (int v = 0; v < 4; ++v) sL[(4 * v + q) * LS + jl] = a[v];
+  wave_sync();
+  double r[16];
+#pragma unroll
+  for (int j = 0; j < 16; ++j) {
+    const double l = sL[jl * LS + j];
+    r[j] = q == 0 ? l : (j == jl ? 1.0 : 0.0);
+  }
   bool bad = false;
-  chol16(a, q, jl, bad);
+#pragma unroll
+  for (int k = 0; k < 16; ++k) {
+    const double piv = bcast(r[k], k);
+    bad = bad || !(piv > 0.0);
+    const double s = sqrt(piv);
+    const double rs = 1.0 / s;
+    r[k] = ln == k ? s : r[k] * rs;
+#pragma unroll
+    for (int j = k + 1; j < 16; ++j) r[j] = fma(-r[k], bcast(r[k], j), r[j]);
+  }
+  // rows of L_d; column j of L_d^-1 is row j of L_d^-T
+  double *out = (q == 0 ? sL : sLi) + jl * LS;
+  if (q < 2) {
+#pragma unroll
+    for (int j = 0; j < 16; ++j) out[j] = r[j];
+  }
+  wave_sync();
 #pragma unroll
   for (int v = 0; v < 4; ++v) {
     const int i = 4 * v + q;
-    sL[i * 16 + jl] = a[v];
     const int d = i - jl;
-    if (d >= 0 && d <= b) band[(int64_t)(col0 + jl) * ld + d] = a[v];
-  }
-  double Lrow[16];  // L_d[jl][k]
-#pragma unroll
-  for (int k = 0; k < 16; ++k) Lrow[k] = sL[jl * 16 + k];
-  d4 x;
-#pragma unroll
-  for (int v = 0; v < 4; ++v) x[v] = (4 * v + q == jl) ? 1.0 : 0.0;
-#pragma unroll
-  for (int k = 0; k < 16; ++k) {
-    if (jl == k) {
-      const double rk = 1.0 / Lrow[k];
-#pragma unroll
-      for (int v = 0; v < 4; ++v) x[v] *= rk;
-    }
-    double xk[4];
-#pragma unroll
-    for (int v = 0; v < 4; ++v) xk[v] = shfl(x[v], 16 * q + k);
-    if (jl > k) {
-#pragma unroll
-      for (int v = 0; v < 4; ++v) x[v] -= xk[v] * Lrow[k];
+    const double l = sL[i * LS + jl];
+    if (d >= 0 && d <= b) {
+      band[(int64_t)(col0 + jl) * ld + d] = l;
+      if (lrow) lrow[(int64_t)(col0 + i) * ld + d] = l;
     }
   }
-#pragma unroll
-  for (int v = 0; v < 4; ++v) sLi[(4 * v + q) * 16 + jl] = x[v];
   if (bad && ln == 0) *sflag = 1;
 }
 
@@ -303,28 +313,49 @@ __device__ inline void tile_times(d4 &acc, const d4 &c, const double *mb, double
   const int ln = lane_id();
   const int q = ln >> 4, jl = ln & 15;
 #pragma unroll
-  for (int v = 0; v < 4; ++v) myC[(4 * v + q) * 16 + jl] = c[v];
+  for (int v = 0; v < 4; ++v) myC[(4 * v + q) * LS + jl] = c[v];
+  wave_sync();
   double af[4];
 #pragma unroll
-  for (int cq = 0; cq < 4; ++cq) af[cq] = myC[jl * 16 + 4 * cq + q];
+  for (int cq = 0; cq < 4; ++cq) af[cq] = myC[jl * LS + 4 * cq + q];
+  wave_sync();  // myC is free again
 #pragma unroll
   for (int cq = 0; cq < 4; ++cq) tile_fma<MF>(acc, af[cq], mb[cq], q, jl);
 }
 
 // store a tile (accumulator layout) of column tile starting at col0 into the band
-__device__ inline void store_tile(const d4 &x, double *__restrict__ band, int64_t ld, int b, int npad, int R,
-                                  int col0) {
+__device__ inline void store_tile(const d4 &x, double *__restrict__ band, double *__restrict__ lrow, int64_t ld,
+                                  int b, int npad, int R, int col0) {
   const int ln = lane_id();
   const int q = ln >> 4, jl = ln & 15;
 #pragma unroll
   for (int v = 0; v < 4; ++v) {
     const int r = R + 4 * v + q;
     const int d = r - (col0 + jl);
-    if (r < npad && d >= 0 && d <= b) band[(int64_t)(col0 + jl) * ld + d] = x[v];
+    if (r < npad && d >= 0 && d <= b) {
+      band[(int64_t)(col0 + jl) * ld + d] = x[v];
+      if (lrow) lrow[(int64_t)r * ld + d] = x[v];
+    }
   }
 }
 
-// Left-looking blocked band Cholesky of one mesh by the whole workgroup, blocks of 32 columns.
+// s_sleep(1) polls of a share for the preceding block before it gives up: seconds, against the
+// microseconds that a block takes.  (The launch is cooperative and the shares are the first items of
+// the queue, one per workgroup: all of them run.)
+constexpr int SHARE_POLLS = 1 << 22;
+
+__device__ inline int publish_failure(int32_t *progress) {
+  if (threadIdx.x == 0) __hip_atomic_store(progress, -1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return PF_NOT_SPD;
+}
+
+// what another share's failure means for this one
+__device__ inline int progress_failed(const int32_t *progress) {
+  return __hip_atomic_load(progress, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == -1 ? PF_NOT_SPD : PF_ERR_HIP;
+}
+
+// Left-looking blocked band Cholesky of one mesh by blocks of 32 columns, a share of its blocks by
+// the whole workgroup.
 // Per block: every wave updates its tiles of rows j0 .. j0+31+b in both column tiles with the
 // previous b columns (MFMA; each A fragment feeds both column tiles; loads of the next group
 // of chunks overlap the products of the current one).  Then wave 0 factors the first
@@ -332,20 +363,45 @@ __device__ inline void store_tile(const d4 &x, double *__restrict__ band, int64_
 // the owner of tile 1 publishes L10; every wave subtracts L(t,0) L10^T from its column-1
 // tiles; wave 1 factors the second diagonal tile (L11, L11^-T); every wave forms
 // L(t,1) = C L11^-T.  Four barriers per block.
-template <int BT, bool MF>
-__device__ int factor_mesh(const DMesh &M, double *__restrict__ band, double *sL, double *sLi, double *sC,
-                           int32_t *sflag) {
+// Bound, one mesh in shares: the chain of a block, 20 us (24,640 equations, b = 350: 15.6 ms for
+// 770 blocks; 84 ms with its two solves before, 26 now); many meshes: the largest one's chain and the
+// stream of the previous b columns that every block rereads.
+template <int BT, bool MF, int MAXT>
+__device__ __forceinline__ int factor_mesh(const DMesh &M, double *band, double *__restrict__ lrow, int share, int shares,
+                           int32_t *progress, double *sL, double *sLi, double *sC, int32_t *sflag) {
   constexpr int W = BT / 64;
-  constexpr int U = 2;   // chunks per group of the steady part
-  constexpr int UR = 2;  // chunks per group of the ramp
+  constexpr int U = MAXT <= 4 ? 4 : 2;  // chunks per group of the steady part, two groups in flight
+  constexpr int UR = U;                 // chunks per group of the ramp
   const int wv = wave_id();
   const int b = M.b, npad = M.npad;
   const int64_t ld = M.ld;
-  double *myC = sC + 256 * wv;
-  double *sLi0 = sLi, *sL10 = sLi + 256, *sLi1 = sLi + 512;
+  double *myC = sC + 16 * LS * wv;
+  double *sLi0 = sLi, *sL10 = sLi + 16 * LS, *sLi1 = sLi + 32 * LS;
   if (threadIdx.x == 0) *sflag = 0;
   __syncthreads();
-  for (int j0 = 0; j0 < npad; j0 += 32) {
+  int have = shares == 1 ? npad : 0;  // columns complete and visible to this workgroup
+  // blocks until at least `want` columns are, false when the mesh has failed
+  const auto columns = [&](int want) {
+    if (have >= want) return true;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      int p, polls = 0;
+      while ((p = __hip_atomic_load(progress, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) >= 0 && 32 * p < want &&
+             ++polls < SHARE_POLLS)
+        __builtin_amdgcn_s_sleep(1);
+      if (p >= 0 && 32 * p < want) {  // the other shares never came: nobody may wait for this one
+        p = -2;
+        __hip_atomic_store(progress, -2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+      sflag[1] = p;
+    }
+    __syncthreads();
+    const int p = uniform(sflag[1]);
+    have = 32 * p;
+    return p >= 0;
+  };
+  for (int j0 = 32 * share; j0 < npad; j0 += 32 * shares) {
     const int lane = lane_id();
     const int q = lane >> 4, jl = lane & 15;
     const int rows = min(32 + b, npad - j0);  // rows j0 .. j0+rows-1 hold the block's nonzeros
@@ -374,26 +430,42 @@ __device__ int factor_mesh(const DMesh &M, double *__restrict__ band, double *sL
           }
         }
       }
-      if (g.tb < T) {
-        // A[block rows, j0..j0+31] -= L[block rows, c] L[j0..j0+31, c]^T, c < j0: a ramp with
-        // predicates up to cs, then the branch-free steady part
-        const int clo = max(0, j0 + 16 * g.tb - b) & ~3;
-        const int nt = min(MAXT, (T - 1 - g.tb) / W + 1);  // existing tiles of this wave
-        const int Rl = j0 + 16 * (g.tb + W * (nt - 1));
-        const int cs = Rl + 16 <= npad ? min(j0, max(clo, (max(Rl + 15, j0 + 31) - b + 3) & ~3)) : j0;
-        for (int c = clo; c < cs; c += 4 * UR) {
-          Frags<UR> f;
-          load_frags<UR>(f, band, g, c, cs, q, jl);
-          mfma_frags<MF, UR>(f, acc, g, c, cs, q, jl);
+      // the block's columns lo .. hi-1 so far: those complete at hand, then the others as they come
+      const int c_first = max(0, j0 - b) & ~31;
+      int lo = c_first;
+      do {
+        // wait for the next block only, and take what is there by then
+        if (!columns(min(j0, max(lo + 32, have)))) return progress_failed(progress);
+        const int hi = min(j0, have);
+        if (g.tb < T) {
+          // A[block rows, j0..j0+31] -= L[block rows, c] L[j0..j0+31, c]^T, c < j0: a ramp with
+          // predicates up to cs, then the branch-free steady part
+          const int clo = max(0, j0 + 16 * g.tb - b) & ~3;
+          const int nt = min(MAXT, (T - 1 - g.tb) / W + 1);  // existing tiles of this wave
+          const int Rl = j0 + 16 * (g.tb + W * (nt - 1));
+          const int cs = Rl + 16 <= npad ? min(j0, max(clo, (max(Rl + 15, j0 + 31) - b + 3) & ~3)) : j0;
+          const int re = min(cs, hi);
+          const int rb = max(clo, lo);
+          if (rb < re) {
+            Frags<UR, MAXT> f0, f1;
+            load_frags(f0, band, g, rb, re, q, jl);
+            for (int c = rb; c < re; c += 8 * UR) {
+              load_frags(f1, band, g, c + 4 * UR, re, q, jl);
+              mfma_frags<MF>(f0, acc, g, c, re, q, jl);
+              load_frags(f0, band, g, c + 8 * UR, re, q, jl);
+              mfma_frags<MF>(f1, acc, g, c + 4 * UR, re, q, jl);
+            }
+          }
+          if (hi > cs) steady_update<MF, U, MAXT>(acc, band, g, max(cs, lo), hi, nt, q, jl);
         }
-        steady_update<MF, U>(acc, band, g, cs, nt, q, jl);
-      }
+        lo = hi;
+      } while (lo < j0);
       if (p == 0) {
-        if (wv == 0) diag_block<MF>(acc[0][0], band, ld, b, j0, sL, sLi0, sflag);
+        if (wv == 0) diag_block(acc[0][0], band, lrow, ld, b, j0, sL, sLi0, sflag);
         __syncthreads();
-        if (*sflag) return PF_NOT_SPD;
+        if (uniform(*sflag)) return publish_failure(progress);
 #pragma unroll
-        for (int cq = 0; cq < 4; ++cq) mb0[cq] = sLi0[(4 * cq + q) * 16 + jl];
+        for (int cq = 0; cq < 4; ++cq) mb0[cq] = sLi0[(4 * cq + q) * LS + jl];
       }
       // column tile 0 below the diagonal: L(t,0) = C L00^-T; tile 1 publishes L10
 #pragma unroll
@@ -403,10 +475,10 @@ __device__ int factor_mesh(const DMesh &M, double *__restrict__ band, double *sL
           d4 x = {0.0, 0.0, 0.0, 0.0};
           tile_times<MF>(x, acc[i][0], mb0, myC);
           acc[i][0] = x;
-          store_tile(x, band, ld, b, npad, j0 + 16 * t, j0);
+          store_tile(x, band, lrow, ld, b, npad, j0 + 16 * t, j0);
           if (t == 1) {
 #pragma unroll
-            for (int v = 0; v < 4; ++v) sL10[(4 * v + q) * 16 + jl] = x[v];
+            for (int v = 0; v < 4; ++v) sL10[(4 * v + q) * LS + jl] = x[v];
           }
         }
       }
@@ -414,7 +486,7 @@ __device__ int factor_mesh(const DMesh &M, double *__restrict__ band, double *sL
         __syncthreads();
         // B fragment of -L10^T: B[kk][n] = -L10[n][4 cq + kk]
 #pragma unroll
-        for (int cq = 0; cq < 4; ++cq) mb10[cq] = -sL10[jl * 16 + 4 * cq + q];
+        for (int cq = 0; cq < 4; ++cq) mb10[cq] = -sL10[jl * LS + 4 * cq + q];
       }
       // column tile 1: C(t,1) -= L(t,0) L10^T
 #pragma unroll
@@ -423,11 +495,11 @@ __device__ int factor_mesh(const DMesh &M, double *__restrict__ band, double *sL
         if (t >= 1 && t < T) tile_times<MF>(acc[i][1], acc[i][0], mb10, myC);
       }
       if (p == 0) {
-        if (wv == 1) diag_block<MF>(acc[0][1], band, ld, b, j0 + 16, sL, sLi1, sflag);
+        if (wv == 1) diag_block(acc[0][1], band, lrow, ld, b, j0 + 16, sL, sLi1, sflag);
         __syncthreads();
-        if (*sflag) return PF_NOT_SPD;
+        if (uniform(*sflag)) return publish_failure(progress);
 #pragma unroll
-        for (int cq = 0; cq < 4; ++cq) mb1[cq] = sLi1[(4 * cq + q) * 16 + jl];
+        for (int cq = 0; cq < 4; ++cq) mb1[cq] = sLi1[(4 * cq + q) * LS + jl];
       }
       // column tile 1 below its diagonal: L(t,1) = C L11^-T
 #pragma unroll
@@ -436,11 +508,14 @@ __device__ int factor_mesh(const DMesh &M, double *__restrict__ band, double *sL
         if (t >= 2 && t < T) {
           d4 x = {0.0, 0.0, 0.0, 0.0};
           tile_times<MF>(x, acc[i][1], mb1, myC);
-          store_tile(x, band, ld, b, npad, j0 + 16 * t, j0 + 16);
+          store_tile(x, band, lrow, ld, b, npad, j0 + 16 * t, j0 + 16);
         }
       }
     }
+    if (shares > 1) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // every wave's part of the block is out
     __syncthreads();
+    if (shares > 1 && threadIdx.x == 0)
+      __hip_atomic_store(progress, j0 / 32 + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
   }
   return PF_OK;
 }
@@ -532,28 +607,50 @@ __global__ void k_direct_queue_reset(int32_t *q) {
   if (threadIdx.x == 0 && blockIdx.x == 0) q[0] = 0;
 }
 
+__global__ void k_direct_progress_reset(int32_t n, int32_t *__restrict__ progress, int32_t *__restrict__ status) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) {
+    progress[i] = 0;
+    status[i] = PF_OK;
+  }
+}
+
 __global__ void k_flag_clear(int32_t *f) {
   if (threadIdx.x == 0 && blockIdx.x == 0) f[0] = 0;
 }
 
-template <int BT, bool MF>
+// mode 0: factor (the whole mesh per workgroup), then solve; 1: solve; 2: factor, in shares
+template <int BT, bool MF, int MAXT>
 __global__ void __launch_bounds__(BT) k_direct(DArgs a) {
-  __shared__ double sL[256];
-  __shared__ double sLi[768];
-  __shared__ double sC[256 * (BT / 64)];
+  __shared__ double sL[16 * LS];
+  __shared__ double sLi[48 * LS];
+  __shared__ double sC[16 * LS * (BT / 64)];
   __shared__ double sY[16];
-  __shared__ int32_t next, sflag;
+  __shared__ int32_t next, sflag[2];
+  const int total = a.mode == 2 ? a.nitem : a.nmesh;
   for (;;) {
     __syncthreads();
     if (threadIdx.x == 0) next = atomicAdd(a.queue, 1);
     __syncthreads();
-    const int32_t qi = next;
-    if (qi >= a.nmesh) break;
-    const int32_t m = a.order[qi];
+    const int32_t qi = uniform(next);
+    if (qi >= total) break;
+    const DItem it = a.mode == 2 ? a.item[qi] : DItem{a.order[qi], 0, 1, 0};
+    const int32_t m = it.m;
     const DMesh M = a.mesh[m];
     const int64_t t0 = wall_clock64();
     double *band = a.band + M.boff;
-    int st = a.mode == 0 ? factor_mesh<BT, MF>(M, band, sL, sLi, sC, &sflag) : a.status[m];
+    int st = a.mode != 1 ? factor_mesh<BT, MF, MAXT>(M, band, a.rows ? a.rows + M.boff : nullptr, it.g, it.G,
+                                               a.progress + m, sL, sLi, sC, sflag)
+                         : a.status[m];
+    if (a.mode == 2) {
+      // the share of the last block reports for the mesh, the first one for its start
+      if (threadIdx.x == 0) {
+        if (st != PF_OK) a.status[m] = st;
+        if (it.g == 0) a.t_raw[2 * m] = t0;
+        if (it.g == (M.npad / 32 - 1) % it.G) a.t_raw[2 * m + 1] = wall_clock64();
+      }
+      continue;
+    }
     double *w = a.w + M.woff;
     const int32_t *perm = a.perm + M.woff;
     if (st == PF_OK) {
@@ -572,6 +669,180 @@ __global__ void __launch_bounds__(BT) k_direct(DArgs a) {
       a.t_raw[2 * m] = t0;
       a.t_raw[2 * m + 1] = wall_clock64();
     }
+  }
+}
+
+// ---- triangular solves with the diagonal blocks' inverses -------------------------------
+constexpr int SB = 32;      // rows per block
+constexpr int SWS = 2048;   // window of the right-hand side in LDS (power of two >= SMAXB + 2 SB)
+constexpr int SMAXB = 1024; // widest band
+
+// inverse of the lower triangular diagonal blocks, one thread per column, four blocks per workgroup
+__global__ void __launch_bounds__(4 * SB) k_diag_inverse(int32_t nmesh, const DMesh *__restrict__ mesh,
+                                                         const int32_t *__restrict__ status,
+                                                         const double *__restrict__ band, double *__restrict__ dinv) {
+  __shared__ double sL[4][SB][SB + 1];
+  const int32_t m = blockIdx.y;
+  const DMesh M = mesh[m];
+  if (status[m] != PF_OK) return;  // whole grid row
+  const int blk = 4 * blockIdx.x + threadIdx.x / SB, j = threadIdx.x % SB;
+  const bool live = SB * blk < M.npad;
+  double(*L)[SB + 1] = sL[threadIdx.x / SB];
+  if (live) {
+    const double *col = band + M.boff + (int64_t)(SB * blk + j) * M.ld;
+    for (int i = 0; i < SB; ++i) L[i][j] = i >= j && i - j <= M.b ? col[i - j] : 0.0;
+  }
+  __syncthreads();
+  if (!live) return;
+  double z[SB];
+#pragma unroll
+  for (int i = 0; i < SB; ++i) {
+    double t = i == j ? 1.0 : 0.0;
+#pragma unroll
+    for (int k = 0; k < i; ++k) t = __builtin_fma(-L[i][k], z[k], t);
+    z[i] = t / L[i][i];
+  }
+  double *out = dinv + (int64_t)SB * (M.woff + SB * blk);
+#pragma unroll
+  for (int i = 0; i < SB; ++i) out[SB * i + j] = z[i];
+}
+
+template <int CTRL>
+__device__ inline double dpp_move(double x) {
+  return __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(x), CTRL, 0xf, 0xf, true),
+                          __builtin_amdgcn_update_dpp(0, __double2loint(x), CTRL, 0xf, 0xf, true));
+}
+
+// One direction of L L^T z = w (FWD: L y = w, else L^T z = y), w in place.  Per block of 32 the
+// workgroup multiplies the block of w by the inverse of the diagonal block, eight lanes per row, and
+// then subtracts the block's columns (rows) from the b <= NR BT entries of w that follow (precede), NR
+// per thread; their loads are issued DEPTH blocks ahead.
+// Bound: what one CU streams (37 GB/s: b = 350, 90 KB per block, 2.4 us per block).  DEPTH: as many blocks as the registers hold (b <= 512: 3.73 ms per
+// solve of 24,640 equations with 2, 4.08 with 1; the solves by blocks of 16: 11 ms).  b <= 1024: 1024
+// threads with one entry each (22.1 ms for 192 meshes up to b = 690) rather than 512 with two
+// (24.8 ms).
+template <int BT, int NR, int DEPTH, bool FWD>
+__device__ __forceinline__ void band_sweep(const DMesh &M, const double *__restrict__ L, const double *__restrict__ dinv,
+                           double *__restrict__ w, double *sw, double *sY) {
+  const int tid = threadIdx.x;
+  const int b = M.b, npad = M.npad, nb = npad / SB;
+  const int64_t ld = M.ld;
+  // entry t = tid of the panel beside block j0: row j0 + SB + t (FWD) or column j0 - 1 - t; its L
+  // values for the block's columns (rows) j lie at distance SB + t - j or j + 1 + t, contiguous over
+  // t.  Those outside the band (distance > b) read a neighbouring entry, at most SB past the
+  // mesh's last (the buffers end with as many), and are dropped.
+  double l[DEPTH][NR][SB];
+  const auto panel = [&](int j0, double (&to)[NR][SB]) {
+#pragma unroll
+    for (int k = 0; k < NR; ++k) {
+      uint32_t tc = (uint32_t)max(min(tid + k * BT, b - 1), 0);
+      asm volatile("" : "+v"(tc));  // keeps the lane's part of the address apart from the scalar part
+      const double *p = L + (int64_t)j0 * ld + (FWD ? SB : 1);
+#pragma unroll
+      for (int j = 0; j < SB; ++j, p += FWD ? ld - 1 : ld + 1) to[k][j] = at(p, tc);
+    }
+  };
+  double di[4];
+  const int mi = tid >> 3, ms = (tid & 7) * 4;  // row of the product, first of this lane's four terms
+  const auto inverse = [&](int J) {
+    if (mi < SB)
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        di[k] = FWD ? dinv[(int64_t)SB * (SB * J + mi) + ms + k] : dinv[(int64_t)SB * (SB * J + ms + k) + mi];
+  };
+  const auto entry = [&](int J, int t) { return FWD ? SB * J + t : npad - 1 - (nb - 1 - J) * SB - t; };
+  // the window: the first block and the b entries beside it; SB more enter with every block
+  const int J0 = FWD ? 0 : nb - 1;
+  for (int t = tid; t < SB + b; t += BT) {
+    const int i = entry(J0, t);
+    if (i >= 0 && i < npad) sw[i & (SWS - 1)] = w[i];
+  }
+#pragma unroll
+  for (int k = 0; k < DEPTH; ++k) panel(SB * (FWD ? min(k, nb - 1) : max(nb - 1 - k, 0)), l[k]);
+  inverse(J0);
+  const auto block = [&](int step, double (&lb)[NR][SB]) {
+    const int J = FWD ? step : nb - 1 - step;
+    const int j0 = SB * J;
+    const int in = entry(J, SB + b + tid);  // enters the window with the next block
+    double win = 0.0;
+    const bool enter = tid < SB && in >= 0 && in < npad;
+    if (enter) win = w[in];
+    __syncthreads();  // the block's entries of w are final
+    if (mi < SB) {
+      double p = 0.0;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) p = __builtin_fma(di[k], sw[(j0 + ms + k) & (SWS - 1)], p);
+      p += dpp_move<0xb1>(p);   // quad_perm 1,0,3,2
+      p += dpp_move<0x4e>(p);   // quad_perm 2,3,0,1
+      p += dpp_move<0x141>(p);  // row_half_mirror: the other four of the eight
+      if ((tid & 7) == 0) {
+        sY[mi] = p;
+        w[j0 + mi] = p;
+      }
+    }
+    if (step + 1 < nb) inverse(FWD ? J + 1 : J - 1);
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < NR; ++k) {
+      int t = tid + k * BT;
+      asm volatile("" : "+v"(t));  // else the masks below are kept over the blocks, and spilled
+      double s0 = 0.0, s1 = 0.0;
+      if (64 * wave_id() + k * BT + 64 + SB <= b) {  // the whole wave inside the band
+#pragma unroll
+        for (int j = 0; j < SB; j += 2) {
+          s0 = __builtin_fma(lb[k][j], sY[j], s0);
+          s1 = __builtin_fma(lb[k][j + 1], sY[j + 1], s1);
+        }
+      } else {
+#pragma unroll
+        for (int j = 0; j < SB; j += 2) {
+          s0 = __builtin_fma((FWD ? SB + t - j : j + 1 + t) <= b ? lb[k][j] : 0.0, sY[j], s0);
+          s1 = __builtin_fma((FWD ? SB + t - j - 1 : j + 2 + t) <= b ? lb[k][j + 1] : 0.0, sY[j + 1], s1);
+        }
+      }
+      const int i = entry(J, SB + t);
+      if (t < b && i >= 0 && i < npad) sw[i & (SWS - 1)] -= s0 + s1;
+    }
+    if (enter) sw[in & (SWS - 1)] = win;
+    panel(SB * (FWD ? min(J + DEPTH, nb - 1) : max(J - DEPTH, 0)), lb);  // past the end: the last once more
+  };
+  for (int step = 0; step < nb; step += DEPTH) {
+#pragma unroll
+    for (int k = 0; k < DEPTH; ++k)
+      if (step + k < nb) block(step + k, l[k]);
+  }
+  __syncthreads();
+}
+
+template <int BT, int NR, int DEPTH>
+__global__ void __launch_bounds__(BT) k_band_solve(DArgs a) {
+  __shared__ double sw[SWS];
+  __shared__ double sY[SB];
+  __shared__ int32_t next;
+  for (;;) {
+    __syncthreads();
+    if (threadIdx.x == 0) next = atomicAdd(a.queue, 1);
+    __syncthreads();
+    const int32_t qi = uniform(next);
+    if (qi >= a.nmesh) break;
+    const int32_t m = a.order[qi];
+    const DMesh M = a.mesh[m];
+    double *w = a.w + M.woff;
+    const int32_t *perm = a.perm + M.woff;
+    if (a.status[m] == PF_OK) {
+      for (int q = threadIdx.x; q < M.npad; q += BT) w[q] = q < M.n ? a.rhs[M.d0 + perm[q]] : 0.0;
+      __syncthreads();
+      const double *dinv = a.dinv + (int64_t)SB * M.woff;
+      band_sweep<BT, NR, DEPTH, true>(M, a.band + M.boff, dinv, w, sw, sY);
+      band_sweep<BT, NR, DEPTH, false>(M, a.rows + M.boff, dinv, w, sw, sY);
+      for (int q = threadIdx.x; q < M.n; q += BT) {
+        const int64_t r = M.d0 + perm[q];
+        a.x[r] = a.mode == 0 ? w[q] : a.x[r] + w[q];
+      }
+    } else if (a.mode == 0) {
+      for (int q = threadIdx.x; q < M.n; q += BT) a.x[M.d0 + q] = 0.0;
+    }
+    if (threadIdx.x == 0 && a.mode == 0) a.t_raw[2 * m + 1] = wall_clock64();
   }
 }
 
@@ -830,6 +1101,13 @@ struct DirectWork {
   DevBuf<int32_t> perm, bidx, dmesh, order, queue, status, flag;
   DevBuf<int64_t> t_raw;
   DevBuf<double> band, w, r, y, norms;
+  DevBuf<double> rows, dinv;   // L row by row and the diagonal blocks' inverses (fast solves)
+  bool fast_solve = false;     // both are kept
+  std::vector<DItem> hitem;    // shares of the factorizations, largest mesh first
+  DevBuf<DItem> item;
+  DevBuf<int32_t> progress;
+  bool shared = false;         // some mesh has more than one
+  int32_t maxb = 0, maxpad = 0;
   int64_t band_entries = 0, work_entries = 0;
   double analyse_ms = 0.0;
   // factor held in band: the matrix version it was computed from (0: none)
@@ -953,12 +1231,28 @@ int pf_direct_analyse(pf_ctx *ctx, DirectWork **pd, int64_t n, const int64_t *ro
   }
   size_t free_b = 0, total_b = 0;
   PF_HIP(hipMemGetInfo(&free_b, &total_b));
-  const double need = 8.0 * (double)boff;
+  const double need = 8.0 * (double)(boff + 2 * SB);
   const double have = (double)free_b + 8.0 * (double)D->band.n;
   if (need > have - 2.0e9) {
     pf_set_error("direct: the band factors need %.2f GB of device memory, %.2f GB are free", need * 1e-9,
                  have * 1e-9);
     return PF_ERR_NOMEM;
+  }
+  D->maxb = D->maxpad = 0;
+  for (const DMesh &M : D->hmesh) {
+    D->maxb = std::max(D->maxb, M.b);
+    D->maxpad = std::max(D->maxpad, M.npad);
+  }
+  // the second copy of the factor and the inverses, where they fit beside the band
+  D->fast_solve = D->maxb <= SMAXB && nmesh <= 65535 &&
+                  need * 2.0 + 8.0 * SB * (double)woff <=
+                      have + 8.0 * ((double)D->rows.n + (double)D->dinv.n) - 4.0e9;
+  if (D->fast_solve) {
+    PF_CHECK(D->rows.ensure(std::max<int64_t>(boff, 1) + 2 * SB));
+    PF_CHECK(D->dinv.ensure(std::max<int64_t>(SB * woff, 1)));
+  } else {
+    D->rows.release();
+    D->dinv.release();
   }
   D->hperm.assign(woff, 0);
   std::vector<int32_t> hbidx(n), hdm(n);
@@ -980,7 +1274,37 @@ int pf_direct_analyse(pf_ctx *ctx, DirectWork **pd, int64_t n, const int64_t *ro
     const DMesh &a = D->hmesh[x], &b = D->hmesh[y];
     return (double)a.npad * a.b * a.b > (double)b.npad * b.b * b.b;
   });
-  PF_CHECK(D->band.ensure(std::max<int64_t>(boff, 1)));
+  // shares: a mesh takes as many workgroups as keep it from outlasting the others (all the work over
+  // all the CUs), up to what its blocks can use: the time of a block on one workgroup (measured:
+  // 50 us at b = 350, 110 us at b = 690) over the time that passes between one block's columns and
+  // the next's (the last update, two diagonal tiles, the exchange: 20 us measured with many shares),
+  // and one.  More shares only take CUs from the other meshes: 24,640 equations of b = 350 took 38.8,
+  // 20.5, 15.6 and 15.6 ms with 1, 2, 4 and 6; 192 meshes up to b = 690, whole passes, 339, 241, 182, 171
+  // and 187 ms with up to 1, 2, 4, 6 and 10.
+  D->hitem.clear();
+  D->shared = false;
+  {
+    const auto block_us = [](const DMesh &M) { return 32.0 * M.b * (double)M.b / 190.0e3 + 29.0; };
+    const auto work = [&](const DMesh &M) { return block_us(M) * (M.npad / 32); };
+    double sum = 0.0;
+    for (const DMesh &M : D->hmesh) sum += work(M);
+    const double even = sum / ctx->num_cus;
+    for (int32_t m : qorder) {
+      const DMesh &M = D->hmesh[m];
+      // all shares of a mesh among the items that the resident workgroups take first, so that no
+      // share ever waits for one that is still in the queue
+      const double room = std::max(1.0, (double)ctx->num_cus - (double)D->hitem.size());
+      const double most = std::min(room, std::min(std::min(16.0, block_us(M) / 16.0 + 1.0), M.npad / 32.0));
+      const int G = std::max(1, (int)std::min(std::ceil(work(M) / even), std::floor(most)));
+      for (int g = 0; g < G; ++g) D->hitem.push_back(DItem{m, g, G, 0});
+      D->shared = D->shared || G > 1;
+    }
+  }
+  PF_CHECK(D->item.ensure(D->hitem.size()));
+  PF_CHECK(D->progress.ensure(nmesh));
+  PF_HIP(hipMemcpyAsync(D->item.p, D->hitem.data(), sizeof(DItem) * D->hitem.size(), hipMemcpyHostToDevice,
+                        ctx->stream));
+  PF_CHECK(D->band.ensure(std::max<int64_t>(boff, 1) + 2 * SB));
   PF_CHECK(D->mesh.ensure(nmesh));
   PF_CHECK(D->perm.ensure(std::max<int64_t>(woff, 1)));
   PF_CHECK(D->w.ensure(std::max<int64_t>(woff, 1)));
@@ -1026,15 +1350,66 @@ int launch_direct(pf_ctx *ctx, DirectWork *D, int mode, const double *rhs, doubl
   a.x = x;
   a.status = D->status.p;
   a.t_raw = D->t_raw.p;
+  a.rows = D->fast_solve ? D->rows.p : nullptr;
+  a.dinv = D->fast_solve ? D->dinv.p : nullptr;
   // two workgroups per CU at most; no more workgroups than meshes
   const int grid = std::max(1, std::min(D->nmesh, 2 * ctx->num_cus));
+  const auto solve = [&]() -> int {
+    k_direct_queue_reset<<<1, 64, 0, ctx->stream>>>(D->queue.p);
+    if (D->maxb <= 256)
+      k_band_solve<256, 1, 2><<<grid, 256, 0, ctx->stream>>>(a);
+    else if (D->maxb <= 512)
+      k_band_solve<512, 1, 2><<<grid, 512, 0, ctx->stream>>>(a);
+    else
+      k_band_solve<1024, 1, 1><<<grid, 1024, 0, ctx->stream>>>(a);
+    PF_HIP(hipGetLastError());
+    return PF_OK;
+  };
+  if (D->fast_solve && mode == 1) return solve();
+  // tiles of the widest block over the waves
+  const int tiles = (32 + D->maxb + 15) / 16;
+  const void *kernel;
+  if (!mfma) kernel = (const void *)k_direct<DBT, false, 2>;
+  else if (tiles <= 2 * (DBT / 64)) kernel = (const void *)k_direct<DBT, true, 2>;
+  else if (tiles <= 4 * (DBT / 64)) kernel = (const void *)k_direct<DBT, true, 4>;
+  else kernel = (const void *)k_direct<DBT, true, 6>;
   k_direct_queue_reset<<<1, 64, 0, ctx->stream>>>(D->queue.p);
   PF_HIP(hipGetLastError());
-  if (mfma)
-    k_direct<DBT, true><<<grid, DBT, 0, ctx->stream>>>(a);
-  else
-    k_direct<DBT, false><<<grid, DBT, 0, ctx->stream>>>(a);
-  PF_HIP(hipGetLastError());
+  if (D->fast_solve) {
+    a.mode = 2;
+    a.item = D->item.p;
+    a.nitem = (int32_t)D->hitem.size();
+    a.progress = D->progress.p;
+    k_direct_progress_reset<<<pf_blocks(D->nmesh, 256), 256, 0, ctx->stream>>>(D->nmesh, D->progress.p, D->status.p);
+    PF_HIP(hipGetLastError());
+    if (D->shared) {
+      // the shares of a mesh wait for each other: all workgroups resident
+      const int g2 = std::min((int)D->hitem.size(), ctx->num_cus);
+      void *args[] = {&a};
+      if (hipLaunchCooperativeKernel(kernel, dim3(g2), dim3(DBT), args, 0, ctx->stream) != hipSuccess) {
+        (void)hipGetLastError();  // whole meshes then
+        std::vector<DItem> whole;
+        for (const DItem &it : D->hitem)
+          if (it.g == 0) whole.push_back(DItem{it.m, 0, 1, 0});
+        D->hitem = whole;
+        D->shared = false;
+        PF_HIP(hipMemcpyAsync(D->item.p, D->hitem.data(), sizeof(DItem) * D->hitem.size(), hipMemcpyHostToDevice,
+                              ctx->stream));
+        a.nitem = (int32_t)D->hitem.size();
+      }
+    }
+  }
+  if (a.mode != 2 || !D->shared) {
+    void *args[] = {&a};
+    PF_HIP(hipLaunchKernel(kernel, dim3(grid), dim3(DBT), args, 0, ctx->stream));
+  }
+  if (D->fast_solve) {
+    const unsigned per = (unsigned)((D->maxpad / SB + 3) / 4);
+    k_diag_inverse<<<dim3(per, (unsigned)D->nmesh), 4 * SB, 0, ctx->stream>>>(D->nmesh, D->mesh.p, D->status.p,
+                                                                             D->band.p, D->dinv.p);
+    a.mode = 0;
+    PF_CHECK(solve());
+  }
   return PF_OK;
 }
 
@@ -1134,6 +1509,7 @@ int pf_direct_solve_device(pf_ctx *ctx, DirectWork *D, int64_t n, const int64_t 
     }
   }
   if (refactor && all_ok) D->factor_version = mat_version;
+  if (status < 0) pf_set_error("direct: a share of a factorization waited in vain for another");
   if (total) {
     std::memset(total, 0, sizeof(*total));
     total->status = status;
