@@ -10,12 +10,15 @@
 // this form does not do.
 //
 // Here every mesh runs bicgstab_CRS_2 (FEMSolverClass.f90:2199-2298) inside ONE launch of a
-// persistent kernel: a workgroup takes the next mesh from a queue (largest cost first),
-// runs that mesh's whole BiCGSTAB with workgroup-level reductions (wavefront shuffles + LDS,
-// bitwise the same scalars in every thread), records the result and takes the next mesh
-// until the queue is empty.  No workgroup ever waits for another, so the kernel needs no
-// fences, no grid barrier and no co-residency.  The queue reset and the kernel are captured
-// in one hipGraph.  Vectors of mesh m live in the DOF range of the mesh inside the union
+// persistent kernel: a workgroup takes the next item from a queue (largest cost first), a mesh
+// or a share of a mesh's rows, runs that mesh's whole BiCGSTAB, records the result and takes the
+// next item until the queue is empty.  The sums of a mesh are bitwise the same scalars in every thread
+// (wavefront shuffles + LDS, and then the shares' sums in share order).  One CU streams a matrix at
+// 40 GB/s or less, so that the largest meshes alone would decide the time: those are shared by several
+// workgroups, which meet five times per iteration (Meet) in a cooperative launch.  224 compact meshes of
+// 192 to 20,577 rows: 380 ms with one workgroup per mesh, 150 ms shared, at 3.1 TB/s of matrix; bound
+// now by that stream and, over half of the time, by the meshes that end last.  Without shares no
+// workgroup waits for another, and the queue reset and the kernel are captured in one hipGraph.  Vectors of mesh m live in the DOF range of the mesh inside the union
 // vectors, so the gathers of a mesh stay inside its own rows.
 //
 // Launch shapes (chosen by the autotuner): the blocked Sell3 layout with 64-node slices, or
@@ -29,6 +32,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <functional>
 #include <numeric>
 #include <vector>
 
@@ -39,6 +43,21 @@ namespace {
 struct BMesh {
   int64_t d0, d1;  // DOF rows d0 .. d1-1 of the union system
   int64_t s0, s1;  // Sell3 slices s0 .. s1-1
+};
+
+// share g of G of a mesh's rows
+struct BItem {
+  int32_t m, g, G, pad;
+};
+
+constexpr int SHARES_MAX = 16;
+
+// where the workgroups that share a mesh meet: arrivals so far, and the sums of each share, those of
+// one meeting kept until all have passed the next
+struct Team {
+  uint32_t arrived, failed;
+  uint32_t pad[30];
+  double part[2][SHARES_MAX][4];
 };
 
 template <typename V>
@@ -54,10 +73,11 @@ struct BMat {
 };
 
 struct BArgs {
-  int32_t nmesh, itrmax, stop_mode, inner_max;
+  int32_t nitem, itrmax, stop_mode, inner_max;
   double er0, rel, target, delta;
   const BMesh *mesh;
-  const int32_t *order;
+  const BItem *item;
+  Team *team;  // per mesh
   int32_t *queue;
   BMat<double> A;
   BMat<float> A32;
@@ -94,11 +114,97 @@ __device__ inline void wg_sum(double (&v)[NV], double (*sh)[BTB / 64]) {
   __syncthreads();
 }
 
+// s_sleep(1) polls for the other shares before a workgroup gives up: seconds, against the microseconds
+// between two meetings.  (The launch is cooperative and the shares are the first items of the
+// queue, one per workgroup: all of them run.)
+constexpr int SHARE_POLLS = 1 << 22;
+
+template <int BTB>
+struct Shared {
+  double sum[4][BTB / 64];
+  double part[SHARES_MAX][4];
+  int32_t next, failed;
+};
+
+// The workgroups of one mesh.  A mesh with one share needs no other workgroup, and then a meeting is
+// a workgroup barrier.  Two of the five meetings of an iteration also hand vectors over (publish):
+// those write the L2 back and drop stale lines, at about 10 us each, which is why a mesh is only shared
+// where its products take much longer.
+template <int BTB>
+struct Meet {
+  Shared<BTB> &sh;
+  Team *team;
+  int g, G;
+  uint32_t count;  // meetings so far
+  bool failed;
+
+  // all shares are here, and have read part of the meeting before the last; publish: what they stored
+  // before it is visible after it
+  __device__ void gather(bool publish) {
+    if (failed) return;
+    if (publish) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // every wave's stores are out
+    __syncthreads();
+    ++count;
+    if (threadIdx.x == 0) {
+      const uint32_t want = count * (uint32_t)G;
+      if (publish)
+        __hip_atomic_fetch_add(&team->arrived, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+      else {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __hip_atomic_fetch_add(&team->arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      int polls = 0;
+      while (__hip_atomic_load(&team->arrived, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < want &&
+             ++polls < SHARE_POLLS &&
+             (polls % 1024 || !__hip_atomic_load(&team->failed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)))
+        __builtin_amdgcn_s_sleep(1);
+      const bool late = __hip_atomic_load(&team->arrived, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < want ||
+                        __hip_atomic_load(&team->failed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (late) __hip_atomic_store(&team->failed, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (publish) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+      sh.failed = late;
+    }
+    __syncthreads();
+    failed = failed || __builtin_amdgcn_readfirstlane(sh.failed) != 0;
+  }
+
+  __device__ void publish() {
+    if (G == 1)
+      __syncthreads();
+    else
+      gather(true);
+  }
+
+  // the sums over the mesh, bitwise the same in every thread of every share
+  template <int NV>
+  __device__ void sum(double (&v)[NV], bool publish = false) {
+    wg_sum<BTB, NV>(v, sh.sum);
+    if (G == 1) return;
+    double (*part)[4] = team->part[count & 1];
+    if (threadIdx.x == 0)
+#pragma unroll
+      for (int k = 0; k < NV; ++k)
+        __hip_atomic_store(&part[g][k], v[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    gather(publish);
+    const int t = threadIdx.x;
+    if (t < 4 * G && (t & 3) < NV)
+      sh.part[t >> 2][t & 3] = __hip_atomic_load(&part[t >> 2][t & 3], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+      double s = 0.0;
+      for (int j = 0; j < G; ++j) s += sh.part[j][k];
+      v[k] = failed ? __builtin_nan("") : s;  // a failed mesh stops at its next test
+    }
+    __syncthreads();
+  }
+};
+
 // every row of the mesh's block of y = A*xf, one call op(row, sum) per row
 template <typename V, int L, int SUB, int BTB, typename XF, typename OP>
 __device__ inline void mesh_rows(const BMat<V> &A, const BMesh &bm, XF xf, OP op) {
   if (L == 1) {
-    const int wid = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
     for (int64_t s = bm.s0 + wid; s < bm.s1; s += BTB / 64) {
       V y0, y1, y2;
       pfdev::sell3_node<V, V>(A.soff, A.width, A.col, A.sval, s, lane, xf, y0, y1, y2);
@@ -139,7 +245,7 @@ struct MeshResult {
 
 // FP64 bicgstab_CRS_2 on one mesh, x0 = 0
 template <int L, int SUB, int BTB>
-__device__ MeshResult solve64(const BArgs &a, const BMesh &bm, double (*sh)[BTB / 64]) {
+__device__ MeshResult solve64(const BArgs &a, const BMesh &bm, Meet<BTB> &team) {
   const int64_t d0 = bm.d0, d1 = bm.d1;
   double t1[1] = {0.0};
   for (int64_t i = d0 + threadIdx.x; i < d1; i += BTB) {
@@ -150,7 +256,7 @@ __device__ MeshResult solve64(const BArgs &a, const BMesh &bm, double (*sh)[BTB 
     a.p[i] = bv;
     t1[0] += bv * bv;
   }
-  wg_sum<BTB, 1>(t1, sh);
+  team.sum(t1, true);
   const double bnorm2 = t1[0];
   double c1 = t1[0], rr = t1[0], rr1 = 0.0;
   MeshResult res{PF_NOT_CONVERGED, 0, 0, rr, 0.0};
@@ -167,7 +273,7 @@ __device__ MeshResult solve64(const BArgs &a, const BMesh &bm, double (*sh)[BTB 
       a.y[row] = yv;
       q1[0] += a.r0[row] * yv;
     });
-    wg_sum<BTB, 1>(q1, sh);
+    team.sum(q1, true);
     const double c2 = q1[0];
     const double alpha = c1 / c2;
     // v = A e, e = r - alpha y ; e.v, v.v
@@ -179,7 +285,7 @@ __device__ MeshResult solve64(const BArgs &a, const BMesh &bm, double (*sh)[BTB 
       q2[0] += e * vv;
       q2[1] += vv * vv;
     });
-    wg_sum<BTB, 2>(q2, sh);
+    team.sum(q2);
     if (q2[1] == 0.0) {  // FEMSolverClass.f90:2266, inside iteration itr+1
       res.status = PF_BREAKDOWN_VV;
       itr += 1;
@@ -196,7 +302,7 @@ __device__ MeshResult solve64(const BArgs &a, const BMesh &bm, double (*sh)[BTB 
       q3[0] += rn * rn;
       q3[1] += a.r0[i] * rn;
     }
-    wg_sum<BTB, 2>(q3, sh);
+    team.sum(q3);
     rr = q3[0];
     itr += 1;
     if (itr == 1) rr1 = rr;
@@ -215,7 +321,7 @@ __device__ MeshResult solve64(const BArgs &a, const BMesh &bm, double (*sh)[BTB 
     if (itr >= a.itrmax) break;
     c1 = q3[1];
     for (int64_t i = d0 + threadIdx.x; i < d1; i += BTB) a.p[i] = a.r[i] + beta * (a.p[i] - omega * a.y[i]);
-    __syncthreads();
+    team.publish();
   }
   res.iterations = itr;
   res.rr = rr;
@@ -225,7 +331,7 @@ __device__ MeshResult solve64(const BArgs &a, const BMesh &bm, double (*sh)[BTB 
 
 // FP32 recurrence on S A S with FP64 reliable updates on one mesh, x0 = 0
 template <int L, int SUB, int BTB>
-__device__ MeshResult solve32(const BArgs &a, const BMesh &bm, double (*sh)[BTB / 64]) {
+__device__ MeshResult solve32(const BArgs &a, const BMesh &bm, Meet<BTB> &team) {
   const int64_t d0 = bm.d0, d1 = bm.d1;
   // z_hi = z_lo = 0: the first true residual S (b - A S z_hi) is S b
   double t2[2] = {0.0, 0.0};
@@ -240,7 +346,7 @@ __device__ MeshResult solve32(const BArgs &a, const BMesh &bm, double (*sh)[BTB 
     t2[0] += (double)rf * (double)rf;
     t2[1] += bv * bv;
   }
-  wg_sum<BTB, 2>(t2, sh);
+  team.sum(t2, true);
   const double bn = sqrt(t2[1]);
   double c1 = t2[0], rr = t2[0];
   double maxr = sqrt(t2[0]);
@@ -257,7 +363,7 @@ __device__ MeshResult solve32(const BArgs &a, const BMesh &bm, double (*sh)[BTB 
       a.y32[row] = yv;
       q1[0] += (double)a.r032[row] * (double)yv;
     });
-    wg_sum<BTB, 1>(q1, sh);
+    team.sum(q1, true);
     const double c2 = q1[0];
     const double alpha_d = c1 / c2;
     if (!isfinite(alpha_d)) {
@@ -273,7 +379,7 @@ __device__ MeshResult solve32(const BArgs &a, const BMesh &bm, double (*sh)[BTB 
       q2[0] += (double)e * (double)vv;
       q2[1] += (double)vv * (double)vv;
     });
-    wg_sum<BTB, 2>(q2, sh);
+    team.sum(q2);
     if (q2[1] == 0.0 || !isfinite(q2[0] / q2[1])) {
       res.status = PF_BREAKDOWN_VV;
       itr += 1;
@@ -290,7 +396,7 @@ __device__ MeshResult solve32(const BArgs &a, const BMesh &bm, double (*sh)[BTB 
       q3[0] += (double)rn * (double)rn;
       q3[1] += (double)a.r032[i] * (double)rn;
     }
-    wg_sum<BTB, 2>(q3, sh);
+    team.sum(q3);
     rr = q3[0];
     itr += 1;
     const double nr = sqrt(rr);
@@ -311,7 +417,7 @@ __device__ MeshResult solve32(const BArgs &a, const BMesh &bm, double (*sh)[BTB 
         a.zhi[i] += (double)a.zlo[i];
         a.zlo[i] = 0.0f;
       }
-      __syncthreads();
+      team.publish();
       // r = S (b - A C z_hi) in FP64 -> FP32 ; |r|^2, |b - A x|^2, r0.r (restart: r0 = p = r)
       double q4[3] = {0.0, 0.0, 0.0};
       mesh_rows<double, L, SUB, BTB>(a.A, bm, ScaledX{a.cscale, a.zhi}, [&](int64_t row, double ax) {
@@ -326,7 +432,7 @@ __device__ MeshResult solve32(const BArgs &a, const BMesh &bm, double (*sh)[BTB 
         q4[1] += bu * bu;
         q4[2] += (double)a.r032[row] * (double)rf;
       });
-      wg_sum<BTB, 3>(q4, sh);
+      team.sum(q4, true);
       nupd += 1;
       itr_rep = itr;
       c1 = q4[2];
@@ -339,7 +445,7 @@ __device__ MeshResult solve32(const BArgs &a, const BMesh &bm, double (*sh)[BTB 
       }
     } else {
       for (int64_t i = d0 + threadIdx.x; i < d1; i += BTB) a.p32[i] = a.r32[i] + beta * (a.p32[i] - omega * a.y32[i]);
-      __syncthreads();
+      team.publish();
     }
   }
   // x = C (z_hi + z_lo)
@@ -350,25 +456,38 @@ __device__ MeshResult solve32(const BArgs &a, const BMesh &bm, double (*sh)[BTB 
   return res;
 }
 
-__global__ void k_queue_reset(int32_t *q) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) q[0] = 0;
+__global__ void k_queue_reset(int32_t *q, int32_t nmesh, Team *team) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i == 0) q[0] = 0;
+  if (i < nmesh) team[i].arrived = team[i].failed = 0;
 }
 
 template <int PREC, int L, int SUB, int BTB>
 __global__ void __launch_bounds__(BTB) k_batch(BArgs a) {
-  __shared__ double sh[4][BTB / 64];
-  __shared__ int32_t next;
+  __shared__ Shared<BTB> sh;
   for (;;) {
     __syncthreads();
-    if (threadIdx.x == 0) next = atomicAdd(a.queue, 1);
+    if (threadIdx.x == 0) sh.next = atomicAdd(a.queue, 1);
     __syncthreads();
-    const int32_t q = next;
-    if (q >= a.nmesh) break;
-    const int32_t m = a.order[q];
-    const BMesh bm = a.mesh[m];
+    const int32_t q = __builtin_amdgcn_readfirstlane(sh.next);
+    if (q >= a.nitem) break;
+    const BItem it = a.item[q];
+    const int32_t m = it.m;
+    BMesh bm = a.mesh[m];
+    Meet<BTB> team{sh, a.team + m, it.g, it.G, 0u, false};
+    if (it.G > 1) {  // this share's rows: slices for the blocked layout, else rows
+      const int64_t ns = bm.s1 - bm.s0, nd = bm.d1 - bm.d0, s0 = bm.s0, d0 = bm.d0;
+      const auto row = [&](int g) {
+        return L == 1 ? d0 + min((int64_t)192 * (ns * g / it.G), nd) : d0 + nd * g / it.G;
+      };
+      bm.s0 = s0 + ns * it.g / it.G;
+      bm.s1 = s0 + ns * (it.g + 1) / it.G;
+      bm.d0 = row(it.g);
+      bm.d1 = row(it.g + 1);
+    }
     const int64_t t0 = wall_clock64();
-    MeshResult res = PREC == 64 ? solve64<L, SUB, BTB>(a, bm, sh) : solve32<L, SUB, BTB>(a, bm, sh);
-    __syncthreads();
+    MeshResult res = PREC == 64 ? solve64<L, SUB, BTB>(a, bm, team) : solve32<L, SUB, BTB>(a, bm, team);
+    team.publish();
     // FP64 true residual |b - A x| / |b| of the mesh
     double t[2] = {0.0, 0.0};
     mesh_rows<double, L, SUB, BTB>(a.A, bm, pfdev::PlainX<double>{a.x}, [&](int64_t row, double ax) {
@@ -376,10 +495,10 @@ __global__ void __launch_bounds__(BTB) k_batch(BArgs a) {
       t[0] += rv * rv;
       t[1] += a.b[row] * a.b[row];
     });
-    wg_sum<BTB, 2>(t, sh);
-    if (threadIdx.x == 0) {
+    team.sum(t);
+    if (threadIdx.x == 0 && it.g == 0) {
       pf_batch_mesh_stats st;
-      st.status = res.status;
+      st.status = team.failed ? PF_ERR_HIP : res.status;
       st.iterations = res.iterations;
       st.replacements = res.replacements;
       st.workgroup = (int32_t)blockIdx.x;
@@ -438,7 +557,11 @@ struct BatchWork {
   std::vector<double> cost;
   std::vector<BMesh> hmesh;
   DevBuf<BMesh> mesh;
-  DevBuf<int32_t> order, queue, flag;
+  DevBuf<BItem> item;
+  DevBuf<Team> team;
+  std::vector<BItem> hitem;  // queue, largest mesh first, the shares of a mesh adjacent
+  bool shared = false;
+  DevBuf<int32_t> queue, flag;
   DevBuf<int64_t> snode, send, t_raw;
   int64_t nslices = 0;
   Sell3<double> s64;
@@ -467,6 +590,51 @@ struct BatchWork {
     if (gexec) (void)hipGraphExecDestroy(gexec);
   }
 };
+
+namespace {
+// The queue: meshes in the given order, each as one item or as the shares of several workgroups.  A
+// mesh is shared when it alone would outlast the batch.  Estimated time of an item: iterations (the cube
+// root of the mesh's rows) times 0.028 us per row of it (both products on one CU, measured: 20,577 rows
+// 600 us) plus what its meetings take (5 us alone, 30 us shared).  For a range of bounds T every mesh
+// takes as few workgroups as bring its items under T (at least 2000 rows each), largest first while
+// all the shares are among the items that the first workgroups take, one per CU, so that none waits
+// for one that is still in the queue; the bound whose queue ends first is kept.
+void share_out(int num_cus, const std::vector<BMesh> &mesh, const std::vector<int32_t> &order,
+               std::vector<BItem> &item, bool *shared) {
+  const auto time = [&](int32_t m, int G) {
+    const double rows = (double)(mesh[m].d1 - mesh[m].d0);
+    return std::cbrt(rows) * (0.028 * rows / G + (G > 1 ? 30.0 : 5.0));
+  };
+  double even = 0.0;
+  for (int32_t m : order) even += time(m, 1) / num_cus;
+  double best = 0.0;
+  for (double T = 0.0; T <= 4.0; T = T == 0.0 ? 0.7 : T * 1.1) {  // 0: no mesh shared
+    std::vector<BItem> trial;
+    std::vector<double> free_at(num_cus, 0.0);  // heap: when each CU takes its next item
+    double end = 0.0;
+    bool any = false;
+    for (int32_t m : order) {
+      const double most = std::min({(double)SHARES_MAX, (double)(mesh[m].d1 - mesh[m].d0) / 2000.0,
+                                    (double)num_cus - (double)trial.size()});
+      int G = 1;
+      while (T > 0.0 && G + 1 <= most && time(m, G) > T * even) ++G;
+      any = any || G > 1;
+      for (int g = 0; g < G; ++g) {
+        trial.push_back(BItem{m, g, G, 0});
+        std::pop_heap(free_at.begin(), free_at.end(), std::greater<double>());
+        free_at.back() += time(m, G);
+        end = std::max(end, free_at.back());
+        std::push_heap(free_at.begin(), free_at.end(), std::greater<double>());
+      }
+    }
+    if (T == 0.0 || end < 0.95 * best) {
+      best = end;
+      item = trial;
+      *shared = any;
+    }
+  }
+}
+}  // namespace
 
 void pf_batch_work_destroy(BatchWork *b) { delete b; }
 
@@ -542,7 +710,9 @@ int pf_batch_configure(pf_ctx *ctx, BatchWork **pb, int64_t n, const int64_t *ro
   std::iota(ord.begin(), ord.end(), 0);
   std::stable_sort(ord.begin(), ord.end(), [&](int32_t x, int32_t y) { return b->cost[x] > b->cost[y]; });
   PF_CHECK(b->mesh.ensure(nmesh));
-  PF_CHECK(b->order.ensure(nmesh));
+  share_out(ctx->num_cus, b->hmesh, ord, b->hitem, &b->shared);
+  PF_CHECK(b->item.ensure(b->hitem.size()));
+  PF_CHECK(b->team.ensure(nmesh));
   PF_CHECK(b->queue.ensure(1));
   PF_CHECK(b->flag.ensure(1));
   PF_CHECK(b->snode.ensure(b->nslices));
@@ -550,7 +720,8 @@ int pf_batch_configure(pf_ctx *ctx, BatchWork **pb, int64_t n, const int64_t *ro
   PF_CHECK(b->t_raw.ensure(2 * (size_t)nmesh));
   PF_CHECK(b->stat.ensure(nmesh));
   PF_HIP(hipMemcpyAsync(b->mesh.p, b->hmesh.data(), sizeof(BMesh) * nmesh, hipMemcpyHostToDevice, ctx->stream));
-  PF_HIP(hipMemcpyAsync(b->order.p, ord.data(), sizeof(int32_t) * nmesh, hipMemcpyHostToDevice, ctx->stream));
+  PF_HIP(hipMemcpyAsync(b->item.p, b->hitem.data(), sizeof(BItem) * b->hitem.size(), hipMemcpyHostToDevice,
+                        ctx->stream));
   PF_HIP(hipMemcpyAsync(b->snode.p, sn.data(), sizeof(int64_t) * b->nslices, hipMemcpyHostToDevice, ctx->stream));
   PF_HIP(hipMemcpyAsync(b->send.p, se.data(), sizeof(int64_t) * b->nslices, hipMemcpyHostToDevice, ctx->stream));
   // block-diagonal check and DOF=3 node blocks (needed by the blocked layout)
@@ -575,8 +746,20 @@ int pf_batch_configure(pf_ctx *ctx, BatchWork **pb, int64_t n, const int64_t *ro
 
 namespace {
 
+// shares wait for each other: a cooperative launch (PF_BATCH_WHOLE: not possible, nothing ran)
+constexpr int PF_BATCH_WHOLE = 1 << 20;
+
 template <int PREC, int L, int SUB, int BTB>
-int launch_one(pf_ctx *ctx, const BArgs &a, unsigned grid) {
+int launch_one(pf_ctx *ctx, const BArgs &a, unsigned grid, bool shared) {
+  if (shared) {
+    BArgs arg = a;
+    void *args[] = {&arg};
+    if (hipLaunchCooperativeKernel((const void *)k_batch<PREC, L, SUB, BTB>, dim3(grid), dim3(BTB), args, 0,
+                                   ctx->stream) == hipSuccess)
+      return PF_OK;
+    (void)hipGetLastError();
+    return PF_BATCH_WHOLE;
+  }
   k_batch<PREC, L, SUB, BTB><<<grid, BTB, 0, ctx->stream>>>(a);
   PF_HIP(hipGetLastError());
   return PF_OK;
@@ -618,9 +801,10 @@ struct Launcher {
   pf_ctx *ctx;
   const BArgs *a;
   unsigned grid;
+  bool shared;
   template <int PREC, int L, int SUB, int BTB>
   int operator()() const {
-    return launch_one<PREC, L, SUB, BTB>(ctx, *a, grid);
+    return launch_one<PREC, L, SUB, BTB>(ctx, *a, grid, shared);
   }
 };
 
@@ -719,7 +903,7 @@ BArgs make_args(BatchWork *b, const int64_t *row_ptr, const int32_t *col_idx, co
                 double *x, const pf_solve_opts &o, bool mixed) {
   BArgs a;
   std::memset(&a, 0, sizeof(a));
-  a.nmesh = b->nmesh;
+  a.nitem = (int32_t)b->hitem.size();
   a.itrmax = o.itrmax;
   a.stop_mode = o.stop_mode == 1 ? 1 : 0;
   a.inner_max = o.inner_max > 0 ? o.inner_max : 0;
@@ -728,7 +912,8 @@ BArgs make_args(BatchWork *b, const int64_t *row_ptr, const int32_t *col_idx, co
   a.target = o.target_relres;
   a.delta = o.inner_tol > 0.0 && o.inner_tol < 1.0 ? o.inner_tol : 0.1;
   a.mesh = b->mesh.p;
-  a.order = b->order.p;
+  a.item = b->item.p;
+  a.team = b->team.p;
   a.queue = b->queue.p;
   a.A = BMat<double>{row_ptr, col_idx, val, b->s64.soff.p, b->s64.width.p, b->s64.col.p, b->s64.val.p,
                      b->snode.p, b->send.p};
@@ -763,8 +948,9 @@ unsigned batch_grid(pf_ctx *ctx, BatchWork *b, const pf_batch_tune &t, bool mixe
   const int rc = mixed ? dispatch<32>(t, Occ{&occ}) : dispatch<64>(t, Occ{&occ});
   if (rc != PF_OK || occ < 1) occ = 1;
   int per_cu = t.blocks_per_cu > 0 ? std::min(t.blocks_per_cu, occ) : occ;
+  if (b->shared) per_cu = 1;  // what the shares are made for (224 compact meshes: 153 ms, 177 with two)
   int64_t g = (int64_t)ctx->num_cus * per_cu;
-  if (g > b->nmesh) g = b->nmesh;
+  g = std::min<int64_t>(g, (int64_t)b->hitem.size());
   return (unsigned)std::max<int64_t>(g, 1);
 }
 
@@ -772,7 +958,10 @@ unsigned batch_grid(pf_ctx *ctx, BatchWork *b, const pf_batch_tune &t, bool mixe
 int run_batch(pf_ctx *ctx, BatchWork *b, const BArgs &a, const pf_batch_tune &t, bool mixed, bool use_graph,
               float *ms) {
   const unsigned grid = batch_grid(ctx, b, t, mixed);
-  const Launcher ln{ctx, &a, grid};
+  const Launcher ln{ctx, &a, grid, b->shared};
+  const auto reset = [&] {
+    k_queue_reset<<<pf_blocks(b->nmesh, 256, INT32_MAX), 256, 0, ctx->stream>>>(b->queue.p, b->nmesh, b->team.p);
+  };
   BatchWork::GraphKey key;
   std::memset(&key, 0, sizeof(key));
   std::memcpy(&key.a, &a, sizeof(BArgs));
@@ -781,7 +970,7 @@ int run_batch(pf_ctx *ctx, BatchWork *b, const BArgs &a, const pf_batch_tune &t,
   key.mixed = mixed ? 1 : 0;
   PF_HIP(hipEventRecord(ctx->ev0, ctx->stream));
   bool launched = false;
-  if (use_graph && pf_graphs_allowed()) {
+  if (use_graph && !b->shared && pf_graphs_allowed()) {  // a cooperative launch is not captured
     if (!b->gexec || !b->gkey_valid || std::memcmp(&b->gkey, &key, sizeof(key)) != 0) {
       if (b->gexec) {
         PF_HIP(hipGraphExecDestroy(b->gexec));
@@ -791,7 +980,7 @@ int run_batch(pf_ctx *ctx, BatchWork *b, const BArgs &a, const pf_batch_tune &t,
       PF_CHECK(pf_capture_graph(
           ctx,
           [&] {
-            k_queue_reset<<<1, 64, 0, ctx->stream>>>(b->queue.p);
+            reset();
             return mixed ? dispatch<32>(t, ln) : dispatch<64>(t, ln);
           },
           &b->gexec));
@@ -806,8 +995,21 @@ int run_batch(pf_ctx *ctx, BatchWork *b, const BArgs &a, const pf_batch_tune &t,
     }
   }
   if (!launched) {
-    k_queue_reset<<<1, 64, 0, ctx->stream>>>(b->queue.p);
-    PF_CHECK(mixed ? dispatch<32>(t, ln) : dispatch<64>(t, ln));
+    reset();
+    const int rc = mixed ? dispatch<32>(t, ln) : dispatch<64>(t, ln);
+    if (rc == PF_BATCH_WHOLE) {  // e.g. fewer CUs available to this process: whole meshes then
+      std::vector<BItem> whole;
+      for (const BItem &it : b->hitem)
+        if (it.g == 0) whole.push_back(BItem{it.m, 0, 1, 0});
+      b->hitem = whole;
+      b->shared = false;
+      PF_HIP(hipMemcpyAsync(b->item.p, b->hitem.data(), sizeof(BItem) * b->hitem.size(), hipMemcpyHostToDevice,
+                            ctx->stream));
+      BArgs aw = a;
+      aw.nitem = (int32_t)b->hitem.size();
+      return run_batch(ctx, b, aw, t, mixed, use_graph, ms);
+    }
+    PF_CHECK(rc);
   }
   PF_HIP(hipEventRecord(ctx->ev1, ctx->stream));
   PF_HIP(hipEventSynchronize(ctx->ev1));
@@ -877,6 +1079,10 @@ int pf_batch_solve_device(pf_ctx *ctx, BatchWork *b, const int64_t *row_ptr, con
     reps += st[m].replacements;
     worst = std::max(worst, st[m].true_relres);
     if (status == PF_OK && st[m].status != PF_OK) status = st[m].status;
+    if (st[m].status == PF_ERR_HIP) {
+      pf_set_error("batch: the workgroups of mesh %d did not run together", m);
+      return PF_ERR_HIP;
+    }
   }
   if (mesh_stats) std::memcpy(mesh_stats, st.data(), sizeof(pf_batch_mesh_stats) * b->nmesh);
   if (total) {

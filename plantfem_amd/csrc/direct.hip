@@ -717,10 +717,10 @@ __device__ inline double dpp_move(double x) {
 // workgroup multiplies the block of w by the inverse of the diagonal block, eight lanes per row, and
 // then subtracts the block's columns (rows) from the b <= NR BT entries of w that follow (precede), NR
 // per thread; their loads are issued DEPTH blocks ahead.
-// Bound: what one CU streams (37 GB/s: b = 350, 90 KB per block, 2.4 us per block).  DEPTH: as many blocks as the registers hold (b <= 512: 3.73 ms per
-// solve of 24,640 equations with 2, 4.08 with 1; the solves by blocks of 16: 11 ms).  b <= 1024: 1024
-// threads with one entry each (22.1 ms for 192 meshes up to b = 690) rather than 512 with two
-// (24.8 ms).
+// Bound: what one CU streams (37 GB/s: b = 350, 90 KB per block, 2.4 us per block).  DEPTH: as many
+// blocks as the registers hold (b <= 512: 3.73 ms per solve of 24,640 equations with 2, 4.08 with 1; the
+// solves by blocks of 16: 11 ms).  b <= 1024: 1024 threads with one entry each (22.1 ms for 192 meshes up
+// to b = 690) rather than 512 with two (24.8 ms).
 template <int BT, int NR, int DEPTH, bool FWD>
 __device__ __forceinline__ void band_sweep(const DMesh &M, const double *__restrict__ L, const double *__restrict__ dinv,
                            double *__restrict__ w, double *sw, double *sY) {

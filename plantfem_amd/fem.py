@@ -1050,7 +1050,7 @@ class FEMSolver:
         """Solve every mesh of the batch in one persistent kernel; returns (x, per-mesh stats).
         preconditioning="PointJacobi" scales the eliminated rows first (JacobiPreconditionerCRS,
         in place) and solves the scaled systems.  algorithm="GaussJordan": the direct solve of
-        solve(algorithm="GaussJordan") for every mesh, one workgroup per mesh."""
+        solve(algorithm="GaussJordan") for every mesh."""
         self._flush()
         if preconditioning is None and algorithm == "GaussJordan":
             st = np.zeros(self._nmesh, dtype=L.BATCH_STATS_DTYPE)
