@@ -95,68 +95,70 @@ __global__ void k_dinv(int64_t n, const int64_t *__restrict__ rp, const int32_t 
   dinv[i] = (red[i] >= 0 && d != 0.0) ? 1.0 / fabs(d) : 0.0;
 }
 
-// columns c of S, AS, BS (n rows) scaled by s[c]
+// columns c of S, AS, BS (n rows) scaled by 1 / sqrt(s[c])
 __global__ void k_scale_cols(int64_t n, int64_t c0, int64_t cols, const double *__restrict__ s, double *__restrict__ S,
                              double *__restrict__ AS, double *__restrict__ BS) {
   for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < n * cols; t += (int64_t)gridDim.x * blockDim.x) {
     const int64_t c = t / n;
     const int64_t g = c0 * n + t;
-    const double f = s[c];
+    const double f = s[c] > 0.0 ? 1.0 / sqrt(s[c]) : 0.0;
     S[g] *= f;
     AS[g] *= f;
     BS[g] *= f;
   }
 }
 
-__global__ void k_copy(int64_t count, const double *__restrict__ a, double *__restrict__ b) {
-  for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < count; t += (int64_t)gridDim.x * blockDim.x)
-    b[t] = a[t];
+// column src to dst, in S alone or (gridDim.y = 3) in S, AS and BS
+__global__ void k_copy(int64_t n, int64_t src, int64_t dst, double *S, double *AS, double *BS) {
+  double *M = blockIdx.y == 0 ? S : (blockIdx.y == 1 ? AS : BS);
+  for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < n; t += (int64_t)gridDim.x * blockDim.x)
+    M[dst * n + t] = M[src * n + t];
 }
 
 // Rayleigh-Ritz update of the search block, in place: for M = S, AS, BS (leading dimension
 // n, k columns [X | W | P]) and the lowest m Ritz vectors C (k x m, leading dimension ldc),
 // X_M = M C and, with k > m, P_M = [W P]_M C[m:k, :] into columns 2m.. of M.  One thread per
-// row reads the row's k entries before it writes the row's new ones.
+// row reads the row's k entries before it writes the row's new ones; blockIdx.y = the matrix (25,704
+// rows, k = 18: 13.8 us; 27 us with 100 workgroups that took the matrices in turn: latency).
 template <int MAXM>
 __global__ void __launch_bounds__(256) k_rr_update(int64_t n, int k, int m, const double *__restrict__ C, int ldc,
                                                    double *S, double *AS, double *BS) {
+  double *M = blockIdx.y == 0 ? S : (blockIdx.y == 1 ? AS : BS);
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-    for (int w = 0; w < 3; ++w) {
-      double *M = w == 0 ? S : (w == 1 ? AS : BS);
-      double xo[MAXM], po[MAXM];
+    double xo[MAXM], po[MAXM];
 #pragma unroll
-      for (int j = 0; j < MAXM; ++j) xo[j] = po[j] = 0.0;
-      for (int c = 0; c < k; ++c) {
-        const double v = M[i + (int64_t)c * n];
-        if (c < m) {
+    for (int j = 0; j < MAXM; ++j) xo[j] = po[j] = 0.0;
+    for (int c = 0; c < k; ++c) {
+      const double v = M[i + (int64_t)c * n];
+      if (c < m) {
 #pragma unroll
-          for (int j = 0; j < MAXM; ++j)
-            if (j < m) xo[j] += v * C[c + j * ldc];
-        } else {
+        for (int j = 0; j < MAXM; ++j)
+          if (j < m) xo[j] += v * C[c + j * ldc];
+      } else {
 #pragma unroll
-          for (int j = 0; j < MAXM; ++j)
-            if (j < m) po[j] += v * C[c + j * ldc];
-        }
+        for (int j = 0; j < MAXM; ++j)
+          if (j < m) po[j] += v * C[c + j * ldc];
       }
-#pragma unroll
-      for (int j = 0; j < MAXM; ++j)
-        if (j < m) {
-          M[i + (int64_t)j * n] = xo[j] + po[j];
-          if (k > m) M[i + (int64_t)(2 * m + j) * n] = po[j];
-        }
     }
+#pragma unroll
+    for (int j = 0; j < MAXM; ++j)
+      if (j < m) {
+        M[i + (int64_t)j * n] = xo[j] + po[j];
+        if (k > m) M[i + (int64_t)(2 * m + j) * n] = po[j];
+      }
   }
 }
 
 // out[c] = sum_i X[i, c] Y[i, c] in two steps: CD_NB blocks per column (blockIdx.y = column)
 // leave one partial each, with four loads in flight per thread; then one thread per column
-// adds its CD_NB partials in order
+// adds its CD_NB partials in order.  blockIdx.z = 1: the columns of the pair X2, Y2, after the first's
 constexpr int CD_NB = 64;
 __global__ void __launch_bounds__(256) k_coldots_part(int64_t n, const double *__restrict__ X,
-                                                      const double *__restrict__ Y, double *__restrict__ part) {
+                                                      const double *__restrict__ Y, const double *__restrict__ X2,
+                                                      const double *__restrict__ Y2, double *__restrict__ part) {
   __shared__ double sh[4];
-  const int64_t c = blockIdx.y;
-  const double *x = X + c * n, *y = Y + c * n;
+  const int64_t c = blockIdx.y + (int64_t)gridDim.y * blockIdx.z;
+  const double *x = (blockIdx.z ? X2 : X) + blockIdx.y * n, *y = (blockIdx.z ? Y2 : Y) + blockIdx.y * n;
   const int64_t stride = (int64_t)CD_NB * 256;
   double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
   int64_t i = blockIdx.x * 256 + threadIdx.x;
@@ -183,10 +185,13 @@ __global__ void k_coldots_sum(int cols, const double *__restrict__ part, double 
 }
 
 // partial Gram matrices G = S^T T over row tiles (S, T column-major n x k, k <= GK): 32 rows
-// of both in LDS per step, thread p accumulates pairs p, p + 1024, ...; part[block][j*k + i]
+// of both in LDS per step, thread p accumulates pairs p, p + 1024, ...; part[j*k + i][block].  blockIdx.y = 1: S^T T2, its
+// pairs after the first's (25,704 rows, k = 18: 15.5 us; 22 us as two launches of 256 workgroups)
 constexpr int GK = 96, GR = 32, GPER = (GK * GK + 1023) / 1024;
 __global__ void __launch_bounds__(1024) k_gram(int64_t n, int k, const double *__restrict__ S,
-                                               const double *__restrict__ T, double *__restrict__ part) {
+                                               const double *__restrict__ T1, const double *__restrict__ T2,
+                                               double *__restrict__ part) {
+  const double *__restrict__ T = blockIdx.y ? T2 : T1;
   __shared__ double sS[GR][GK];
   __shared__ double sT[GR][GK];
   const int npair = k * k;
@@ -217,7 +222,7 @@ __global__ void __launch_bounds__(1024) k_gram(int64_t n, int k, const double *_
 #pragma unroll
   for (int q = 0; q < GPER; ++q) {
     const int p = threadIdx.x + q * 1024;
-    if (p < npair) part[(int64_t)p * gridDim.x + blockIdx.x] = acc[q];
+    if (p < npair) part[((int64_t)npair * blockIdx.y + p) * gridDim.x + blockIdx.x] = acc[q];
   }
 }
 
@@ -297,10 +302,10 @@ bool small_pencil(int k, const std::vector<double> &GA, const std::vector<double
           C[(size_t)p * k + r] = cs * xp - sn * xq;
           C[(size_t)q * k + r] = sn * xp + cs * xq;
         }
-        for (int r = 0; r < k; ++r) {
-          const double vp = V[(size_t)r * k + p], vq = V[(size_t)r * k + q];
-          V[(size_t)r * k + p] = cs * vp - sn * vq;
-          V[(size_t)r * k + q] = sn * vp + cs * vq;
+        for (int r = 0; r < k; ++r) {  // V is kept transposed: rows
+          const double vp = V[(size_t)p * k + r], vq = V[(size_t)q * k + r];
+          V[(size_t)p * k + r] = cs * vp - sn * vq;
+          V[(size_t)q * k + r] = sn * vp + cs * vq;
         }
       }
   }
@@ -313,13 +318,21 @@ bool small_pencil(int k, const std::vector<double> &GA, const std::vector<double
     const int o = ord[c];
     theta[c] = C[(size_t)o * k + o];
     for (int i = k - 1; i >= 0; --i) {  // z = L^-T y (back substitution)
-      double t = V[(size_t)i * k + o];
+      double t = V[(size_t)o * k + i];
       for (int q = i + 1; q < k; ++q) t -= Lm[(size_t)q * k + i] * Z[(size_t)c * k + q];
       Z[(size_t)c * k + i] = t / Lm[(size_t)i * k + i];
     }
   }
   return true;
 }
+
+// what the host exchanges with the device in an iteration, pinned
+struct Pinned {
+  double *p = nullptr;
+  ~Pinned() {
+    if (p) (void)hipHostFree(p);
+  }
+};
 
 struct Handle {
   rocblas_handle h = nullptr;
@@ -410,76 +423,80 @@ int pf_eig_device(pf_ctx *ctx, int64_t n, const int64_t *row_ptr, const int32_t 
   }
   *count = nev;
   const int64_t K = 3 * m;
-  DevBuf<double> S, AS, BS, R, dinv, GA, GB, th, E, sc;
-  DevBuf<rocblas_int> info;
+  DevBuf<double> S, AS, BS, R, dinv, G, sc;
   PF_CHECK(S.ensure((size_t)(n * K)));
   PF_CHECK(AS.ensure((size_t)(n * K)));
   PF_CHECK(BS.ensure((size_t)(n * K)));
   PF_CHECK(R.ensure((size_t)(n * m)));
   PF_CHECK(dinv.ensure((size_t)n));
-  PF_CHECK(GA.ensure((size_t)(K * K)));
-  PF_CHECK(GB.ensure((size_t)(K * K)));
-  PF_CHECK(th.ensure((size_t)K));
-  PF_CHECK(E.ensure((size_t)K));
+  // the projected pencil (two k x k matrices), then its vectors (k x k) and the lowest m values
+  PF_CHECK(G.ensure((size_t)(2 * K * K)));
   PF_CHECK(sc.ensure((size_t)K));
-  PF_CHECK(info.ensure(1));
+  Pinned host;
+  PF_HIP(hipHostMalloc((void **)&host.p, sizeof(double) * (size_t)(2 * K * K + K), hipHostMallocDefault));
   // one workgroup per CU for the partial Gram matrices (a wavefront per entry sums them)
   const unsigned gram_blocks = (unsigned)std::min<int64_t>((n + GR - 1) / GR, (int64_t)std::max(ctx->num_cus, 1));
   DevBuf<double> gpart;
-  PF_CHECK(gpart.ensure((size_t)gram_blocks * K * K + 1));
+  PF_CHECK(gpart.ensure((size_t)gram_blocks * 2 * K * K + 1));
   double *X = S.p, *Wb = S.p + n * m;  // P: columns 2m .. 3m
   double *AX = AS.p, *AW = AS.p + n * m;
   double *BX = BS.p, *BW = BS.p + n * m;
   k_dinv<<<pf_blocks(n, 256, INT32_MAX), 256, 0, st>>>(n, row_ptr, col_idx, A, red.p, dinv.p);
   k_init_block<<<grid_for(n * m), 256, 0, st>>>(n, m, red.p, X);
   PF_HIP(hipGetLastError());
-  // every column of a block in one launch (the matrix streamed once, not once per column)
-  auto spmv_block = [&](const double *M, const double *in, double *out, int64_t cols) -> int {
-    return pf_spmm_crs_launch(ctx, n, cols, row_ptr, col_idx, M, in, out, avg_row);
+  // A and B times every column of a block in one launch
+  auto products = [&](const double *in, double *outA, double *outB, int64_t cols) -> int {
+    return pf_spmm_pair_launch(ctx, n, cols, row_ptr, col_idx, A, B, in, outA, outB, avg_row);
   };
   // out[0 .. cols) = column dots of X and Y (column-major, leading dimension n)
   DevBuf<double> cdpart;
   PF_CHECK(cdpart.ensure((size_t)K * CD_NB));
-  auto coldots = [&](const double *Xc, const double *Yc, int64_t cols, double *out) -> int {
-    k_coldots_part<<<dim3(CD_NB, (unsigned)cols), 256, 0, st>>>(n, Xc, Yc, cdpart.p);
-    k_coldots_sum<<<(unsigned)((cols + 63) / 64), 64, 0, st>>>((int)cols, cdpart.p, out);
+  // (and, X2 given, cols more of X2 and Y2)
+  auto coldots = [&](const double *Xc, const double *Yc, int64_t cols, double *out, const double *X2,
+                     const double *Y2) -> int {
+    k_coldots_part<<<dim3(CD_NB, (unsigned)cols, X2 ? 2 : 1), 256, 0, st>>>(n, Xc, Yc, X2, Y2, cdpart.p);
+    const int64_t all = X2 ? 2 * cols : cols;
+    k_coldots_sum<<<(unsigned)((all + 63) / 64), 64, 0, st>>>((int)all, cdpart.p, out);
     PF_HIP(hipGetLastError());
     return PF_OK;
   };
   // Rayleigh-Ritz on the first k columns of S; keeps the lowest m in X (and, with k > m, the
   // W/P part of the combination in P).  Returns 1 when dsygvd fails.
   std::vector<double> h_th((size_t)K);
+  const double *th = nullptr;  // the lowest m values on the device
   auto rayleigh_ritz = [&](int64_t k, int *failed) -> int {
     // Gram matrices S^T (A S) and S^T (B S) (a transposed tall-skinny product, which the
     // library GEMM runs on a handful of workgroups: 21 ms for k = 30, n = 134k; this: one pass)
-    k_gram<<<gram_blocks, 1024, 0, st>>>(n, (int)k, S.p, AS.p, gpart.p);
-    k_gram_sum<<<(unsigned)((k * k * 64 + 255) / 256), 256, 0, st>>>((int)(k * k), (int)gram_blocks, gpart.p, GA.p);
-    k_gram<<<gram_blocks, 1024, 0, st>>>(n, (int)k, S.p, BS.p, gpart.p);
-    k_gram_sum<<<(unsigned)((k * k * 64 + 255) / 256), 256, 0, st>>>((int)(k * k), (int)gram_blocks, gpart.p, GB.p);
+    const int64_t kk = k * k;
+    k_gram<<<dim3(gram_blocks, 2), 1024, 0, st>>>(n, (int)k, S.p, AS.p, BS.p, gpart.p);
+    k_gram_sum<<<(unsigned)((2 * kk * 64 + 255) / 256), 256, 0, st>>>((int)(2 * kk), (int)gram_blocks, gpart.p, G.p);
     PF_HIP(hipGetLastError());
-    std::vector<double> hA((size_t)k * k), hB((size_t)k * k), hth, hZ;
-    PF_HIP(hipMemcpyAsync(hA.data(), GA.p, sizeof(double) * k * k, hipMemcpyDeviceToHost, st));
-    PF_HIP(hipMemcpyAsync(hB.data(), GB.p, sizeof(double) * k * k, hipMemcpyDeviceToHost, st));
+    PF_HIP(hipMemcpyAsync(host.p, G.p, sizeof(double) * 2 * kk, hipMemcpyDeviceToHost, st));
     PF_HIP(hipStreamSynchronize(st));
+    const std::vector<double> hA(host.p, host.p + kk), hB(host.p + kk, host.p + 2 * kk);
+    std::vector<double> hth, hZ;
     *failed = !small_pencil((int)k, hA, hB, hth, hZ);
     if (*failed) return PF_OK;
     for (int64_t c = 0; c < k; ++c) h_th[c] = hth[c];
-    PF_HIP(hipMemcpyAsync(GA.p, hZ.data(), sizeof(double) * k * k, hipMemcpyHostToDevice, st));
-    // X = S C, AX = AS C, BX = BS C for the lowest m vectors C = GA[:, 0:m], and with k > m
+    // vectors and values in one copy
+    std::copy(hZ.begin(), hZ.end(), host.p);
+    std::copy(hth.begin(), hth.begin() + m, host.p + kk);
+    th = G.p + kk;
+    PF_HIP(hipMemcpyAsync(G.p, host.p, sizeof(double) * (kk + m), hipMemcpyHostToDevice, st));
+    // X = S C, AX = AS C, BX = BS C for the lowest m vectors C = G[:, 0:m], and with k > m
     // P = [W P] C[m:k, :] (the same for AS, BS): one pass over the block, in place
-    const unsigned rg = pf_blocks(n, 256, (int64_t)ctx->num_cus * 8);
+    const dim3 rg(pf_blocks(n, 256, (int64_t)ctx->num_cus * 8), 3);
     if (m <= 8)
-      k_rr_update<8><<<rg, 256, 0, st>>>(n, (int)k, (int)m, GA.p, (int)k, S.p, AS.p, BS.p);
+      k_rr_update<8><<<rg, 256, 0, st>>>(n, (int)k, (int)m, G.p, (int)k, S.p, AS.p, BS.p);
     else if (m <= 16)
-      k_rr_update<16><<<rg, 256, 0, st>>>(n, (int)k, (int)m, GA.p, (int)k, S.p, AS.p, BS.p);
+      k_rr_update<16><<<rg, 256, 0, st>>>(n, (int)k, (int)m, G.p, (int)k, S.p, AS.p, BS.p);
     else
-      k_rr_update<32><<<rg, 256, 0, st>>>(n, (int)k, (int)m, GA.p, (int)k, S.p, AS.p, BS.p);
+      k_rr_update<32><<<rg, 256, 0, st>>>(n, (int)k, (int)m, G.p, (int)k, S.p, AS.p, BS.p);
     PF_HIP(hipGetLastError());
     return PF_OK;
   };
 
-  PF_CHECK(spmv_block(A, X, AX, m));
-  PF_CHECK(spmv_block(B, X, BX, m));
+  PF_CHECK(products(X, AX, BX, m));
   int failed = 0;
   PF_CHECK(rayleigh_ritz(m, &failed));
   if (failed) {
@@ -488,18 +505,15 @@ int pf_eig_device(pf_ctx *ctx, int64_t n, const int64_t *row_ptr, const int32_t 
     return res.status;
   }
   bool have_p = false;
-  std::vector<double> rn((size_t)m), bn((size_t)m), wn((size_t)(2 * m));
+  std::vector<double> rn((size_t)m), bn((size_t)m);
   int it = 0;
   res.status = PF_NOT_CONVERGED;
   for (it = 1; it <= maxit; ++it) {
-    PF_HIP(hipMemcpyAsync(th.p, h_th.data(), sizeof(double) * m, hipMemcpyHostToDevice, st));
-    k_residual_block<<<grid_for(n * m), 256, 0, st>>>(n, m, AX, BX, th.p, dinv.p, red.p, R.p, Wb);
+    k_residual_block<<<grid_for(n * m), 256, 0, st>>>(n, m, AX, BX, th, dinv.p, red.p, R.p, Wb);
     PF_HIP(hipGetLastError());
-    PF_CHECK(coldots(R.p, R.p, m, sc.p));
-    PF_CHECK(coldots(BX, BX, m, sc.p + m));
-    PF_HIP(hipGetLastError());
-    std::vector<double> nrm((size_t)(2 * m));
-    PF_HIP(hipMemcpyAsync(nrm.data(), sc.p, sizeof(double) * 2 * m, hipMemcpyDeviceToHost, st));
+    PF_CHECK(coldots(R.p, R.p, m, sc.p, BX, BX));
+    double *nrm = host.p + 2 * K * K;  // 2 m of the K there, apart from the upload that may still run
+    PF_HIP(hipMemcpyAsync(nrm, sc.p, sizeof(double) * 2 * m, hipMemcpyDeviceToHost, st));
     PF_HIP(hipStreamSynchronize(st));
     for (int64_t c = 0; c < m; ++c) {
       rn[c] = std::sqrt(nrm[c]);
@@ -524,28 +538,17 @@ int pf_eig_device(pf_ctx *ctx, int64_t n, const int64_t *row_ptr, const int32_t 
     const int64_t na = (int64_t)act.size();
     // compact [X | W_act | P_act]: every copy moves a column to a lower index, in order
     for (int64_t q = 0; q < na; ++q)
-      if (act[q] != q) k_copy<<<grid_for(n), 256, 0, st>>>(n, Wb + act[q] * n, Wb + q * n);
+      if (act[q] != q) k_copy<<<grid_for(n), 256, 0, st>>>(n, m + act[q], m + q, S.p, AS.p, BS.p);
     if (have_p)
       for (int64_t q = 0; q < na; ++q) {
         const int64_t src = 2 * m + act[q], dst = m + na + q;
-        if (src != dst) {
-          k_copy<<<grid_for(n), 256, 0, st>>>(n, S.p + src * n, S.p + dst * n);
-          k_copy<<<grid_for(n), 256, 0, st>>>(n, AS.p + src * n, AS.p + dst * n);
-          k_copy<<<grid_for(n), 256, 0, st>>>(n, BS.p + src * n, BS.p + dst * n);
-        }
+        if (src != dst) k_copy<<<dim3(grid_for(n), 3), 256, 0, st>>>(n, src, dst, S.p, AS.p, BS.p);
       }
     PF_HIP(hipGetLastError());
-    PF_CHECK(spmv_block(A, Wb, AW, na));
-    PF_CHECK(spmv_block(B, Wb, BW, na));
+    PF_CHECK(products(Wb, AW, BW, na));
     // unit B-norm columns of W (and P)
     const int64_t ncols = have_p ? 2 * na : na;
-    PF_CHECK(coldots(S.p + m * n, BS.p + m * n, ncols, sc.p));
-    PF_HIP(hipGetLastError());
-    PF_HIP(hipMemcpyAsync(wn.data(), sc.p, sizeof(double) * ncols, hipMemcpyDeviceToHost, st));
-    PF_HIP(hipStreamSynchronize(st));
-    std::vector<double> f((size_t)ncols);
-    for (int64_t c = 0; c < ncols; ++c) f[c] = wn[c] > 0.0 ? 1.0 / std::sqrt(wn[c]) : 0.0;
-    PF_HIP(hipMemcpyAsync(sc.p, f.data(), sizeof(double) * ncols, hipMemcpyHostToDevice, st));
+    PF_CHECK(coldots(S.p + m * n, BS.p + m * n, ncols, sc.p, nullptr, nullptr));
     k_scale_cols<<<grid_for(n * ncols), 256, 0, st>>>(n, m, ncols, sc.p, S.p, AS.p, BS.p);
     PF_HIP(hipGetLastError());
     PF_CHECK(rayleigh_ritz(m + ncols, &failed));
