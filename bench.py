@@ -69,6 +69,12 @@ def spmv_bytes(kind: int, n: int, nnz: int) -> float:
     return 4.0 * nnz + 4.0 * nblocks + 12.0 * nslices + 8 + 8.0 * n  # blocked FP32
 
 
+def elem_bytes(n: int, ne: int) -> float:
+    """Algorithmic HBM bytes of one y = A x from the elements (nodes, coordinates and the two material
+    values once, x once, y once)."""
+    return (8 * 4.0 + 2 * 8.0) * ne + 8.0 * n + 16.0 * n
+
+
 def main(argv=None):
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
@@ -149,7 +155,7 @@ def main(argv=None):
         s.solve(precision=48, target_relres=1e-30, stop_mode=1, download=False, use_graph=0,
                 raise_on_breakdown=False, **P48)
         log(f"profile: {s.last_stats['iterations']} precision 48 iterations")
-        for kind in (1, 4):  # the fused iteration on CRS rows, plain and with x staged in LDS
+        for kind in (2, 1, 4):  # the fused iteration blocked, on CRS rows, and with x staged in LDS
             s.solve(stop_mode=1, download=False, use_graph=0, raise_on_breakdown=False, spmv_kind=kind)
             log(f"profile: {s.last_stats['iterations']} FP64 iterations, spmv kind {s.last_stats['spmv_kind_used']}")
         # element-matrix kernels: the reference-order one (kind 0, in the assembly above) against
@@ -281,20 +287,23 @@ def main(argv=None):
         spmv[name] = {"ms": round(ms, 4), "GB/s": round(gbs, 1), "frac_hbm": round(gbs / HBM_PEAK_GBS, 3)}
         log(f"spmv {name}: {ms:.3f} ms {gbs:.0f} GB/s")
 
-    # ---- roofline of the dominant kernel: y = A p (+ r0.y), blocked FP64 ---------------
-    k1_bytes = spmv_bytes(2, n, nnz) + 8.0 * n  # + r0 read for the fused dot
+    # ---- roofline of the dominant kernel: y = A p (+ r0.y), from the elements or blocked FP64 ----
+    kind = int(st64["spmv_kind_used"])
+    k1_bytes = (elem_bytes(n, a.size ** 3) if kind == 5 else spmv_bytes(kind, n, nnz)) + 8.0 * n  # + r0 (fused dot)
     k1_ms = float(np.mean([x["spmv_p_ms"] for x in stats]))
     k1_gbs = k1_bytes / (k1_ms * 1e-3) / 1e9
     # measured HBM bytes per K1 launch (rocprofv3 FETCH_SIZE + WRITE_SIZE, copy-kernel calibrated)
     traffic = None
     tfile = ROOT / "profiles" / f"traffic_box{a.size}.json"
-    if tfile.exists():
+    if kind == 2 and tfile.exists():
         tr = json.loads(tfile.read_text())
         if tr.get("n_dof") == n and tr.get("nnz") == nnz:
             traffic = tr["bytes_per_launch"]
     roofline = {"bound": "hbm", "achieved": round(k1_gbs, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": round(k1_gbs / HBM_PEAK_GBS, 4), "traffic": traffic,
-                "kernel": "k_spmv_p (blocked FP64 y=A p fused with r0.y)", "bytes_per_launch": k1_bytes,
+                "kernel": ("k_el_p + k_el_rows_p (y=A p element by element, fused with r0.y)" if kind == 5 else
+                           "k_spmv_p (" + {1: "CRS rows", 2: "blocked", 4: "CRS rows, x staged in LDS"}[kind]
+                           + " FP64 y=A p fused with r0.y)"), "bytes_per_launch": k1_bytes,
                 "avg_launch_ms": round(k1_ms, 4)}
     s.close()
 
