@@ -60,10 +60,11 @@ typedef struct {
                                 matrix, computed at the first such solve and kept (ILU_MATRIX);
                               3 "PointJacobi" as the reference's branch runs it: the scaling and no
                                 solver call, so x = x0 (zeros) with the fixed values */
-  int32_t spmv_kind;     /* 0 auto (element by element on large systems whose values are exactly a
-                            hex8 mesh's stiffness; else blocked when the CRS has DOF=3 node blocks and pads little, else CRS
-                            rows, with x staged in LDS for the unpreconditioned FP64 solve from 2^18
-                            rows on), 1 CRS row kernel, 2 blocked, 4 CRS rows with x staged in LDS per
+  int32_t spmv_kind;     /* 0 auto (FP64 systems small enough: CRS rows kept on the chip, all iterations
+                            in one kernel; else element by element from 40,000 rows on when the values
+                            are exactly a hex8 mesh's stiffness; else blocked when the CRS has DOF=3
+                            node blocks and pads little; else CRS rows, with x staged in LDS for the
+                            unpreconditioned FP64 solve from 2^18 rows on), 1 CRS row kernel, 2 blocked, 4 CRS rows with x staged in LDS per
                             row block (FP64, no ILU) */
   int32_t check_every;   /* iterations enqueued between host polls of the stop flag (default 32) */
   int32_t use_graph;     /* capture the polled chunk in a hipGraph (default 1) */
@@ -90,8 +91,8 @@ typedef struct {
   int32_t status;           /* PF_* code of the solve */
   int32_t iterations;       /* BiCGSTAB iterations (FP64 or, for precision 32, FP32) */
   int32_t outer_iterations; /* FP64 residual replacements (mixed), 0 for FP64 */
-  int32_t spmv_kind_used;   /* 1 CRS row kernel, 2 blocked, 4 CRS rows with x staged in LDS, 5 element
-                               by element */
+  int32_t spmv_kind_used;   /* 1 CRS rows, 2 blocked, 4 CRS rows with x staged in LDS, 5 element by
+                               element */
   double rr;                /* final r.r of the recurrence (FP64 form) */
   double rr1;               /* r.r after iteration 1 */
   double true_relres;       /* ||b - A x|| / ||b|| in FP64 after the solve (eliminated system) */
@@ -466,8 +467,8 @@ int pf_system_batch_autotune(pf_system *sys, const pf_solve_opts *opts, int32_t 
  * device), solve_ms (factorization, substitutions and residuals, device). */
 int pf_system_solve_direct(pf_system *sys, int32_t refine, double *x_out, pf_stats *stats);
 
-/* Every mesh of a batch (pf_system_batch_set) in one persistent kernel: one workgroup per mesh
- * from a largest-first queue (cost = n b^2).  mesh_stats (may be NULL): status, iterations
+/* Every mesh of a batch (pf_system_batch_set) in one persistent kernel: a workgroup takes the
+ * next mesh, or its share of a large one, from a largest-first queue (cost = n b^2).  mesh_stats (may be NULL): status, iterations
  * (1 + refine), true_relres, start_ms/end_ms of the mesh's factorization and first
  * substitution.  Returns PF_OK, or the status of the first mesh (in mesh order) that failed. */
 int pf_system_batch_direct(pf_system *sys, int32_t refine, double *x_out, pf_batch_mesh_stats *mesh_stats,

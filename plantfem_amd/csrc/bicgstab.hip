@@ -4,7 +4,7 @@
 //   c1 = r0.r ; y = A p ; c2 = r0.y ; alp = c1/c2 ; e = r - alp y ; v = A e ;
 //   c3 = (e.v)/(v.v) ; x += alp p + c3 e ; r = e - c3 v ; rr = r.r ; stop tests ;
 //   c1 = r0.r ; bet = c1/(c2 c3) ; p = r + bet (p - c3 y)
-// and runs as four kernels:
+// and runs, for systems small enough, in one cooperative kernel (k_persist), else as four kernels:
 //   K1  y = A p                                      partials r0.y
 //   K2  c2, alpha from K1's partials; v = A e with e = r - alpha y formed while gathering
 //                                                    partials e.v, v.v
@@ -21,6 +21,8 @@
 // host enqueues iterations in chunks (one hipGraph per chunk) and polls a pinned copy of
 // the scalars once per chunk.  The redundant loop-top c1 = r0.r of the reference equals
 // the c1 of the previous iteration's end and is not recomputed.  e is never stored.
+// For a hex8 mesh's stiffness K1 and K2 are each two kernels, the element tiles and the node sums
+// (k_el_*), and read no matrix.
 //
 // The same kernels, instantiated for float vectors and matrix values (FP32 SpMV with FP32
 // accumulation) with double partial sums, are the inner solver of the mixed-precision
