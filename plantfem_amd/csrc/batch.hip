@@ -18,7 +18,8 @@
 // workgroups, which meet five times per iteration (Meet) in a cooperative launch.  224 compact meshes of
 // 192 to 20,577 rows: 380 ms with one workgroup per mesh, 150 ms shared, at 3.1 TB/s of matrix; bound
 // now by that stream and, over half of the time, by the meshes that end last.  Without shares no
-// workgroup waits for another, and the queue reset and the kernel are captured in one hipGraph.  Vectors of mesh m live in the DOF range of the mesh inside the union
+// workgroup waits for another, and the queue reset and the kernel are captured in one hipGraph.
+// Vectors of mesh m live in the DOF range of the mesh inside the union
 // vectors, so the gathers of a mesh stay inside its own rows.
 //
 // Launch shapes (chosen by the autotuner): the blocked Sell3 layout with 64-node slices, or

@@ -367,8 +367,9 @@ __device__ inline int progress_failed(const int32_t *progress) {
 // 770 blocks; 84 ms with its two solves before, 26 now); many meshes: the largest one's chain and the
 // stream of the previous b columns that every block rereads.
 template <int BT, bool MF, int MAXT>
-__device__ __forceinline__ int factor_mesh(const DMesh &M, double *band, double *__restrict__ lrow, int share, int shares,
-                           int32_t *progress, double *sL, double *sLi, double *sC, int32_t *sflag) {
+__device__ __forceinline__ int factor_mesh(const DMesh &M, double *band, double *__restrict__ lrow, int share,
+                                           int shares, int32_t *progress, double *sL, double *sLi, double *sC,
+                                           int32_t *sflag) {
   constexpr int W = BT / 64;
   constexpr int U = MAXT <= 4 ? 4 : 2;  // chunks per group of the steady part, two groups in flight
   constexpr int UR = U;                 // chunks per group of the ramp
@@ -722,8 +723,9 @@ __device__ inline double dpp_move(double x) {
 // solves by blocks of 16: 11 ms).  b <= 1024: 1024 threads with one entry each (22.1 ms for 192 meshes up
 // to b = 690) rather than 512 with two (24.8 ms).
 template <int BT, int NR, int DEPTH, bool FWD>
-__device__ __forceinline__ void band_sweep(const DMesh &M, const double *__restrict__ L, const double *__restrict__ dinv,
-                           double *__restrict__ w, double *sw, double *sY) {
+__device__ __forceinline__ void band_sweep(const DMesh &M, const double *__restrict__ L,
+                                           const double *__restrict__ dinv, double *__restrict__ w, double *sw,
+                                           double *sY) {
   const int tid = threadIdx.x;
   const int b = M.b, npad = M.npad, nb = npad / SB;
   const int64_t ld = M.ld;

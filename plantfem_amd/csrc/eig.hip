@@ -185,7 +185,8 @@ __global__ void k_coldots_sum(int cols, const double *__restrict__ part, double 
 }
 
 // partial Gram matrices G = S^T T over row tiles (S, T column-major n x k, k <= GK): 32 rows
-// of both in LDS per step, thread p accumulates pairs p, p + 1024, ...; part[j*k + i][block].  blockIdx.y = 1: S^T T2, its
+// of both in LDS per step, thread p accumulates pairs p, p + 1024, ...; part[j*k + i][block].
+// blockIdx.y = 1: S^T T2, its
 // pairs after the first's (25,704 rows, k = 18: 15.5 us; 22 us as two launches of 256 workgroups)
 constexpr int GK = 96, GR = 32, GPER = (GK * GK + 1023) / 1024;
 __global__ void __launch_bounds__(1024) k_gram(int64_t n, int k, const double *__restrict__ S,
