@@ -344,8 +344,10 @@ __device__ inline void store_tile(const d4 &x, double *__restrict__ band, double
 // the queue, one per workgroup: all of them run.)
 constexpr int SHARE_POLLS = 1 << 22;
 
-__device__ inline int publish_failure(int32_t *progress) {
-  if (threadIdx.x == 0) __hip_atomic_store(progress, -1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+// progress is only read, and only written, where a mesh has several shares
+__device__ inline int publish_failure(int32_t *progress, int shares) {
+  if (shares > 1 && threadIdx.x == 0)
+    __hip_atomic_store(progress, -1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   return PF_NOT_SPD;
 }
 
@@ -464,7 +466,7 @@ __device__ __forceinline__ int factor_mesh(const DMesh &M, double *band, double 
       if (p == 0) {
         if (wv == 0) diag_block(acc[0][0], band, lrow, ld, b, j0, sL, sLi0, sflag);
         __syncthreads();
-        if (uniform(*sflag)) return publish_failure(progress);
+        if (uniform(*sflag)) return publish_failure(progress, shares);
 #pragma unroll
         for (int cq = 0; cq < 4; ++cq) mb0[cq] = sLi0[(4 * cq + q) * LS + jl];
       }
@@ -498,7 +500,7 @@ __device__ __forceinline__ int factor_mesh(const DMesh &M, double *band, double 
       if (p == 0) {
         if (wv == 1) diag_block(acc[0][1], band, lrow, ld, b, j0 + 16, sL, sLi1, sflag);
         __syncthreads();
-        if (uniform(*sflag)) return publish_failure(progress);
+        if (uniform(*sflag)) return publish_failure(progress, shares);
 #pragma unroll
         for (int cq = 0; cq < 4; ++cq) mb1[cq] = sLi1[(4 * cq + q) * LS + jl];
       }
@@ -1339,7 +1341,7 @@ int pf_direct_analyse(pf_ctx *ctx, DirectWork **pd, int64_t n, const int64_t *ro
 
 namespace {
 int launch_direct(pf_ctx *ctx, DirectWork *D, int mode, const double *rhs, double *x, bool mfma) {
-  DArgs a;
+  DArgs a{};
   a.mesh = D->mesh.p;
   a.order = D->order.p;
   a.queue = D->queue.p;
@@ -1352,6 +1354,7 @@ int launch_direct(pf_ctx *ctx, DirectWork *D, int mode, const double *rhs, doubl
   a.x = x;
   a.status = D->status.p;
   a.t_raw = D->t_raw.p;
+  a.progress = D->progress.p;
   a.rows = D->fast_solve ? D->rows.p : nullptr;
   a.dinv = D->fast_solve ? D->dinv.p : nullptr;
   // two workgroups per CU at most; no more workgroups than meshes
@@ -1381,7 +1384,6 @@ int launch_direct(pf_ctx *ctx, DirectWork *D, int mode, const double *rhs, doubl
     a.mode = 2;
     a.item = D->item.p;
     a.nitem = (int32_t)D->hitem.size();
-    a.progress = D->progress.p;
     k_direct_progress_reset<<<pf_blocks(D->nmesh, 256), 256, 0, ctx->stream>>>(D->nmesh, D->progress.p, D->status.p);
     PF_HIP(hipGetLastError());
     if (D->shared) {

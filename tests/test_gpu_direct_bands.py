@@ -75,3 +75,22 @@ def test_bad_pivot_in_a_shared_mesh(ctx, row):
     s.close()
     ref = sl.solveh_banded(lower, rhs, lower=True)
     assert np.linalg.norm(x - ref) <= 2 * 4 * 20 * (kd + 1) * EPS * np.linalg.norm(ref)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("row", [0, 800, 1499])
+@pytest.mark.parametrize("mfma", [True, False])
+def test_bad_pivot_in_a_wide_band(ctx, row, mfma):
+    """Above half bandwidth 1024 one workgroup factors and solves the mesh and has no progress to publish."""
+    from plantfem_amd import _lib as L
+    n, kd = 1500, 1100
+    lower, rp, ci, val, rhs = band_system(n, kd, 4)
+    print("bad pivot, wide", row, mfma, flush=True)
+    bad = val.copy()
+    bad[rp[row] - 1 + min(row, kd)] *= -1.0  # the diagonal entry
+    s = solver(ctx, rp, ci, bad, rhs)
+    s.setDirectKernel(mfma)
+    with pytest.raises(L.PFError) as e:
+        s.solve(algorithm="GaussJordan")
+    assert e.value.code == L.PF_NOT_SPD
+    s.close()
