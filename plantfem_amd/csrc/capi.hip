@@ -698,6 +698,9 @@ static int apply_bc(pf_system *s) {
   return PF_OK;
 }
 
+// the element-by-element product of the current mesh is that of the CRS
+static bool elem_ready(const pf_system *s) { return s->elem_matrix && s->graph_crs && 3 * s->g.nn == s->n; }
+
 static ElemSource elem_source(pf_system *s) {
   return ElemSource{&s->g, s->E.p, s->nu.p, s->jmode, s->has_fix ? s->fixed.p : nullptr,
                     s->rscaled ? s->rscale.p : nullptr};
@@ -753,6 +756,7 @@ extern "C" int pf_system_set_mesh(pf_system *s, int64_t nn, int64_t ne, int32_t 
                                   const int32_t *elemnod) {
   PF_CHECK(sys_check(s, false));
   DeviceGuard guard(s->ctx);
+  s->elem_matrix = false;  // the CRS, if there is one, stays that of the mesh before
   PF_CHECK(set_mesh(s->ctx, s->g, nn, ne, nne, nodcoord, elemnod));
   PF_CHECK(pf_graph_check_mesh(s->ctx, s->g));
   s->has_mesh = true;
@@ -771,6 +775,7 @@ extern "C" int pf_system_zero_matrix(pf_system *s, int32_t dof, int64_t *nnz) {
   }
   pf_ctx *ctx = s->ctx;
   DeviceGuard guard(ctx);
+  s->elem_matrix = false;
   PF_CHECK(pf_graph_node_cols(ctx, s->g));
   s->dof = dof;
   s->n = (int64_t)dof * s->g.nn;
@@ -801,6 +806,7 @@ extern "C" int pf_system_set_crs(pf_system *s, int64_t n, int64_t nnz, const int
   pf_ctx *ctx = s->ctx;
   DeviceGuard guard(ctx);
   const bool resize = (n != s->n);
+  s->elem_matrix = false;
   s->n = n;
   s->nnz = nnz;
   s->dof = 0;
@@ -870,6 +876,7 @@ extern "C" int pf_system_stiffness(pf_system *s, const double *E, const double *
     PF_CHECK(pf_system_zero_matrix(s, 3, nullptr));
   pf_ctx *ctx = s->ctx;
   DeviceGuard guard(ctx);
+  s->elem_matrix = false;  // until the values are those of the new materials
   if (E) {
     PF_CHECK(upload(ctx, s->E, E, (size_t)s->g.ne));
     PF_CHECK(upload(ctx, s->nu, nu, (size_t)s->g.ne));
@@ -893,6 +900,7 @@ extern "C" int pf_system_stiffness_dev(pf_system *s, const double *E_dev, const 
     PF_CHECK(pf_system_zero_matrix(s, 3, nullptr));
   pf_ctx *ctx = s->ctx;
   DeviceGuard guard(ctx);
+  s->elem_matrix = false;
   PF_CHECK(s->E.ensure((size_t)s->g.ne));
   PF_CHECK(s->nu.ensure((size_t)s->g.ne));
   PF_HIP(hipMemcpyAsync(s->E.p, E_dev, sizeof(double) * s->g.ne, hipMemcpyDeviceToDevice, ctx->stream));
@@ -1067,7 +1075,7 @@ extern "C" int pf_system_solve(pf_system *s, const pf_solve_opts *opts, const do
   } else {
     const ElemSource es = elem_source(s);
     PF_CHECK(pf_bicgstab_device(ctx, s->work, s->n, s->row_ptr.p, s->col_idx.p, s->val.p, s->nnz, s->rhs.p,
-                                s->x.p, o, s->matrix_changed, res, s->elem_matrix ? &es : nullptr));
+                                s->x.p, o, s->matrix_changed, res, elem_ready(s) ? &es : nullptr));
     s->matrix_changed = false;
   }
   if (s->has_fix) PF_CHECK(pf_bc_set_fixed_x(ctx, s->n, s->fixed.p, s->ubar.p, s->x.p));
@@ -1265,7 +1273,7 @@ extern "C" int pf_system_elem_apply(pf_system *s, const double *x, double *y) {
   DeviceGuard guard(ctx);
   PF_CHECK(apply_bc(s));
   bool ok = false;
-  if (s->elem_matrix) PF_CHECK(pf_elem_plan(ctx, s->g, &ok));
+  if (elem_ready(s)) PF_CHECK(pf_elem_plan(ctx, s->g, &ok));
   if (!ok) {
     pf_set_error("pf_system_elem_apply: the CRS values are not the stiffness of a hex8 mesh");
     return PF_INVALID;
@@ -1594,6 +1602,7 @@ extern "C" int pf_system_multi_crs(pf_system *s, int32_t dof, int32_t any_overse
   PF_CHECK(check_connects(s, ncon, elem, gauss_point, pair_elem));
   pf_ctx *ctx = s->ctx;
   DeviceGuard guard(ctx);
+  s->elem_matrix = false;
   s->dof = dof;
   s->n = (int64_t)dof * s->g.nn;
   PF_CHECK(s->row_ptr.ensure((size_t)s->n + 1));

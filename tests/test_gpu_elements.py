@@ -168,3 +168,48 @@ def test_solve(mesh, kw):
         assert s.last_stats["status"] == 0 and s.last_stats["true_relres"] < 2e-10
         assert s.last_stats["spmv_kind_used"] == (1 if extra else 5)
     assert np.linalg.norm(out[0] - out[1]) <= 1e-7 * np.linalg.norm(out[1])
+
+
+def _system(nod, el, seed=0):
+    rng = np.random.default_rng(seed)
+    s = fem.FEMSolver()
+    s.setDomain(fem.FEMDomain(nod, el))
+    s.setCRS(DOF=3)
+    s.setStiffness(1e7 * np.exp(0.3 * rng.standard_normal(el.shape[0])), np.full(el.shape[0], 0.3))
+    return s
+
+
+@pytest.mark.parametrize("other", ["same", "larger", "smaller"])
+def test_mesh_replaced_under_the_matrix(other):
+    """A new mesh leaves the CRS as it was: products with it are those of the CRS, never of the new mesh."""
+    nod, el = fem.cube3d(6, 6, 6)
+    s = _system(nod, el)
+    x = np.random.default_rng(1).standard_normal(s.n)
+    y = _apply(s, x)
+    new = {"same": (np.asfortranarray(nod * [1.0, 2.0, 0.5]), el), "larger": fem.cube3d(9, 9, 9),
+           "smaller": fem.cube3d(2, 2, 2)}[other]
+    s.setDomain(fem.FEMDomain(*new))
+    with pytest.raises(L.PFError):
+        _apply(s, x)
+    A = s.getCRS().to_scipy()
+    assert np.all(np.abs(A @ x - y) <= 1e-12 * (abs(A) @ np.abs(x)))
+    s.setCRS(DOF=3)  # and with a stiffness of the new mesh the product is back
+    s.setStiffness(np.full(new[1].shape[0], 1e7), np.full(new[1].shape[0], 0.3))
+    x = np.random.default_rng(2).standard_normal(s.n)
+    A = s.getCRS().to_scipy()
+    assert np.all(np.abs(_apply(s, x) - A @ x) <= 1e-12 * (abs(A) @ np.abs(x)))
+
+
+@pytest.mark.parametrize("precision", [64, 48])
+def test_solve_after_the_mesh_moved(precision):
+    """The solve is that of the stored CRS when the mesh was replaced after the assembly."""
+    nod, el = fem.cube3d(29, 28, 27)  # 73,080 rows: the element form in its range
+    s = _system(nod, el)
+    s.addTraction([-1e300, 1e300, -1e300, 1e300, 1 - 1e-9, 1 + 1e-9], -1e4)
+    base = np.nonzero(nod[:, 2] == 0)[0]
+    s.fix(1, (3 * base[:, None] + np.arange(1, 4)).ravel().astype(np.int32), FixValue=0.0)
+    s.setDomain(fem.FEMDomain(np.asfortranarray(nod * [1.0, 3.0, 0.5]), el))
+    s.relative_er = 1e-10
+    s.solve(precision=precision, stop_mode=1, target_relres=1e-10)
+    assert s.last_stats["status"] == 0 and s.last_stats["true_relres"] < 2e-10
+    assert s.last_stats["spmv_kind_used"] != 5
