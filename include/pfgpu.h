@@ -380,7 +380,8 @@ int pf_system_spmv(pf_system *sys, int32_t kind, const double *x, double *y, int
 int pf_system_elem_apply(pf_system *sys, const double *x, double *y);
 
 /* Device pointers of the system's arrays, for torch interop (valid until the next call
- * that reallocates: set_mesh, zero_matrix, set_crs, destroy). */
+ * that reallocates: set_mesh, zero_matrix, set_crs, multi_crs, destroy).  The caller may write through
+ * them: until such a call, solves use the stored values, never the element-by-element product. */
 typedef struct {
   int64_t n, nnz, nn, ne;
   int64_t *row_ptr;

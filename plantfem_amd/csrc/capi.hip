@@ -647,6 +647,7 @@ struct pf_system {
   bool elem_matrix = false;   // val = the stiffness of g with E, nu, jmode, eliminated by the fixes and
                               // scaled by rscale (if set): the element-by-element product applies it
   bool rscaled = false;
+  bool view_out = false;      // a caller holds pointers to the values and the mesh and may write through them
   DevBuf<double> rscale, rdiag;
   bool ubar_nonzero = false;  // some fixed DOF has a nonzero prescribed value
   // keepThisMatrixAs: named copies of the CRS values (same pattern) and the fix_eig list
@@ -699,7 +700,9 @@ static int apply_bc(pf_system *s) {
 }
 
 // the element-by-element product of the current mesh is that of the CRS
-static bool elem_ready(const pf_system *s) { return s->elem_matrix && s->graph_crs && 3 * s->g.nn == s->n; }
+static bool elem_ready(const pf_system *s) {
+  return s->elem_matrix && !s->view_out && s->graph_crs && 3 * s->g.nn == s->n;
+}
 
 static ElemSource elem_source(pf_system *s) {
   return ElemSource{&s->g, s->E.p, s->nu.p, s->jmode, s->has_fix ? s->fixed.p : nullptr,
@@ -763,6 +766,7 @@ extern "C" int pf_system_set_mesh(pf_system *s, int64_t nn, int64_t ne, int32_t 
   s->has_mat = false;
   s->graph_crs = false;
   s->multi_crs = false;
+  s->view_out = false;
   ++s->pattern_version;
   return PF_OK;
 }
@@ -793,6 +797,7 @@ extern "C" int pf_system_zero_matrix(pf_system *s, int32_t dof, int64_t *nnz) {
   PF_HIP(hipStreamSynchronize(ctx->stream));
   s->graph_crs = true;
   s->multi_crs = false;
+  s->view_out = false;
   ++s->pattern_version;
   mark_changed(s);
   if (nnz) *nnz = s->nnz;
@@ -822,6 +827,7 @@ extern "C" int pf_system_set_crs(pf_system *s, int64_t n, int64_t nnz, const int
   PF_HIP(hipStreamSynchronize(ctx->stream));
   s->graph_crs = false;
   s->multi_crs = false;
+  s->view_out = false;
   ++s->pattern_version;
   mark_changed(s);
   return PF_OK;
@@ -1233,7 +1239,8 @@ extern "C" int pf_system_get_x(pf_system *s, double *x) {
 extern "C" int pf_system_view_get(pf_system *s, pf_system_view *v) {
   PF_CHECK(sys_check(s, false));
   if (!v) return PF_INVALID;
-  s->elem_matrix = false;  // the caller may write the values
+  s->view_out = true;
+  s->g.elem.tried = s->g.elem.ok = false;  // tiles of the mesh as the caller leaves it
   v->n = s->n;
   v->nnz = s->nnz;
   v->nn = s->g.nn;
@@ -1640,6 +1647,7 @@ extern "C" int pf_system_multi_crs(pf_system *s, int32_t dof, int32_t any_overse
   PF_HIP(hipStreamSynchronize(ctx->stream));
   s->graph_crs = false;
   s->multi_crs = true;
+  s->view_out = false;
   ++s->pattern_version;
   mark_changed(s);
   if (nnz) *nnz = s->nnz;

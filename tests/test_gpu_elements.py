@@ -10,6 +10,8 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 
+torch = pytest.importorskip("torch")  # its HIP runtime starts before the library's
+
 from plantfem_amd import _lib as L  # noqa: E402
 from plantfem_amd import fem, workloads  # noqa: E402
 
@@ -213,3 +215,44 @@ def test_solve_after_the_mesh_moved(precision):
     s.solve(precision=precision, stop_mode=1, target_relres=1e-10)
     assert s.last_stats["status"] == 0 and s.last_stats["true_relres"] < 2e-10
     assert s.last_stats["spmv_kind_used"] != 5
+
+
+def _array(ptr, count):
+    """A torch tensor over device memory (float64)."""
+    class Mem:
+        __cuda_array_interface__ = {"shape": (count,), "typestr": "<f8", "version": 2,
+                                    "data": (C.cast(ptr, C.c_void_p).value, False)}
+
+    return torch.as_tensor(Mem(), device="cuda")
+
+
+@pytest.mark.parametrize("precision", [64, 48])
+def test_writes_through_an_earlier_view(precision):
+    """Values and coordinates written through a view that was taken before the assembly count."""
+    nod, el = fem.cube3d(29, 28, 27)
+    s = _system(nod, el)
+    _apply(s, np.ones(s.n))  # the tiles of the mesh as it is
+    v = L.SystemView()
+    L.check(L.load().pf_system_view_get(s.h, C.byref(v)), "view")
+    top = [-1e300, 1e300, -1e300, 1e300, 1 - 1e-9, 1 + 1e-9]
+    base = np.nonzero(nod[:, 2] == 0)[0]
+    ids = (3 * base[:, None] + np.arange(1, 4)).ravel().astype(np.int32)
+    s.relative_er = 1e-10
+    s.addTraction(top, -1e4)
+    s.fix(1, ids, FixValue=0.0)
+    _array(v.nodcoord, 3 * nod.shape[0])[: nod.shape[0]] *= 2.0  # x of every node
+    torch.cuda.synchronize()
+    s.setStiffness()
+    _array(v.val, int(v.nnz)).mul_(3.0)
+    torch.cuda.synchronize()
+    with pytest.raises(L.PFError):
+        _apply(s, np.ones(s.n))
+    s.solve(precision=precision, stop_mode=1, target_relres=1e-10)
+    assert s.last_stats["status"] == 0 and s.last_stats["true_relres"] < 2e-10
+    assert s.last_stats["spmv_kind_used"] != 5
+    # the pointers end with the CRS; the tiles are then those of the moved nodes
+    s.setCRS(DOF=3)
+    s.setStiffness()
+    x = np.random.default_rng(2).standard_normal(s.n)
+    A = s.getCRS().to_scipy()
+    assert np.all(np.abs(_apply(s, x) - A @ x) <= 1e-11 * (abs(A) @ np.abs(x)))
