@@ -116,6 +116,14 @@ int pf_ctx_synchronize(pf_ctx *ctx);
 /* The context's HIP stream (hipStream_t as void*), for callers that order their own work. */
 void *pf_ctx_stream(pf_ctx *ctx);
 
+/* How the last solves on this context ran, for tests and measurements. */
+typedef struct {
+  int32_t one_kernel;    /* last BiCGSTAB solve of one system: 1 all iterations in one kernel, 0 by launches */
+  int32_t batch_shares;  /* last batched BiCGSTAB: most workgroups that shared a mesh (1: none did) */
+  int32_t direct_shares; /* last direct factorization: the same */
+} pf_forms;
+int pf_ctx_forms(pf_ctx *ctx, pf_forms *forms);
+
 /* ---- stateless host-pointer entry points ---------------------------------------- */
 
 /* ZeroMatrix_as_CRS_FEMDomain(DOF) (FEMDomainClass.f90:10581-10840): CRS graph of the

@@ -80,6 +80,13 @@ class Stats(C.Structure):
         return {k: getattr(self, k) for k, _ in self._fields_}
 
 
+class Forms(C.Structure):
+    _fields_ = [("one_kernel", C.c_int32), ("batch_shares", C.c_int32), ("direct_shares", C.c_int32)]
+
+    def as_dict(self) -> dict:
+        return {k: getattr(self, k) for k, _ in self._fields_}
+
+
 class SystemView(C.Structure):
     _fields_ = [
         ("n", C.c_int64), ("nnz", C.c_int64), ("nn", C.c_int64), ("ne", C.c_int64),
@@ -125,6 +132,7 @@ SIGNATURES = {
     "pf_ctx_destroy": (C.c_int, [P]),
     "pf_ctx_synchronize": (C.c_int, [P]),
     "pf_ctx_stream": (P, [P]),
+    "pf_ctx_forms": (C.c_int, [P, C.POINTER(Forms)]),
     "pf_crs_graph": (C.c_int, [P, I64, I64, I32, PI32, I32, PI64, PI64, PI32]),
     "pf_hex8_stiffness": (C.c_int, [P, I64, I64, PF64, PI32, PF64, PF64, I32, I64, I64, PF64]),
     "pf_hex8_stiffness_crs": (C.c_int, [P, I64, I64, PF64, PI32, PF64, PF64, I32, PI64, PI32, PF64]),
@@ -267,6 +275,12 @@ class Context:
 
     def synchronize(self):
         check(load().pf_ctx_synchronize(self.h), "pf_ctx_synchronize")
+
+    def forms(self) -> dict:
+        """How the last solves on this context ran (pf_forms)."""
+        f = Forms()
+        check(load().pf_ctx_forms(self.h, C.byref(f)), "pf_ctx_forms")
+        return f.as_dict()
 
     def close(self):
         if getattr(self, "h", None):

@@ -1058,6 +1058,8 @@ int pf_batch_solve_device(pf_ctx *ctx, BatchWork *b, const int64_t *row_ptr, con
   const BArgs a = make_args(b, row_ptr, col_idx, val, rhs, x, o, mixed);
   float ms = 0.f;
   PF_CHECK(run_batch(ctx, b, a, t, mixed, o.use_graph != 0, &ms));
+  ctx->forms.batch_shares = 1;
+  for (const BItem &it : b->hitem) ctx->forms.batch_shares = std::max(ctx->forms.batch_shares, it.G);
   // per-mesh results; wall-clock ticks -> ms from the first mesh's start
   std::vector<pf_batch_mesh_stats> st(b->nmesh);
   std::vector<int64_t> raw(2 * (size_t)b->nmesh);

@@ -1944,6 +1944,7 @@ int pf_bicgstab_device(pf_ctx *ctx, SolverWork *w, int64_t n, const int64_t *row
   PF_CHECK(w->sc.ensure(2));
   PF_CHECK(w->flag.ensure(1));
   PF_CHECK(w->part.ensure((size_t)ctx->num_cus * 8 * PART_SLOTS + 16));
+  ctx->forms.one_kernel = 0;
 
   PF_HIP(hipEventRecord(ctx->ev0, ctx->stream));
   const double avg_row = (double)nnz / (double)n;
@@ -2113,6 +2114,7 @@ int pf_bicgstab_device(pf_ctx *ctx, SolverWork *w, int64_t n, const int64_t *row
       PF_CHECK(w->xstart.ensure(n));
       PF_HIP(hipMemcpyAsync(w->xstart.p, x, sizeof(double) * n, hipMemcpyDeviceToDevice, ctx->stream));
       PF_CHECK(run_persist(ctx, w, n, row_ptr, val, x, o, &ran));
+      ctx->forms.one_kernel = ran;
       if (!ran) {  // from the start again, by launches
         PF_HIP(hipMemcpyAsync(x, w->xstart.p, sizeof(double) * n, hipMemcpyDeviceToDevice, ctx->stream));
         PF_CHECK(prepare_scalars(ctx, w, 0, o, o.itrmax, o.relative_er, kmode, 0, guard));

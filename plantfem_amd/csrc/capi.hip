@@ -196,6 +196,13 @@ extern "C" int pf_ctx_synchronize(pf_ctx *ctx) {
 
 extern "C" void *pf_ctx_stream(pf_ctx *ctx) { return ctx ? (void *)ctx->stream : nullptr; }
 
+extern "C" int pf_ctx_forms(pf_ctx *ctx, pf_forms *forms) {
+  PF_CHECK(check_ctx(ctx));
+  if (!forms) return PF_INVALID;
+  *forms = ctx->forms;
+  return PF_OK;
+}
+
 // ====================================================================== stateless calls
 extern "C" int pf_crs_graph(pf_ctx *ctx, int64_t nn, int64_t ne, int32_t nne, const int32_t *elemnod, int32_t dof,
                             int64_t *nnz, int64_t *row_ptr, int32_t *col_idx) {

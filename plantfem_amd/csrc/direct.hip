@@ -1407,6 +1407,9 @@ int launch_direct(pf_ctx *ctx, DirectWork *D, int mode, const double *rhs, doubl
     void *args[] = {&a};
     PF_HIP(hipLaunchKernel(kernel, dim3(grid), dim3(DBT), args, 0, ctx->stream));
   }
+  ctx->forms.direct_shares = 1;
+  if (D->fast_solve)
+    for (const DItem &it : D->hitem) ctx->forms.direct_shares = std::max(ctx->forms.direct_shares, it.G);
   if (D->fast_solve) {
     const unsigned per = (unsigned)((D->maxpad / SB + 3) / 4);
     k_diag_inverse<<<dim3(per, (unsigned)D->nmesh), 4 * SB, 0, ctx->stream>>>(D->nmesh, D->mesh.p, D->status.p,

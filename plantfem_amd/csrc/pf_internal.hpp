@@ -35,6 +35,7 @@ struct pf_ctx {
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   int num_cus = 256;
   SolverWork *work = nullptr;  // workspace of the stateless solver entry point
+  pf_forms forms{};            // how the last solves ran
 };
 
 // ---------------------------------------------------------------------------------

@@ -25,6 +25,7 @@ def test_shared_meshes(ctx, precision, tune):
     print("shared batch", precision, tune, flush=True)
     for again in range(2):  # the second solve starts from the first one's meeting counters
         x, st = s.solveBatch(precision=precision, tune=tune, stop_mode=1, target_relres=REL)
+        assert ctx.forms()["batch_shares"] > 1
     s.close()
     for m, o in enumerate(organs):
         rp, ci, val, rhs = organ_system(o)
@@ -46,6 +47,7 @@ def test_one_shared_mesh_matches_the_single_solver(ctx):
     s.relative_er = REL
     print("one shared mesh", flush=True)
     x, st = s.solveBatch(stop_mode=1)
+    assert ctx.forms()["batch_shares"] > 1
     s.close()
     rp, ci, val, rhs = organ_system(o)
     A = to_scipy(rp, ci, val)

@@ -47,6 +47,7 @@ def test_band_solve(ctx, n, kd, mfma):
     s = solver(ctx, rp, ci, val, rhs)
     s.setDirectKernel(mfma)
     x = s.solve(algorithm="GaussJordan", refine=0)
+    assert (ctx.forms()["direct_shares"] > 1) == (n > 32 and kd <= 1024)
     assert s.directInfo()["bandwidth"] <= kd
     s.close()
     ref = sl.solveh_banded(lower, rhs, lower=True)
@@ -67,7 +68,7 @@ def test_bad_pivot_in_a_shared_mesh(ctx, row):
     s = solver(ctx, rp, ci, bad, rhs)
     with pytest.raises(L.PFError) as e:
         s.solve(algorithm="GaussJordan")
-    assert e.value.code == L.PF_NOT_SPD
+    assert e.value.code == L.PF_NOT_SPD and ctx.forms()["direct_shares"] > 1
     from plantfem_amd.fem import CRS
     s.setCRS(CRS=CRS(rp, ci, val))
     s.setRHS(rhs)
@@ -92,5 +93,5 @@ def test_bad_pivot_in_a_wide_band(ctx, row, mfma):
     s.setDirectKernel(mfma)
     with pytest.raises(L.PFError) as e:
         s.solve(algorithm="GaussJordan")
-    assert e.value.code == L.PF_NOT_SPD
+    assert e.value.code == L.PF_NOT_SPD and ctx.forms()["direct_shares"] == 1
     s.close()

@@ -8,7 +8,12 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 
+from plantfem_amd import _lib as L  # noqa: E402
 from plantfem_amd.fem import FEMDomain, FEMSolver, bicgstab_crs, cube3d  # noqa: E402
+
+
+def _one_kernel():
+    return L.default_context().forms()["one_kernel"]
 
 
 def _crs(rows):
@@ -29,7 +34,7 @@ def _matrix(kind, n, seed=0):
         elif kind == "long":  # a few rows of hundreds of entries among short ones
             m = 700 if i % 97 == 5 else 4
             cols = [c for c in rng.integers(max(0, i - 800), min(n, i + 800), m) if c != i]
-        else:  # scattered: more distinct columns per workgroup than it stages (the launches run)
+        else:  # scattered: from 8000 rows on more distinct columns per workgroup than it stages
             cols = [c for c in rng.integers(0, n, 90) if c != i]
         row = {int(c): float(rng.uniform(-1, 1)) for c in cols}
         row[i] = 1.5 * sum(abs(v) for v in row.values()) + 1.0
@@ -60,6 +65,21 @@ def test_general_matrices(kind, n, x0):
         x, st = bicgstab_crs(*crs, b, x0=start, stop_mode=1, relative_er=1e-12, spmv_kind=k)
         assert st["status"] == 0 and st["true_relres"] < 1e-11
         assert np.linalg.norm(x - ref) <= 1e-9 * np.linalg.norm(ref), (k, st)
+        # launches below 64 rows, and where a workgroup's 2048 entries are more than 512 rows (three per row)
+        assert _one_kernel() == (k == 0 and n >= 64 and not (kind == "tridiagonal" and n > 512))
+
+
+def test_too_many_columns():
+    """More distinct columns per workgroup than it stages: the launches run."""
+    n = 8000
+    crs = _crs(_matrix("scattered", n))
+    b = np.random.default_rng(4).standard_normal(n)
+    out = []
+    for k in (0, 1):
+        x, st = bicgstab_crs(*crs, b, stop_mode=1, relative_er=1e-12, spmv_kind=k)
+        assert st["status"] == 0 and st["true_relres"] < 1e-11 and _one_kernel() == 0
+        out.append(x)
+    assert np.linalg.norm(out[0] - out[1]) <= 1e-9 * np.linalg.norm(out[1])
 
 
 @pytest.mark.parametrize("mode", [0, 1, 2])
@@ -69,6 +89,7 @@ def test_stop_rules_and_counts(mode):
     b = np.random.default_rng(2).standard_normal(2000)
     kw = {"stop_mode": mode, "relative_er": 1e-10, "er0": 1e-20 if mode == 2 else 1e-300}
     x0, s0 = bicgstab_crs(*crs, b, spmv_kind=0, **kw)
+    assert _one_kernel() == 1
     x1, s1 = bicgstab_crs(*crs, b, spmv_kind=1, **kw)
     assert s0["status"] == s1["status"] == 0 and s0["iterations"] == s1["iterations"]
     assert np.linalg.norm(x0 - x1) <= 1e-9 * np.linalg.norm(x1)
@@ -89,6 +110,7 @@ def test_empty_rows_and_zero_rhs():
     keep = np.arange(900) % 7 != 0
     b = np.where(keep, np.random.default_rng(3).standard_normal(900), 0.0)
     x, st = bicgstab_crs(*_crs(rows), b, stop_mode=1, relative_er=1e-12)
+    assert _one_kernel() == 1
     ref = np.zeros(900)
     ref[keep] = np.linalg.solve(_dense(rows)[np.ix_(keep, keep)], b[keep])
     assert st["status"] == 0 and np.linalg.norm(x - ref) <= 1e-9 * np.linalg.norm(ref)
@@ -104,6 +126,7 @@ def test_breakdown_and_nan():
         for k in (0, 1):
             x, st = bicgstab_crs(*_crs(rows), np.ones(n), spmv_kind=k, er0=0.0, relative_er=0.0)
             assert st["status"] == 1 and st["iterations"] == 1 and not x.any(), (k, st)
+            assert _one_kernel() == (k == 0 and n == 100)  # of 5000 rows with one entry each a workgroup gets 2048
         b = np.ones(n)
         b[n // 2] = np.nan
         x, st = bicgstab_crs(*_crs(rows), b, stop_mode=1, relative_er=1e-10, itrmax=50)
@@ -123,5 +146,6 @@ def test_same_on_every_run(dims):
         base = np.nonzero(nod[:, 2] == 0)[0]
         s.fix(1, (3 * base[:, None] + np.arange(1, 4)).ravel().astype(np.int32), FixValue=0.0)
         out.append(s.solve())
+        assert _one_kernel() == 1
         assert s.last_stats["status"] == 0 and s.last_stats["true_relres"] < 1e-8
     assert np.array_equal(out[0], out[1]) and np.array_equal(out[0], out[2])
