@@ -124,6 +124,11 @@ typedef struct {
 } pf_forms;
 int pf_ctx_forms(pf_ctx *ctx, pf_forms *forms);
 
+/* Some solves run workgroups that wait for each other (all iterations in one kernel, meshes shared by
+ * several workgroups).  allow 0: the context refuses such launches and runs the forms without waits;
+ * 1 (default): they run where all workgroups fit the card together. */
+int pf_ctx_together(pf_ctx *ctx, int32_t allow);
+
 /* ---- stateless host-pointer entry points ---------------------------------------- */
 
 /* ZeroMatrix_as_CRS_FEMDomain(DOF) (FEMDomainClass.f90:10581-10840): CRS graph of the

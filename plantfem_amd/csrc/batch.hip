@@ -755,8 +755,7 @@ int launch_one(pf_ctx *ctx, const BArgs &a, unsigned grid, bool shared) {
   if (shared) {
     BArgs arg = a;
     void *args[] = {&arg};
-    if (hipLaunchCooperativeKernel((const void *)k_batch<PREC, L, SUB, BTB>, dim3(grid), dim3(BTB), args, 0,
-                                   ctx->stream) == hipSuccess)
+    if (pf_launch_together(ctx, (const void *)k_batch<PREC, L, SUB, BTB>, grid, BTB, args, 0) == hipSuccess)
       return PF_OK;
     (void)hipGetLastError();
     return PF_BATCH_WHOLE;

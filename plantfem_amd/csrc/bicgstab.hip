@@ -1658,7 +1658,7 @@ int run_persist(pf_ctx *ctx, SolverWork *w, int64_t n, const int64_t *row_ptr, c
     hipError_t e = hipSuccess;
     if (lds > 64 * 1024) e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e == hipSuccess)
-      e = hipLaunchCooperativeKernel(kernel, dim3((unsigned)p.G), dim3(PT), args, (unsigned)lds, ctx->stream);
+      e = pf_launch_together(ctx, kernel, (unsigned)p.G, PT, args, lds);
     if (e != hipSuccess) {  // e.g. fewer CUs available to this process: the launches then
       (void)hipGetLastError();
       return PF_OK;

@@ -203,6 +203,12 @@ extern "C" int pf_ctx_forms(pf_ctx *ctx, pf_forms *forms) {
   return PF_OK;
 }
 
+extern "C" int pf_ctx_together(pf_ctx *ctx, int32_t allow) {
+  PF_CHECK(check_ctx(ctx));
+  ctx->together = allow != 0;
+  return PF_OK;
+}
+
 // ====================================================================== stateless calls
 extern "C" int pf_crs_graph(pf_ctx *ctx, int64_t nn, int64_t ne, int32_t nne, const int32_t *elemnod, int32_t dof,
                             int64_t *nnz, int64_t *row_ptr, int32_t *col_idx) {

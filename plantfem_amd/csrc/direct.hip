@@ -1390,7 +1390,7 @@ int launch_direct(pf_ctx *ctx, DirectWork *D, int mode, const double *rhs, doubl
       // the shares of a mesh wait for each other: all workgroups resident
       const int g2 = std::min((int)D->hitem.size(), ctx->num_cus);
       void *args[] = {&a};
-      if (hipLaunchCooperativeKernel(kernel, dim3(g2), dim3(DBT), args, 0, ctx->stream) != hipSuccess) {
+      if (pf_launch_together(ctx, kernel, (unsigned)g2, DBT, args, 0) != hipSuccess) {
         (void)hipGetLastError();  // whole meshes then
         std::vector<DItem> whole;
         for (const DItem &it : D->hitem)

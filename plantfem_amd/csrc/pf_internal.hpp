@@ -36,7 +36,16 @@ struct pf_ctx {
   int num_cus = 256;
   SolverWork *work = nullptr;  // workspace of the stateless solver entry point
   pf_forms forms{};            // how the last solves ran
+  bool together = true;        // kernels whose workgroups wait for each other may be launched
 };
+
+// cooperative launch of a kernel whose workgroups wait for each other; refused like one that does not
+// fit the card where the context does not allow it
+inline hipError_t pf_launch_together(pf_ctx *ctx, const void *kernel, unsigned grid, unsigned block, void **args,
+                                     size_t lds) {
+  if (!ctx->together) return hipErrorCooperativeLaunchTooLarge;
+  return hipLaunchCooperativeKernel(kernel, dim3(grid), dim3(block), args, (unsigned)lds, ctx->stream);
+}
 
 // ---------------------------------------------------------------------------------
 // device buffer: owns a hipMalloc'd array; grows, never shrinks

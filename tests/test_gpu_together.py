@@ -1,0 +1,84 @@
+"""Solves whose workgroups wait for each other, on a context that refuses such launches: the same
+systems by launches (plantfem_amd/csrc/bicgstab.hip) and with whole meshes (batch.hip, direct.hip)."""
+
+import numpy as np
+import pytest
+import scipy.linalg as sl
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")  # its HIP runtime starts before the library's
+
+from plantfem_amd import _lib as L  # noqa: E402
+from plantfem_amd import batch as B  # noqa: E402
+from plantfem_amd.fem import bicgstab_crs  # noqa: E402
+from test_direct import organ_system, relres, rounding_floor, to_scipy  # noqa: E402
+from test_gpu_direct_bands import EPS, band_system, solver  # noqa: E402
+from test_gpu_one_kernel import _crs, _matrix  # noqa: E402
+
+REL = 1e-9
+
+
+@pytest.fixture
+def alone():
+    c = L.Context(0)
+    c.together(False)
+    yield c
+    c.close()
+
+
+@pytest.mark.parametrize("x0", [False, True])
+def test_one_kernel_refused(alone, x0):
+    crs = _crs(_matrix("ragged", 3000))
+    rng = np.random.default_rng(1)
+    b = rng.standard_normal(3000)
+    start = rng.standard_normal(3000) if x0 else None
+    kw = {"x0": start, "ctx": alone, "stop_mode": 1, "relative_er": 1e-12}
+    x, st = bicgstab_crs(*crs, b, **kw)
+    assert alone.forms()["one_kernel"] == 0 and st["status"] == 0
+    y, sy = bicgstab_crs(*crs, b, spmv_kind=1, **kw)  # the same launches
+    assert np.array_equal(x, y) and st["iterations"] == sy["iterations"]
+
+
+@pytest.mark.parametrize("precision", [64, 32])
+def test_batch_shares_refused(alone, precision):
+    rng = np.random.default_rng(11)
+    organs = [B.block(n, rng) for n in (3, 13, 10, 5, 11)]
+    u = B.union(organs)
+    s = B.build_solver(u, alone)
+    s.relative_er = REL
+    print("whole meshes", precision, flush=True)
+    out = []
+    for _ in range(3):  # the first solve is refused, the others start with whole meshes (and a graph)
+        x, st = s.solveBatch(precision=precision, stop_mode=1, target_relres=REL)
+        assert alone.forms()["batch_shares"] == 1
+        out.append(x)
+    s.close()
+    assert np.array_equal(out[0], out[1]) and np.array_equal(out[0], out[2])
+    for m, o in enumerate(organs):
+        rp, ci, val, rhs = organ_system(o)
+        A, xm = to_scipy(rp, ci, val), out[0][u.dof_range(m)]
+        assert st["status"][m] == 0
+        assert relres(A, xm, rhs) <= REL * (1.0 if precision == 32 else 1.5) + rounding_floor(A, xm, rhs)
+
+
+@pytest.mark.parametrize("bad", [None, 700])
+def test_direct_shares_refused(alone, bad):
+    n, kd = 1499, 300
+    lower, rp, ci, val, rhs = band_system(n, kd, 3)
+    print("whole mesh", bad, flush=True)
+    if bad is not None:
+        v = val.copy()
+        v[rp[bad] - 1 + min(bad, kd)] *= -1.0  # the diagonal entry
+        s = solver(alone, rp, ci, v, rhs)
+        with pytest.raises(L.PFError) as e:
+            s.solve(algorithm="GaussJordan")
+        assert e.value.code == L.PF_NOT_SPD
+    else:
+        s = solver(alone, rp, ci, val, rhs)
+        ref = sl.solveh_banded(lower, rhs, lower=True)
+        for _ in range(2):  # the second solve keeps the factor
+            x = s.solve(algorithm="GaussJordan", refine=0)
+            assert np.linalg.norm(x - ref) <= 2 * 4 * 20 * (kd + 1) * EPS * np.linalg.norm(ref)
+    assert alone.forms()["direct_shares"] == 1
+    s.close()
