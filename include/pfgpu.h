@@ -126,8 +126,9 @@ int pf_ctx_forms(pf_ctx *ctx, pf_forms *forms);
 
 /* Some solves run workgroups that wait for each other (all iterations in one kernel, meshes shared by
  * several workgroups).  allow 0: the context refuses such launches and runs the forms without waits;
- * 1 (default): they run where all workgroups fit the card together. */
-int pf_ctx_together(pf_ctx *ctx, int32_t allow);
+ * 1 (default): they run where all workgroups fit the card together.  Every wait ends after `polls` polls
+ * (0, the default: seconds at most); a solve with a wait that ended so is done again without waits. */
+int pf_ctx_together(pf_ctx *ctx, int32_t allow, int32_t polls);
 
 /* ---- stateless host-pointer entry points ---------------------------------------- */
 

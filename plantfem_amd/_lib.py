@@ -133,7 +133,7 @@ SIGNATURES = {
     "pf_ctx_synchronize": (C.c_int, [P]),
     "pf_ctx_stream": (P, [P]),
     "pf_ctx_forms": (C.c_int, [P, C.POINTER(Forms)]),
-    "pf_ctx_together": (C.c_int, [P, I32]),
+    "pf_ctx_together": (C.c_int, [P, I32, I32]),
     "pf_crs_graph": (C.c_int, [P, I64, I64, I32, PI32, I32, PI64, PI64, PI32]),
     "pf_hex8_stiffness": (C.c_int, [P, I64, I64, PF64, PI32, PF64, PF64, I32, I64, I64, PF64]),
     "pf_hex8_stiffness_crs": (C.c_int, [P, I64, I64, PF64, PI32, PF64, PF64, I32, PI64, PI32, PF64]),
@@ -283,9 +283,9 @@ class Context:
         check(load().pf_ctx_forms(self.h, C.byref(f)), "pf_ctx_forms")
         return f.as_dict()
 
-    def together(self, allow: bool = True):
-        """Allow or refuse kernels whose workgroups wait for each other (pf_ctx_together)."""
-        check(load().pf_ctx_together(self.h, int(allow)), "pf_ctx_together")
+    def together(self, allow: bool = True, polls: int = 0):
+        """Allow or refuse kernels whose workgroups wait for each other, and bound the waits (pf_ctx_together)."""
+        check(load().pf_ctx_together(self.h, int(allow), int(polls)), "pf_ctx_together")
 
     def close(self):
         if getattr(self, "h", None):

@@ -203,9 +203,14 @@ extern "C" int pf_ctx_forms(pf_ctx *ctx, pf_forms *forms) {
   return PF_OK;
 }
 
-extern "C" int pf_ctx_together(pf_ctx *ctx, int32_t allow) {
+extern "C" int pf_ctx_together(pf_ctx *ctx, int32_t allow, int32_t polls) {
   PF_CHECK(check_ctx(ctx));
+  if (polls < 0) {
+    pf_set_error("pf_ctx_together: polls must not be negative");
+    return PF_INVALID;
+  }
   ctx->together = allow != 0;
+  ctx->polls = polls;
   return PF_OK;
 }
 

@@ -67,6 +67,7 @@ struct DArgs {
   const DItem *item;     // factorization: queue of shares, those of a mesh adjacent
   int32_t nitem;
   int32_t *progress;     // per mesh: blocks of 32 columns complete (-1: not positive definite, -2: gave up)
+  int32_t polls;         // of a share for the preceding block before it gives up
   int32_t *queue;
   int32_t nmesh;
   int32_t mode;          // 0: factor, then solve x = A^-1 rhs; 1: solve only, x += A^-1 rhs; 2: factor only
@@ -341,8 +342,9 @@ __device__ inline void store_tile(const d4 &x, double *__restrict__ band, double
 
 // s_sleep(1) polls of a share for the preceding block before it gives up: seconds, against the
 // microseconds that a block takes.  (The launch is cooperative and the shares are the first items of
-// the queue, one per workgroup: all of them run.)
-constexpr int SHARE_POLLS = 1 << 22;
+// the queue, one per workgroup: all of them run.  Where they do not all the same, the mesh is factored
+// again by one workgroup.)
+constexpr int32_t SHARE_POLLS = 1 << 22;
 
 // progress is only read, and only written, where a mesh has several shares
 __device__ inline int publish_failure(int32_t *progress, int shares) {
@@ -370,8 +372,8 @@ __device__ inline int progress_failed(const int32_t *progress) {
 // stream of the previous b columns that every block rereads.
 template <int BT, bool MF, int MAXT>
 __device__ __forceinline__ int factor_mesh(const DMesh &M, double *band, double *__restrict__ lrow, int share,
-                                           int shares, int32_t *progress, double *sL, double *sLi, double *sC,
-                                           int32_t *sflag) {
+                                           int shares, int32_t *progress, int32_t polls_max, double *sL,
+                                           double *sLi, double *sC, int32_t *sflag) {
   constexpr int W = BT / 64;
   constexpr int U = MAXT <= 4 ? 4 : 2;  // chunks per group of the steady part, two groups in flight
   constexpr int UR = U;                 // chunks per group of the ramp
@@ -390,7 +392,7 @@ __device__ __forceinline__ int factor_mesh(const DMesh &M, double *band, double 
     if (threadIdx.x == 0) {
       int p, polls = 0;
       while ((p = __hip_atomic_load(progress, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) >= 0 && 32 * p < want &&
-             ++polls < SHARE_POLLS)
+             ++polls < polls_max)
         __builtin_amdgcn_s_sleep(1);
       if (p >= 0 && 32 * p < want) {  // the other shares never came: nobody may wait for this one
         p = -2;
@@ -517,8 +519,13 @@ __device__ __forceinline__ int factor_mesh(const DMesh &M, double *band, double 
     }
     if (shares > 1) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // every wave's part of the block is out
     __syncthreads();
-    if (shares > 1 && threadIdx.x == 0)
-      __hip_atomic_store(progress, j0 / 32 + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+    if (shares > 1 && threadIdx.x == 0) {
+      // the blocks complete in order, so the mesh stands at this one unless a share gave up meanwhile: that
+      // stays (the next wait finds it), or the others would wait out their bounds one after the other
+      int32_t at = j0 / 32;
+      (void)__hip_atomic_compare_exchange_strong(progress, &at, j0 / 32 + 1, __ATOMIC_RELEASE, __ATOMIC_RELAXED,
+                                                 __HIP_MEMORY_SCOPE_AGENT);
+    }
   }
   return PF_OK;
 }
@@ -643,7 +650,7 @@ __global__ void __launch_bounds__(BT) k_direct(DArgs a) {
     const int64_t t0 = wall_clock64();
     double *band = a.band + M.boff;
     int st = a.mode != 1 ? factor_mesh<BT, MF, MAXT>(M, band, a.rows ? a.rows + M.boff : nullptr, it.g, it.G,
-                                               a.progress + m, sL, sLi, sC, sflag)
+                                               a.progress + m, a.polls, sL, sLi, sC, sflag)
                          : a.status[m];
     if (a.mode == 2) {
       // the share of the last block reports for the mesh, the first one for its start
@@ -1340,6 +1347,18 @@ int pf_direct_analyse(pf_ctx *ctx, DirectWork **pd, int64_t n, const int64_t *ro
 }
 
 namespace {
+// from now on (until the next analysis) every mesh is factored by one workgroup
+int whole_meshes(pf_ctx *ctx, DirectWork *D) {
+  std::vector<DItem> whole;
+  for (const DItem &it : D->hitem)
+    if (it.g == 0) whole.push_back(DItem{it.m, 0, 1, 0});
+  D->hitem = whole;
+  D->shared = false;
+  PF_HIP(hipMemcpyAsync(D->item.p, D->hitem.data(), sizeof(DItem) * D->hitem.size(), hipMemcpyHostToDevice,
+                        ctx->stream));
+  return PF_OK;
+}
+
 int launch_direct(pf_ctx *ctx, DirectWork *D, int mode, const double *rhs, double *x, bool mfma) {
   DArgs a{};
   a.mesh = D->mesh.p;
@@ -1355,6 +1374,7 @@ int launch_direct(pf_ctx *ctx, DirectWork *D, int mode, const double *rhs, doubl
   a.status = D->status.p;
   a.t_raw = D->t_raw.p;
   a.progress = D->progress.p;
+  a.polls = ctx->polls > 0 ? ctx->polls : SHARE_POLLS;
   a.rows = D->fast_solve ? D->rows.p : nullptr;
   a.dinv = D->fast_solve ? D->dinv.p : nullptr;
   // two workgroups per CU at most; no more workgroups than meshes
@@ -1391,14 +1411,8 @@ int launch_direct(pf_ctx *ctx, DirectWork *D, int mode, const double *rhs, doubl
       const int g2 = std::min((int)D->hitem.size(), ctx->num_cus);
       void *args[] = {&a};
       if (pf_launch_together(ctx, kernel, (unsigned)g2, DBT, args, 0) != hipSuccess) {
-        (void)hipGetLastError();  // whole meshes then
-        std::vector<DItem> whole;
-        for (const DItem &it : D->hitem)
-          if (it.g == 0) whole.push_back(DItem{it.m, 0, 1, 0});
-        D->hitem = whole;
-        D->shared = false;
-        PF_HIP(hipMemcpyAsync(D->item.p, D->hitem.data(), sizeof(DItem) * D->hitem.size(), hipMemcpyHostToDevice,
-                              ctx->stream));
+        (void)hipGetLastError();  // e.g. fewer CUs available to this process
+        PF_CHECK(whole_meshes(ctx, D));
         a.nitem = (int32_t)D->hitem.size();
       }
     }
@@ -1490,6 +1504,13 @@ int pf_direct_solve_device(pf_ctx *ctx, DirectWork *D, int64_t n, const int64_t 
   PF_HIP(hipMemcpyAsync(raw.data(), D->t_raw.p, sizeof(int64_t) * 2 * nm, hipMemcpyDeviceToHost, ctx->stream));
   PF_HIP(hipMemcpyAsync(nrm.data(), D->norms.p, sizeof(double) * 2 * nm, hipMemcpyDeviceToHost, ctx->stream));
   PF_HIP(hipStreamSynchronize(ctx->stream));
+  if (D->shared && std::find(st.begin(), st.end(), (int32_t)PF_ERR_HIP) != st.end()) {
+    // a share waited in vain for another: again, without waits (the band holds a part of the factor)
+    PF_CHECK(whole_meshes(ctx, D));
+    D->factor_version = 0;
+    return pf_direct_solve_device(ctx, D, n, row_ptr, col_idx, val, nnz, rhs, x, mat_version, refine, mfma, mesh_stats,
+                                  total);
+  }
   int rate_khz = 0;
   PF_HIP(hipDeviceGetAttribute(&rate_khz, hipDeviceAttributeWallClockRate, ctx->device));
   const double tick_ms = rate_khz > 0 ? 1.0 / (double)rate_khz : 0.0;
@@ -1516,7 +1537,6 @@ int pf_direct_solve_device(pf_ctx *ctx, DirectWork *D, int64_t n, const int64_t 
     }
   }
   if (refactor && all_ok) D->factor_version = mat_version;
-  if (status < 0) pf_set_error("direct: a share of a factorization waited in vain for another");
   if (total) {
     std::memset(total, 0, sizeof(*total));
     total->status = status;

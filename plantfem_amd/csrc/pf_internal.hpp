@@ -37,6 +37,7 @@ struct pf_ctx {
   SolverWork *work = nullptr;  // workspace of the stateless solver entry point
   pf_forms forms{};            // how the last solves ran
   bool together = true;        // kernels whose workgroups wait for each other may be launched
+  int32_t polls = 0;           // bound of their waits (0: each kernel's own)
 };
 
 // cooperative launch of a kernel whose workgroups wait for each other; refused like one that does not

@@ -1,4 +1,4 @@
-"""Solves whose workgroups wait for each other, on a context that refuses such launches: the same
+"""Solves whose workgroups wait for each other, where such launches are refused or a wait gives up: the same
 systems by launches (plantfem_amd/csrc/bicgstab.hip) and with whole meshes (batch.hip, direct.hip)."""
 
 import numpy as np
@@ -81,4 +81,35 @@ def test_direct_shares_refused(alone, bad):
             x = s.solve(algorithm="GaussJordan", refine=0)
             assert np.linalg.norm(x - ref) <= 2 * 4 * 20 * (kd + 1) * EPS * np.linalg.norm(ref)
     assert alone.forms()["direct_shares"] == 1
+    s.close()
+
+
+@pytest.fixture
+def impatient():
+    """Every wait ends after one poll, so that workgroups give up where another is not there yet."""
+    c = L.Context(0)
+    c.together(True, polls=1)
+    yield c
+    c.close()
+
+
+@pytest.mark.parametrize("bad", [None, 700, 1498])
+def test_direct_shares_that_give_up(impatient, bad):
+    n, kd = 1499, 300
+    lower, rp, ci, val, rhs = band_system(n, kd, 3)
+    print("shares give up", bad, flush=True)
+    if bad is not None:
+        v = val.copy()
+        v[rp[bad] - 1 + min(bad, kd)] *= -1.0  # the diagonal entry
+        s = solver(impatient, rp, ci, v, rhs)
+        with pytest.raises(L.PFError) as e:
+            s.solve(algorithm="GaussJordan")
+        assert e.value.code == L.PF_NOT_SPD
+    else:
+        s = solver(impatient, rp, ci, val, rhs)
+        ref = sl.solveh_banded(lower, rhs, lower=True)
+        for _ in range(2):  # the second solve keeps the factor
+            x = s.solve(algorithm="GaussJordan", refine=0)
+            assert np.linalg.norm(x - ref) <= 2 * 4 * 20 * (kd + 1) * EPS * np.linalg.norm(ref)
+    assert impatient.forms()["direct_shares"] == 1
     s.close()
