@@ -75,6 +75,7 @@ struct BMat {
 
 struct BArgs {
   int32_t nitem, itrmax, stop_mode, inner_max;
+  int32_t polls, pad;  // of a workgroup for the other shares of its mesh before it gives up
   double er0, rel, target, delta;
   const BMesh *mesh;
   const BItem *item;
@@ -117,8 +118,9 @@ __device__ inline void wg_sum(double (&v)[NV], double (*sh)[BTB / 64]) {
 
 // s_sleep(1) polls for the other shares before a workgroup gives up: seconds, against the microseconds
 // between two meetings.  (The launch is cooperative and the shares are the first items of the
-// queue, one per workgroup: all of them run.)
-constexpr int SHARE_POLLS = 1 << 22;
+// queue, one per workgroup: all of them run.  Where they do not all the same, the batch is solved again
+// with whole meshes.)
+constexpr int32_t SHARE_POLLS = 1 << 22;
 
 template <int BTB>
 struct Shared {
@@ -136,6 +138,7 @@ struct Meet {
   Shared<BTB> &sh;
   Team *team;
   int g, G;
+  int32_t polls_max;
   uint32_t count;  // meetings so far
   bool failed;
 
@@ -156,7 +159,7 @@ struct Meet {
       }
       int polls = 0;
       while (__hip_atomic_load(&team->arrived, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < want &&
-             ++polls < SHARE_POLLS &&
+             ++polls < polls_max &&
              (polls % 1024 || !__hip_atomic_load(&team->failed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)))
         __builtin_amdgcn_s_sleep(1);
       const bool late = __hip_atomic_load(&team->arrived, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < want ||
@@ -475,7 +478,7 @@ __global__ void __launch_bounds__(BTB) k_batch(BArgs a) {
     const BItem it = a.item[q];
     const int32_t m = it.m;
     BMesh bm = a.mesh[m];
-    Meet<BTB> team{sh, a.team + m, it.g, it.G, 0u, false};
+    Meet<BTB> team{sh, a.team + m, it.g, it.G, a.polls, 0u, false};
     if (it.G > 1) {  // this share's rows: slices for the blocked layout, else rows
       const int64_t ns = bm.s1 - bm.s0, nd = bm.d1 - bm.d0, s0 = bm.s0, d0 = bm.d0;
       const auto row = [&](int g) {
@@ -954,6 +957,18 @@ unsigned batch_grid(pf_ctx *ctx, BatchWork *b, const pf_batch_tune &t, bool mixe
   return (unsigned)std::max<int64_t>(g, 1);
 }
 
+// from now on (until the batch is set again) every mesh is solved by one workgroup
+int whole_meshes(pf_ctx *ctx, BatchWork *b) {
+  std::vector<BItem> whole;
+  for (const BItem &it : b->hitem)
+    if (it.g == 0) whole.push_back(BItem{it.m, 0, 1, 0});
+  b->hitem = whole;
+  b->shared = false;
+  PF_HIP(hipMemcpyAsync(b->item.p, b->hitem.data(), sizeof(BItem) * b->hitem.size(), hipMemcpyHostToDevice,
+                        ctx->stream));
+  return PF_OK;
+}
+
 // queue reset + persistent kernel, captured once per (shape, pointers) and replayed
 int run_batch(pf_ctx *ctx, BatchWork *b, const BArgs &a, const pf_batch_tune &t, bool mixed, bool use_graph,
               float *ms) {
@@ -997,14 +1012,8 @@ int run_batch(pf_ctx *ctx, BatchWork *b, const BArgs &a, const pf_batch_tune &t,
   if (!launched) {
     reset();
     const int rc = mixed ? dispatch<32>(t, ln) : dispatch<64>(t, ln);
-    if (rc == PF_BATCH_WHOLE) {  // e.g. fewer CUs available to this process: whole meshes then
-      std::vector<BItem> whole;
-      for (const BItem &it : b->hitem)
-        if (it.g == 0) whole.push_back(BItem{it.m, 0, 1, 0});
-      b->hitem = whole;
-      b->shared = false;
-      PF_HIP(hipMemcpyAsync(b->item.p, b->hitem.data(), sizeof(BItem) * b->hitem.size(), hipMemcpyHostToDevice,
-                            ctx->stream));
+    if (rc == PF_BATCH_WHOLE) {  // e.g. fewer CUs available to this process
+      PF_CHECK(whole_meshes(ctx, b));
       BArgs aw = a;
       aw.nitem = (int32_t)b->hitem.size();
       return run_batch(ctx, b, aw, t, mixed, use_graph, ms);
@@ -1054,7 +1063,8 @@ int pf_batch_solve_device(pf_ctx *ctx, BatchWork *b, const int64_t *row_ptr, con
   }
   PF_CHECK(valid_tune(t, b->block_ok));
   PF_CHECK(prepare(ctx, b, row_ptr, col_idx, val, nnz, mixed, t.layout, o.jacobi == 2 ? 2 : (o.jacobi != 0 ? 1 : 0)));
-  const BArgs a = make_args(b, row_ptr, col_idx, val, rhs, x, o, mixed);
+  BArgs a = make_args(b, row_ptr, col_idx, val, rhs, x, o, mixed);
+  a.polls = ctx->polls > 0 ? ctx->polls : SHARE_POLLS;
   float ms = 0.f;
   PF_CHECK(run_batch(ctx, b, a, t, mixed, o.use_graph != 0, &ms));
   ctx->forms.batch_shares = 1;
@@ -1071,6 +1081,11 @@ int pf_batch_solve_device(pf_ctx *ctx, BatchWork *b, const int64_t *row_ptr, con
   const double tick_ms = rate_khz > 0 ? 1.0 / (double)rate_khz : 0.0;
   int64_t tmin = raw[0];
   for (int32_t m = 0; m < b->nmesh; ++m) tmin = std::min(tmin, raw[2 * m]);
+  if (b->shared && std::any_of(st.begin(), st.end(), [](const auto &s) { return s.status == PF_ERR_HIP; })) {
+    // a share waited in vain for another: again, without waits
+    PF_CHECK(whole_meshes(ctx, b));
+    return pf_batch_solve_device(ctx, b, row_ptr, col_idx, val, nnz, rhs, x, o, tune, mat_version, mesh_stats, total);
+  }
   int status = PF_OK;
   int64_t iters = 0, reps = 0;
   double worst = 0.0;
@@ -1081,10 +1096,6 @@ int pf_batch_solve_device(pf_ctx *ctx, BatchWork *b, const int64_t *row_ptr, con
     reps += st[m].replacements;
     worst = std::max(worst, st[m].true_relres);
     if (status == PF_OK && st[m].status != PF_OK) status = st[m].status;
-    if (st[m].status == PF_ERR_HIP) {
-      pf_set_error("batch: the workgroups of mesh %d did not run together", m);
-      return PF_ERR_HIP;
-    }
   }
   if (mesh_stats) std::memcpy(mesh_stats, st.data(), sizeof(pf_batch_mesh_stats) * b->nmesh);
   if (total) {

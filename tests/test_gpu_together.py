@@ -113,3 +113,22 @@ def test_direct_shares_that_give_up(impatient, bad):
             assert np.linalg.norm(x - ref) <= 2 * 4 * 20 * (kd + 1) * EPS * np.linalg.norm(ref)
     assert impatient.forms()["direct_shares"] == 1
     s.close()
+
+
+@pytest.mark.parametrize("precision", [64, 32])
+@pytest.mark.parametrize("tune", [None, {"layout": 0, "sub": 16, "block": 256, "blocks_per_cu": 0}])
+def test_batch_shares_that_give_up(impatient, alone, precision, tune):
+    out = []
+    for c in (impatient, alone):
+        rng = np.random.default_rng(11)
+        u = B.union([B.block(n, rng) for n in (3, 13, 10, 5, 11)])
+        s = B.build_solver(u, c)
+        s.relative_er = REL
+        print("shares give up", precision, tune, flush=True)
+        for _ in range(2):
+            x, st = s.solveBatch(precision=precision, tune=tune, stop_mode=1, target_relres=REL)
+            assert not st["status"].any() and c.forms()["batch_shares"] == 1
+            out.append(x)
+        s.close()
+    for x in out[:-1]:  # the solve that was done again is the one without shares
+        assert np.array_equal(x, out[-1])
