@@ -590,7 +590,7 @@ __global__ void __launch_bounds__(BT) k_pupdate(int64_t n, V *__restrict__ p, co
 // the launches above.
 constexpr int PT = 512;  // threads of a workgroup: 256 registers each, half of them for the matrix
 constexpr unsigned long long EMPTY = 0xfff8dead5107e317ull;
-constexpr int POLLS = 1 << 17;                                    // about 0.1 s
+constexpr int32_t POLLS = 1 << 17;                                // about 0.1 s
 constexpr int PG_MAX = 1024;                                      // workgroups a sum's buffer holds
 constexpr int SUM_WORDS = 8 * 2 * PG_MAX;                         // buffers x sums x workgroups
 
@@ -608,6 +608,7 @@ struct PersistArgs {
   Scal *sc;
   int32_t *fail;
   int32_t most;                // iterations of this launch
+  int32_t polls;               // of a place before a workgroup gives up
 };
 
 __device__ inline void put(unsigned long long *p, double d) {
@@ -622,7 +623,7 @@ __device__ inline void empty(unsigned long long *p) {
 
 // out[k] = *at(k) for k < cnt <= N, all of them awaited together
 template <int N, typename F>
-__device__ inline void take(F at, int cnt, double (&out)[N], int &bad) {
+__device__ inline void take(F at, int cnt, double (&out)[N], int polls_max, int &bad) {
   unsigned long long v[N];
   int polls = 0;
   bool more;
@@ -633,7 +634,7 @@ __device__ inline void take(F at, int cnt, double (&out)[N], int &bad) {
       v[k] = k < cnt ? __hip_atomic_load(at(k), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0ull;
 #pragma unroll
     for (int k = 0; k < N; ++k) more = more || v[k] == EMPTY;
-  } while (more && ++polls < POLLS);
+  } while (more && ++polls < polls_max);
   if (more) bad = 1;
 #pragma unroll
   for (int k = 0; k < N; ++k) out[k] = __longlong_as_double((long long)v[k]);
@@ -704,7 +705,7 @@ __device__ inline bool all_sum(const PersistArgs &a, unsigned seq, double (&d)[N
         double got[PG_LANE];
         const int left = G - g0 - tid;  // this lane's workgroups: g0 + tid + 64 i
         take<PG_LANE>([&](int i) { return buf + k * PG_MAX + g0 + tid + 64 * i; }, left > 0 ? (left + 63) / 64 : 0,
-                      got, bad);
+                      got, a.polls, bad);
 #pragma unroll
         for (int i = 0; i < PG_LANE; ++i) t += got[i];
       }
@@ -870,7 +871,7 @@ __global__ void __launch_bounds__(PT) k_persist(PersistArgs a) {
       d1[0] = r0 * y;
     }
     if (!all_sum<1>(a, seq++, d1, red, bad,
-                    [&] { take<PH>([&](int k) { return a.yg + now + hc[k]; }, hn, hy, bad); }))
+                    [&] { take<PH>([&](int k) { return a.yg + now + hc[k]; }, hn, hy, a.polls, bad); }))
       return;
     const double c2 = d1[0], alpha = cc1 / c2;
     if (guard && !isfinite(alpha)) {  // r0.Ap lost: stop before x is touched
@@ -897,7 +898,7 @@ __global__ void __launch_bounds__(PT) k_persist(PersistArgs a) {
     }
     double hv[PH];
     if (!all_sum<2>(a, seq++, d2, red, bad,
-                    [&] { take<PH>([&](int k) { return a.vg + now + hc[k]; }, hn, hv, bad); }))
+                    [&] { take<PH>([&](int k) { return a.vg + now + hc[k]; }, hn, hv, a.polls, bad); }))
       return;
     if (d2[1] == 0.0) {  // "Bicgstab devide by zero" (FEMSolverClass.f90:2266)
       status = PF_BREAKDOWN_VV;
@@ -1567,6 +1568,9 @@ int run_loop(pf_ctx *ctx, SolverWork *w, int slot, const Launch &L, const Mat<V,
 // rounding decides the iteration count, and theirs ends where the reference's does.
 constexpr int64_t PERSIST_MIN_ROWS = 64, PERSIST_MAX_ROWS = 100000;
 constexpr int PERSIST_CHUNK = 4096;  // iterations of a launch (tens of milliseconds)
+// where the workgroups did not run together (other processes on the card) the wait took 0.1 s: the next
+// solves go by launches at once
+constexpr int PERSIST_REST = 16;
 
 // the kernel for `sub` lanes per segment and at least `need` segments per subgroup
 const void *persist_kernel(int sub, int need) {
@@ -1599,6 +1603,10 @@ int persist_prepare(pf_ctx *ctx, SolverWork *w, int64_t n, const int64_t *row_pt
                     bool *ok) {
   *ok = false;
   if (n < PERSIST_MIN_ROWS || n > PERSIST_MAX_ROWS || nnz < 1) return PF_OK;
+  if (ctx->persist_rest > 0) {
+    --ctx->persist_rest;
+    return PF_OK;
+  }
   RowSplit &p = w->split;
   if (!p.ready) {
     const double avg = (double)nnz / (double)n;
@@ -1646,6 +1654,7 @@ int run_persist(pf_ctx *ctx, SolverWork *w, int64_t n, const int64_t *row_ptr, c
   a.sums = w->sums.p;
   a.sc = w->sc.p;
   a.fail = w->pfail.p;
+  a.polls = ctx->polls > 0 ? ctx->polls : POLLS;
   a.most = o.debug && o.check_every > 0 ? o.check_every : PERSIST_CHUNK;
   const size_t lds = persist_lds(p);
   const void *kernel = persist_kernel(p.sub, persist_segments(p));
@@ -1661,12 +1670,16 @@ int run_persist(pf_ctx *ctx, SolverWork *w, int64_t n, const int64_t *row_ptr, c
       e = pf_launch_together(ctx, kernel, (unsigned)p.G, PT, args, lds);
     if (e != hipSuccess) {  // e.g. fewer CUs available to this process: the launches then
       (void)hipGetLastError();
+      ctx->persist_rest = PERSIST_REST;
       return PF_OK;
     }
     PF_HIP(hipMemcpyAsync(hs, w->sc.p, sizeof(Scal), hipMemcpyDeviceToHost, ctx->stream));
     PF_HIP(hipMemcpyAsync(w->h_fail, w->pfail.p, sizeof(int32_t), hipMemcpyDeviceToHost, ctx->stream));
     PF_HIP(hipStreamSynchronize(ctx->stream));
-    if (*w->h_fail) return PF_OK;
+    if (*w->h_fail) {
+      ctx->persist_rest = PERSIST_REST;
+      return PF_OK;
+    }
     if (o.debug) std::printf("BiCGSTAB >> itr %d  sqrt(rr) %.6e\n", hs->itr_last, std::sqrt(hs->rr));
     if (hs->done) break;
   }

@@ -38,6 +38,7 @@ struct pf_ctx {
   pf_forms forms{};            // how the last solves ran
   bool together = true;        // kernels whose workgroups wait for each other may be launched
   int32_t polls = 0;           // bound of their waits (0: each kernel's own)
+  int persist_rest = 0;        // BiCGSTAB solves by launches before the one kernel is tried again
 };
 
 // cooperative launch of a kernel whose workgroups wait for each other; refused like one that does not

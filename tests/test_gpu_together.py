@@ -132,3 +132,23 @@ def test_batch_shares_that_give_up(impatient, alone, precision, tune):
         s.close()
     for x in out[:-1]:  # the solve that was done again is the one without shares
         assert np.array_equal(x, out[-1])
+
+
+@pytest.mark.parametrize("x0", [False, True])
+def test_one_kernel_that_gives_up(impatient, alone, x0):
+    crs = _crs(_matrix("ragged", 3000))
+    rng = np.random.default_rng(1)
+    b = rng.standard_normal(3000)
+    kw = {"x0": rng.standard_normal(3000) if x0 else None, "stop_mode": 1, "relative_er": 1e-12}
+    print("one kernel gives up", x0, flush=True)
+    x, st = bicgstab_crs(*crs, b, ctx=impatient, **kw)
+    y, sy = bicgstab_crs(*crs, b, ctx=alone, **kw)
+    assert impatient.forms()["one_kernel"] == 0 and st["status"] == 0
+    assert np.array_equal(x, y) and st["iterations"] == sy["iterations"]
+    impatient.together(True)
+    ran = []
+    for _ in range(17):  # launches at once for a while, then the one kernel again
+        x, st = bicgstab_crs(*crs, b, ctx=impatient, **kw)
+        ran.append(impatient.forms()["one_kernel"])
+        assert st["status"] == 0 and np.linalg.norm(x - y) <= 1e-9 * np.linalg.norm(y)
+    assert ran == [0] * 16 + [1]
