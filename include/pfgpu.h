@@ -432,7 +432,8 @@ typedef struct {
   int32_t layout;        /* 1: blocked Sell3 (64-node slices, DOF=3 node blocks); 0: CRS rows */
   int32_t sub;           /* layout 0: lanes per CRS row (8, 16 or 32) */
   int32_t block;         /* threads per workgroup: 256, 512 or 1024 */
-  int32_t blocks_per_cu; /* resident workgroups per CU in the grid (0: the occupancy limit) */
+  int32_t blocks_per_cu; /* resident workgroups per CU in the grid (0: the occupancy limit, or 1 where
+                            several workgroups share a mesh) */
 } pf_batch_tune;
 
 /* Result of one mesh. */

@@ -950,8 +950,8 @@ unsigned batch_grid(pf_ctx *ctx, BatchWork *b, const pf_batch_tune &t, bool mixe
   int occ = 1;
   const int rc = mixed ? dispatch<32>(t, Occ{&occ}) : dispatch<64>(t, Occ{&occ});
   if (rc != PF_OK || occ < 1) occ = 1;
-  int per_cu = t.blocks_per_cu > 0 ? std::min(t.blocks_per_cu, occ) : occ;
-  if (b->shared) per_cu = 1;  // what the shares are made for (224 compact meshes: 153 ms, 177 with two)
+  // left open, shares get the one per CU that they are made for (224 compact meshes: 153 ms, 177 with two)
+  const int per_cu = t.blocks_per_cu > 0 ? std::min(t.blocks_per_cu, occ) : (b->shared ? 1 : occ);
   int64_t g = (int64_t)ctx->num_cus * per_cu;
   g = std::min<int64_t>(g, (int64_t)b->hitem.size());
   return (unsigned)std::max<int64_t>(g, 1);

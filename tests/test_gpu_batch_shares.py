@@ -53,3 +53,18 @@ def test_one_shared_mesh_matches_the_single_solver(ctx):
     A = to_scipy(rp, ci, val)
     assert st["status"][0] == 0
     assert relres(A, x, rhs) <= 1.5 * REL + rounding_floor(A, x, rhs)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("per_cu", [0, 1, 2])
+def test_workgroups_per_cu_with_shares(ctx, per_cu):
+    """The caller's number of workgroups per CU counts with shared meshes too; left open it is one."""
+    rng = np.random.default_rng(13)
+    u = B.union([B.block(13, rng)] + [B.block(2, rng) for _ in range(300)])
+    s = B.build_solver(u, ctx)
+    s.relative_er = REL
+    print("workgroups per CU", per_cu, flush=True)
+    x, st = s.solveBatch(tune={"layout": 1, "sub": 64, "block": 256, "blocks_per_cu": per_cu}, stop_mode=1)
+    s.close()
+    assert not st["status"].any() and np.all(st["true_relres"] <= 1.5 * REL) and ctx.forms()["batch_shares"] > 1
+    assert (st["workgroup"].max() >= 256) == (per_cu == 2)  # 256 CUs
