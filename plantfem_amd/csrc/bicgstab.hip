@@ -1349,7 +1349,22 @@ int choose_sub(double avg_row) {  // ~five nonzeros per lane, 4..64 lanes per CR
     else { constexpr bool A_ = false; __VA_ARGS__; }                        \
   }
 
-constexpr int REPL_EVERY = 8;
+// Mixed precision: iterations between the points at which a due residual replacement is done.  The two
+// kernels of such a point cost 11 us when nothing is due, 2% of a 3.1M-row iteration, so they come every
+// 8 iterations; the iterations between the request and the point return at entry.  Where replacements
+// are asked for more often these would outweigh them (320 iterations at 27,783 rows, every 8 against every
+// iteration: inner_max 2 23.9 / 16.4 ms, inner_tol 0.9 22.7 / 16.1, 0.6 14.5 / 13.8, 0.3 equal): a limit of
+// iterations below 32 gets a divisor, which the request meets at once, and a tolerance that is reached in few
+// iterations (18 ln(1 / inner_tol) in these solves) half of them or fewer.
+int replace_every(const pf_solve_opts &o) {
+  int every = 8;
+  if (o.inner_max > 0 && o.inner_max < 32)
+    while (o.inner_max % every) every /= 2;
+  const double tol = o.inner_tol > 0.0 && o.inner_tol < 1.0 ? o.inner_tol : 0.1;
+  const int at_tol = tol <= 0.37 ? 8 : (tol <= 0.64 ? 4 : (tol <= 0.8 ? 2 : 1));
+  return std::min(every, at_tol);
+}
+
 // rows from which the element tiles are taken: their iteration is six launches, 25-31 us up to
 // 50,000 rows on MI355X, the other forms four.  Microseconds per iteration, blocked / tiles:
 // Cube3D 28k rows 44 / 31, 73k 49 / 33, 207k 80 / 44, 681k 200 / 70, 3.09M 846 / 228;
@@ -1417,7 +1432,7 @@ int enqueue_init(pf_ctx *ctx, const Launch &L, const Mat<V, M> &m, const V *b, V
 template <typename V, typename M>
 int enqueue_iters(pf_ctx *ctx, const Launch &L, const Mat<V, M> &m, V *x, V *r, const V *r0, V *p, V *y, V *v,
                   Scal *sc, double *part, double *hist, int count, const Rel<V> *rel, V *ebuf,
-                  hipEvent_t *ev = nullptr, bool ev_all = true) {
+                  hipEvent_t *ev = nullptr, bool ev_all = true, int every = 1) {
   PF_CHECK(check_grid(ctx, L));
   // ev: events 0 and 1 bracket y = A p; with ev_all, events 2-4 follow the other kernels
   hipEvent_t *eva = ev_all ? ev : nullptr;
@@ -1470,9 +1485,7 @@ int enqueue_iters(pf_ctx *ctx, const Launch &L, const Mat<V, M> &m, V *x, V *r, 
     k_pupdate<V><<<L.grid_e, BT, 0, st>>>(m.n, p, r, y, sc, p3, ge, par, hist, rel ? rel->zhi : nullptr,
                                           rel ? x : nullptr);
     if (eva) PF_HIP(hipEventRecord(eva[5 * it + 4], st));
-    // a due replacement is done every REPL_EVERY iterations (the ones in between return at
-    // entry): its two kernels cost 11 us when nothing is due, 2% of a 3.1M-row iteration
-    if (rel && (ev || it % REPL_EVERY == REPL_EVERY - 1 || it == count - 1))
+    if (rel && (ev || it % every == every - 1 || it == count - 1))
       PF_CHECK(enqueue_replacement<false>(ctx, *rel, sc, part + PART_PI * G));
   }
   PF_HIP(hipGetLastError());
@@ -1489,6 +1502,7 @@ int run_loop(pf_ctx *ctx, SolverWork *w, int slot, const Launch &L, const Mat<V,
   chunk += chunk & 1;  // even: the parity of the iteration counter slots carries across chunks
   const bool timing = o.kernel_timing != 0;
   bool use_graph = o.use_graph != 0 && !timing && pf_graphs_allowed();
+  const int every = rel ? replace_every(o) : 1;
   if (timing) {
     while ((int)w->evs.size() < 5 * chunk) {
       hipEvent_t e;
@@ -1499,7 +1513,7 @@ int run_loop(pf_ctx *ctx, SolverWork *w, int slot, const Launch &L, const Mat<V,
   // everything the captured chunk bakes in: a replay is valid only while all of it is
   const uint64_t key[KEY_WORDS] = {
       (uint64_t)(uintptr_t)ebuf, (uint64_t)L.grid, (uint64_t)L.grid_e * 131 + (uint64_t)L.sub, (uint64_t)L.layout,
-      (uint64_t)chunk, (uint64_t)m.n, (uint64_t)(uintptr_t)m.row_ptr, (uint64_t)(uintptr_t)m.col_idx,
+      (uint64_t)chunk * 16 + (uint64_t)every, (uint64_t)m.n, (uint64_t)(uintptr_t)m.row_ptr, (uint64_t)(uintptr_t)m.col_idx,
       (uint64_t)(uintptr_t)m.val, (uint64_t)m.nn, (uint64_t)m.nslices, (uint64_t)(uintptr_t)m.soff,
       (uint64_t)(uintptr_t)m.width, (uint64_t)(uintptr_t)m.col, (uint64_t)(uintptr_t)m.sval,
       (uint64_t)(uintptr_t)x, (uint64_t)(uintptr_t)r, (uint64_t)(uintptr_t)r0, (uint64_t)(uintptr_t)p,
@@ -1523,7 +1537,11 @@ int run_loop(pf_ctx *ctx, SolverWork *w, int slot, const Launch &L, const Mat<V,
       w->gexec[slot] = nullptr;
     }
     PF_CHECK(pf_capture_graph(
-        ctx, [&] { return enqueue_iters<V>(ctx, L, m, x, r, r0, p, y, v, sc, w->part.p, hist, chunk, rel, ebuf); },
+        ctx,
+        [&] {
+          return enqueue_iters<V>(ctx, L, m, x, r, r0, p, y, v, sc, w->part.p, hist, chunk, rel, ebuf, nullptr, true,
+                                  every);
+        },
         &w->gexec[slot]));
     if (w->gexec[slot])
       std::memcpy(w->gkey[slot], key, sizeof(key));
@@ -1536,7 +1554,7 @@ int run_loop(pf_ctx *ctx, SolverWork *w, int slot, const Launch &L, const Mat<V,
       PF_HIP(hipGraphLaunch(w->gexec[slot], ctx->stream));
     } else {
       PF_CHECK(enqueue_iters<V>(ctx, L, m, x, r, r0, p, y, v, sc, w->part.p, hist, chunk, rel, ebuf,
-                                timing ? w->evs.data() : nullptr, o.kernel_timing != 2));
+                                timing ? w->evs.data() : nullptr, o.kernel_timing != 2, every));
     }
     PF_HIP(hipMemcpyAsync(hs, sc, sizeof(Scal), hipMemcpyDeviceToHost, ctx->stream));
     PF_HIP(hipStreamSynchronize(ctx->stream));

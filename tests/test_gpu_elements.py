@@ -256,3 +256,22 @@ def test_writes_through_an_earlier_view(precision):
     x = np.random.default_rng(2).standard_normal(s.n)
     A = s.getCRS().to_scipy()
     assert np.all(np.abs(_apply(s, x) - A @ x) <= 1e-11 * (abs(A) @ np.abs(x)))
+
+
+@pytest.mark.parametrize("kw", [{"inner_max": 1}, {"inner_max": 2}, {"inner_max": 6}, {"inner_max": 7}, {"inner_max": 33},
+                                {"inner_tol": 0.5}, {"inner_tol": 0.7}, {"inner_tol": 0.95}])
+@pytest.mark.parametrize("precision,dims", [(32, (9, 8, 7)), (48, (9, 8, 7)), (48, (29, 28, 27))])
+def test_replacement_intervals(precision, dims, kw):
+    """Residual replacements asked for after every few iterations are done as asked: no iteration is run
+    between the request and the replacement, whatever the interval at which they are looked for."""
+    nod, el = fem.cube3d(*dims)
+    s = _system(nod, el)
+    s.addTraction([-1e300, 1e300, -1e300, 1e300, 1 - 1e-9, 1 + 1e-9], -1e4)
+    base = np.nonzero(nod[:, 2] == 0)[0]
+    s.fix(1, (3 * base[:, None] + np.arange(1, 4)).ravel().astype(np.int32), FixValue=0.0)
+    s.itrmax = 66
+    s.solve(precision=precision, target_relres=1e-30, raise_on_breakdown=False, **kw)
+    st = s.last_stats
+    assert st["iterations"] <= 66
+    if "inner_max" in kw:  # one at least every inner_max iterations (the last iteration asks for none)
+        assert st["outer_iterations"] >= (st["iterations"] - 1) // kw["inner_max"]
