@@ -1365,6 +1365,13 @@ int replace_every(const pf_solve_opts &o) {
   return std::min(every, at_tol);
 }
 
+// Every third iteration or oftener the residuals, which the element form takes from CRS rows, cost more than
+// its products save (320 iterations at 292k rows, element / blocked: inner_max 1 45.4 / 35.7 ms, 2 30.7 / 28.1,
+// 3 26.5 / 25.6, 8 19.8 / 22.4; inner_tol 0.9 28.5 / 26.7, 0.75 21.1 / 22.9)
+bool replaces_often(const pf_solve_opts &o) {
+  return (o.inner_max > 0 && o.inner_max < 4) || (o.inner_tol > 0.8 && o.inner_tol < 1.0);
+}
+
 // rows from which the element tiles are taken: their iteration is six launches, 25-31 us up to
 // 50,000 rows on MI355X, the other forms four.  Microseconds per iteration, blocked / tiles:
 // Cube3D 28k rows 44 / 31, 73k 49 / 33, 207k 80 / 44, 681k 200 / 70, 3.09M 846 / 228;
@@ -1985,14 +1992,15 @@ int pf_bicgstab_device(pf_ctx *ctx, SolverWork *w, int64_t n, const int64_t *row
     return PF_INVALID;
   }
   // element by element when the matrix is a mesh's stiffness, from ELEM_MIN_ROWS rows on, unless
-  // the options ask for a matrix layout, the ILU factor or the symmetric scaling
+  // the options ask for a matrix layout, the ILU factor, the symmetric scaling or frequent replacements
   ElemView ev{};
   double *epart = nullptr;
   bool persist = false;
   if (o.spmv_kind == 0 && o.precision == 64 && o.preconditioning != 2 && o.kernel_timing == 0)
     PF_CHECK(persist_prepare(ctx, w, n, row_ptr, col_idx, nnz, &persist));
   if (!persist && elem && o.spmv_kind == 0 && n >= ELEM_MIN_ROWS && o.preconditioning != 2 &&
-      (o.precision == 64 || ((o.precision == 48 || o.precision == 32) && (o.jacobi == 0 || o.jacobi == 2)))) {
+      (o.precision == 64 || ((o.precision == 48 || o.precision == 32) && (o.jacobi == 0 || o.jacobi == 2) &&
+                             !replaces_often(o)))) {
     bool ok = false;
     PF_CHECK(pf_elem_plan(ctx, *elem->g, &ok));
     if (ok) {
