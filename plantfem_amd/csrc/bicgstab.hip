@@ -1592,6 +1592,7 @@ int run_loop(pf_ctx *ctx, SolverWork *w, int slot, const Launch &L, const Mat<V,
 // Below 64 rows the launches stay: systems of a few rows end by finite termination, where one
 // rounding decides the iteration count, and theirs ends where the reference's does.
 constexpr int64_t PERSIST_MIN_ROWS = 64, PERSIST_MAX_ROWS = 100000;
+constexpr size_t PERSIST_LDS = 140 * 1024;
 constexpr int PERSIST_CHUNK = 4096;  // iterations of a launch (tens of milliseconds)
 // where the workgroups did not run together (other processes on the card) the wait took 0.1 s: the next
 // solves go by launches at once
@@ -1646,7 +1647,7 @@ int persist_prepare(pf_ctx *ctx, SolverWork *w, int64_t n, const int64_t *row_pt
     PF_CHECK(pf_row_split_build(ctx, n, row_ptr, col_idx, nnz, (int)G, sub, p));
     p.ready = true;
   }
-  *ok = p.staged && p.maxrows <= PT && persist_kernel(p.sub, persist_segments(p)) && persist_lds(p) <= 140 * 1024;
+  *ok = p.staged && p.maxrows <= PT && persist_kernel(p.sub, persist_segments(p)) && persist_lds(p) <= PERSIST_LDS;
   return PF_OK;
 }
 
@@ -1679,7 +1680,7 @@ int run_persist(pf_ctx *ctx, SolverWork *w, int64_t n, const int64_t *row_ptr, c
   a.sums = w->sums.p;
   a.sc = w->sc.p;
   a.fail = w->pfail.p;
-  a.polls = ctx->polls > 0 ? ctx->polls : POLLS;
+  a.polls = ctx->polls > 0 && p.G > 1 ? ctx->polls : POLLS;
   a.most = o.debug && o.check_every > 0 ? o.check_every : PERSIST_CHUNK;
   const size_t lds = persist_lds(p);
   const void *kernel = persist_kernel(p.sub, persist_segments(p));
@@ -1690,9 +1691,12 @@ int run_persist(pf_ctx *ctx, SolverWork *w, int64_t n, const int64_t *row_ptr, c
     PF_HIP(hipGetLastError());
     void *args[] = {&a};
     hipError_t e = hipSuccess;
-    if (lds > 64 * 1024) e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    // the kernel's limit, not this system's need: another thread may launch the same kernel
+    if (lds > 64 * 1024) e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)PERSIST_LDS);
+    // one workgroup waits for no other: an ordinary launch, which does not take turns with other contexts'
     if (e == hipSuccess)
-      e = pf_launch_together(ctx, kernel, (unsigned)p.G, PT, args, lds);
+      e = p.G > 1 ? pf_launch_together(ctx, kernel, (unsigned)p.G, PT, args, lds)
+                  : hipLaunchKernel(kernel, dim3(1), dim3(PT), args, lds, ctx->stream);
     if (e != hipSuccess) {  // e.g. fewer CUs available to this process: the launches then
       (void)hipGetLastError();
       ctx->persist_rest = PERSIST_REST;

@@ -152,3 +152,58 @@ def test_one_kernel_that_gives_up(impatient, alone, x0):
         ran.append(impatient.forms()["one_kernel"])
         assert st["status"] == 0 and np.linalg.norm(x - y) <= 1e-9 * np.linalg.norm(y)
     assert ran == [0] * 16 + [1]
+
+
+def test_one_workgroup_waits_for_none(alone):
+    """A system that one workgroup holds needs no such launch and takes its kernel all the same."""
+    crs = _crs(_matrix("tridiagonal", 300))
+    b = np.random.default_rng(2).standard_normal(300)
+    x, st = bicgstab_crs(*crs, b, ctx=alone, stop_mode=1, relative_er=1e-12)
+    assert alone.forms()["one_kernel"] == 1 and st["status"] == 0 and st["true_relres"] < 1e-11
+
+
+def test_threads():
+    """Contexts in threads of their own, each with solves whose workgroups wait for each other: the launches
+    take turns, and every result is that of a solve alone."""
+    import threading
+    crs = _crs(_matrix("ragged", 3000))
+    rng = np.random.default_rng(1)
+    b = rng.standard_normal(3000)
+    lower, rp, ci, val, rhs = band_system(1499, 300, 3)
+    u = B.union([B.block(n, rng) for n in (3, 13, 10)])
+
+    def one(c, out):
+        for _ in range(20):
+            out.append((bicgstab_crs(*crs, b, ctx=c, stop_mode=1, relative_er=1e-12)[0], c.forms()["one_kernel"]))
+
+    def direct(c, out):
+        s = solver(c, rp, ci, val, rhs)
+        for _ in range(10):
+            s.setDirectKernel(True)  # drops the factor
+            out.append((s.solve(algorithm="GaussJordan", refine=0), c.forms()["direct_shares"]))
+        s.close()
+
+    def shares(c, out):
+        s = B.build_solver(u, c)
+        s.relative_er = REL
+        for _ in range(4):
+            out.append((s.solveBatch(stop_mode=1)[0], c.forms()["batch_shares"]))
+        s.close()
+
+    print("threads", flush=True)
+    work = [one, direct, shares]
+    ctxs = [L.Context(0) for _ in range(2 * len(work))]
+    logs = [[] for _ in ctxs]
+    for f, c, out in zip(work, ctxs, logs):  # alone
+        f(c, out)
+    threads = [threading.Thread(target=f, args=(c, out)) for f, c, out in zip(work, ctxs[3:], logs[3:])]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for c in ctxs:
+        c.close()
+    for first, second in zip(logs[:3], logs[3:]):
+        assert len(first) == len(second)
+        for x, form in first + second:
+            assert np.array_equal(x, first[0][0]) and form == first[0][1]
