@@ -559,8 +559,9 @@ __global__ void __launch_bounds__(BT) k_pupdate(int64_t n, V *__restrict__ p, co
 }
 
 // ---- whole iterations in one kernel (small systems) --------------------------------------
-// Below about 80,000 rows an iteration of four to six launches is their latency (17-49 us); here
-// one workgroup per CU keeps its rows' matrix entries and vectors in registers, every x entry its
+// In small systems an iteration of four to six launches is their latency (17-49 us); where the matrix
+// fits the registers of all CUs (hex8 meshes up to about 50,000 rows), one workgroup per CU keeps its
+// rows' matrix entries and vectors in registers, every x entry its
 // rows use (its "halo", the sorted distinct columns of RowSplit) in LDS, and iterates without
 // returning to the host.  Per iteration the workgroups publish y = A p and v = A e once each; r, p
 // and e of the halo are updated by everyone from y, v and the scalars with the owner's operations
@@ -665,8 +666,8 @@ constexpr int PG_LANE = 8;                       // workgroups' sums a lane of t
 // d summed over all threads of all workgroups, the same value in every thread; `between` runs after
 // this workgroup's sum is out and before the others' are awaited; false when a poll gave up
 template <int NV, typename F>
-__device__ inline bool all_sum(const PersistArgs &a, unsigned seq, double (&d)[NV], double (&red)[2][PW + 1], int &bad,
-                               F between) {
+__device__ inline bool all_sum(const PersistArgs &a, int polls_max, unsigned seq, double (&d)[NV],
+                               double (&red)[2][PW + 1], int &bad, F between) {
   const int tid = threadIdx.x, G = gridDim.x;
 #pragma unroll
   for (int k = 0; k < NV; ++k) {
@@ -705,7 +706,7 @@ __device__ inline bool all_sum(const PersistArgs &a, unsigned seq, double (&d)[N
         double got[PG_LANE];
         const int left = G - g0 - tid;  // this lane's workgroups: g0 + tid + 64 i
         take<PG_LANE>([&](int i) { return buf + k * PG_MAX + g0 + tid + 64 * i; }, left > 0 ? (left + 63) / 64 : 0,
-                      got, a.polls, bad);
+                      got, polls_max, bad);
 #pragma unroll
         for (int i = 0; i < PG_LANE; ++i) t += got[i];
       }
@@ -734,6 +735,8 @@ __global__ void __launch_bounds__(PT) k_persist(PersistArgs a) {
   const int tid = threadIdx.x, b = blockIdx.x;
   Scal *sc = a.sc;
   if (sc->done) return;
+  int polls_max = a.polls;
+  asm volatile("" : "+v"(polls_max));  // stays in a register: read again for every poll it costs 3% of an iteration
   const int row0 = a.roff[b], rows = a.roff[b + 1] - row0;
   const int U = a.ucnt[b];
   double *hp = psh, *he = hp + a.umax, *cell = he + a.umax;
@@ -870,8 +873,8 @@ __global__ void __launch_bounds__(PT) k_persist(PersistArgs a) {
       put(a.yg + now + gi, y);
       d1[0] = r0 * y;
     }
-    if (!all_sum<1>(a, seq++, d1, red, bad,
-                    [&] { take<PH>([&](int k) { return a.yg + now + hc[k]; }, hn, hy, a.polls, bad); }))
+    if (!all_sum<1>(a, polls_max, seq++, d1, red, bad,
+                    [&] { take<PH>([&](int k) { return a.yg + now + hc[k]; }, hn, hy, polls_max, bad); }))
       return;
     const double c2 = d1[0], alpha = cc1 / c2;
     if (guard && !isfinite(alpha)) {  // r0.Ap lost: stop before x is touched
@@ -897,8 +900,8 @@ __global__ void __launch_bounds__(PT) k_persist(PersistArgs a) {
       d2[1] = v * v;
     }
     double hv[PH];
-    if (!all_sum<2>(a, seq++, d2, red, bad,
-                    [&] { take<PH>([&](int k) { return a.vg + now + hc[k]; }, hn, hv, a.polls, bad); }))
+    if (!all_sum<2>(a, polls_max, seq++, d2, red, bad,
+                    [&] { take<PH>([&](int k) { return a.vg + now + hc[k]; }, hn, hv, polls_max, bad); }))
       return;
     if (d2[1] == 0.0) {  // "Bicgstab devide by zero" (FEMSolverClass.f90:2266)
       status = PF_BREAKDOWN_VV;
@@ -916,7 +919,7 @@ __global__ void __launch_bounds__(PT) k_persist(PersistArgs a) {
     d2[0] = own ? r * r : 0.0;
     d2[1] = own ? r0 * r : 0.0;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the emptied places are empty for everyone
-    if (!all_sum<2>(a, seq++, d2, red, bad, [&] {
+    if (!all_sum<2>(a, polls_max, seq++, d2, red, bad, [&] {
 #pragma unroll
           for (int k = 0; k < PH; ++k) hr[k] = __builtin_fma(-omega, hv[k], hr[k]);
         }))
@@ -1537,7 +1540,8 @@ int run_loop(pf_ctx *ctx, SolverWork *w, int slot, const Launch &L, const Mat<V,
       (uint64_t)(uintptr_t)m.st.lidx, (uint64_t)(uintptr_t)m.st.ucnt, (uint64_t)(uintptr_t)m.st.ubase,
       (uint64_t)(uintptr_t)m.st.ucol, (uint64_t)m.st.nb * 4099 + (uint64_t)m.st.rpb,
       (uint64_t)(uintptr_t)m.el.tdesc, (uint64_t)(uintptr_t)m.epart, (uint64_t)(uintptr_t)m.el.nrec,
-      (uint64_t)(uintptr_t)m.el.rscale, ((uint64_t)m.el.ntile << 32) + (uint64_t)m.el.umax * 4 + (uint64_t)m.el.affine * 2 + (uint64_t)m.jmode};
+      (uint64_t)(uintptr_t)m.el.rscale,
+      ((uint64_t)m.el.ntile << 32) + (uint64_t)m.el.umax * 4 + (uint64_t)m.el.affine * 2 + (uint64_t)m.jmode};
   if (use_graph && (w->gexec[slot] == nullptr || std::memcmp(w->gkey[slot], key, sizeof(key)) != 0)) {
     if (w->gexec[slot]) {
       PF_HIP(hipGraphExecDestroy(w->gexec[slot]));
@@ -1588,7 +1592,8 @@ int run_loop(pf_ctx *ctx, SolverWork *w, int slot, const Launch &L, const Mat<V,
 // ---- one-kernel iterations ---------------------------------------------------------------
 // Microseconds per iteration, one kernel / CRS rows / blocked or (73k rows) element tiles, Cube3D on
 // MI355X: 1029 rows 8.2 / 18 / 28, 10k 8.7 / 21 / 38, 28k 10.8 / 30 / 43, 47k 12.3 / 39 / 46 (tiles 31).
-// Above, the entries do not fit the registers of 256 workgroups (16384 each).
+// Above, a hex8 mesh's entries do not fit the registers of 256 workgroups (16384 each); shorter rows do up
+// to PERSIST_MAX_ROWS, but for fewer than four entries per row: 2048 entries are then more than PT rows.
 // Below 64 rows the launches stay: systems of a few rows end by finite termination, where one
 // rounding decides the iteration count, and theirs ends where the reference's does.
 constexpr int64_t PERSIST_MIN_ROWS = 64, PERSIST_MAX_ROWS = 100000;
