@@ -62,10 +62,11 @@ typedef struct {
                                 solver call, so x = x0 (zeros) with the fixed values */
   int32_t spmv_kind;     /* 0 auto (FP64 systems small enough: CRS rows kept on the chip, all iterations
                             in one kernel; else element by element from 40,000 rows on when the values
-                            are exactly a hex8 mesh's stiffness; else blocked when the CRS has DOF=3
+                            are exactly a hex8 mesh's stiffness, unless a mixed form replaces its residual
+                            every third iteration or oftener; else blocked when the CRS has DOF=3
                             node blocks and pads little; else CRS rows, with x staged in LDS for the
-                            unpreconditioned FP64 solve from 2^18 rows on), 1 CRS row kernel, 2 blocked, 4 CRS rows with x staged in LDS per
-                            row block (FP64, no ILU) */
+                            unpreconditioned FP64 solve from 2^18 rows on), 1 CRS row kernel, 2 blocked,
+                            4 CRS rows with x staged in LDS per row block (FP64, no ILU) */
   int32_t check_every;   /* iterations enqueued between host polls of the stop flag (default 32) */
   int32_t use_graph;     /* capture the polled chunk in a hipGraph (default 1) */
   int32_t debug;         /* print sqrt(r.r) per poll */
@@ -487,8 +488,8 @@ int pf_system_batch_autotune(pf_system *sys, const pf_solve_opts *opts, int32_t 
 int pf_system_solve_direct(pf_system *sys, int32_t refine, double *x_out, pf_stats *stats);
 
 /* Every mesh of a batch (pf_system_batch_set) in one persistent kernel: a workgroup takes the
- * next mesh, or its share of a large one, from a largest-first queue (cost = n b^2).  mesh_stats (may be NULL): status, iterations
- * (1 + refine), true_relres, start_ms/end_ms of the mesh's factorization and first
+ * next mesh, or its share of a large one, from a largest-first queue (cost = n b^2).  mesh_stats (may
+ * be NULL): status, iterations (1 + refine), true_relres, start_ms/end_ms of the mesh's factorization and first
  * substitution.  Returns PF_OK, or the status of the first mesh (in mesh order) that failed. */
 int pf_system_batch_direct(pf_system *sys, int32_t refine, double *x_out, pf_batch_mesh_stats *mesh_stats,
                            pf_stats *total);

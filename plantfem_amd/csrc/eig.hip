@@ -7,9 +7,9 @@
 //    on the device and rocSOLVER's dsygvd (itype 1, eigenvectors, upper) solves them; the
 //    eigenvectors come back B-orthonormal, eigenvalues ascending, as DSPGVD returns them.
 //  * the nev lowest pairs (the reference's use_LOBPCG option): block LOBPCG in the full DOF
-//    space with the fixed rows held at zero, the CRS SpMV for A and B, a Jacobi (diag A)
-//    preconditioner, Rayleigh-Ritz on [X W P] with rocBLAS Gram products; the projected
-//    pencil (at most 3 nev square, nev <= 64) is solved on the host by Cholesky of the B-Gram
+//    space with the fixed rows held at zero, A and B times a block in one launch, a Jacobi (diag A)
+//    preconditioner, Rayleigh-Ritz on [X W P] with both Gram matrices in one launch; the projected
+//    pencil (at most 3 nev square, nev <= 32) is solved on the host by Cholesky of the B-Gram
 //    matrix and cyclic Jacobi rotations (a few microseconds; a device solver for matrices
 //    this small costs milliseconds of launches); W and P are scaled to unit B-norm first.
 #include <rocblas/rocblas.h>
@@ -462,7 +462,7 @@ int pf_eig_device(pf_ctx *ctx, int64_t n, const int64_t *row_ptr, const int32_t 
     return PF_OK;
   };
   // Rayleigh-Ritz on the first k columns of S; keeps the lowest m in X (and, with k > m, the
-  // W/P part of the combination in P).  Returns 1 when dsygvd fails.
+  // W/P part of the combination in P).  *failed: the projected B is not positive definite.
   std::vector<double> h_th((size_t)K);
   const double *th = nullptr;  // the lowest m values on the device
   auto rayleigh_ritz = [&](int64_t k, int *failed) -> int {
