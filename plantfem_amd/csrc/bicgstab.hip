@@ -2245,6 +2245,7 @@ int pf_bicgstab_crs_workspace(pf_ctx *ctx, int64_t n, const int64_t *row_ptr, co
                               const double *val, int64_t nnz, const double *b, double *x, const pf_solve_opts &o,
                               double *ws, size_t ws_doubles, SolveResult &res) {
   res = SolveResult();
+  ctx->forms.one_kernel = 0;
   if (o.precision != 64 || o.preconditioning != 0 || o.kernel_timing != 0) {
     pf_set_error("workspace solver: precision 64, no preconditioning and no kernel timing only");
     return PF_INVALID;
